@@ -111,14 +111,17 @@ def tune(op, precision: int = 64, reps: int = 10, max_shapes: int = 8, verbose: 
     y = DeviceArray(n, dt)
     results = []
     base_tiling = op.get_tiling()
-    cands = []
+    # the operator's own tiling first: the default one leaves the choice of
+    # kernel to the operator (one lane per element on large rectilinear meshes)
+    cands = [(tuple(base_tiling), 0, 1)] if 0 in variants and 1 in wg_tiles else []
     for v in variants:
         if v == COLOUR:
             cands.append((tuple(base_tiling), v, 1))
             continue
         for t in candidates(op.mx, op.my, op.mz, max_shapes):
             for w in (wg_tiles if v == 0 else (1,)):
-                cands.append((tuple(t), v, w))
+                if (tuple(t), v, w) not in cands:
+                    cands.append((tuple(t), v, w))
     for t, v, w in cands:
         op.set_kernel_variant(v)
         op.set_tiling(*t)

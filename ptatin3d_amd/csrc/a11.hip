@@ -36,6 +36,7 @@
 // global atomic adds; it serves the host-array PETSc adapter contract.
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "ptmf_internal.h"
@@ -1149,10 +1150,11 @@ __global__ void __launch_bounds__(64)
 // Adds the neighbours' face-buffer contributions into the nodes on the lower
 // faces of each tile (the work-group's threads take one node each in turn;
 // every node's sum has one thread and a fixed order).
-template <typename T>
+// kSkip: the Dirichlet dofs (bcn) are left alone, their rows are already y = x.
+template <typename T, bool kSkip = false>
 __device__ __forceinline__ void face_sum(const TileArgs &a, long tile, const T *__restrict__ fbx,
                                          const T *__restrict__ fby, const T *__restrict__ fbz,
-                                         T *__restrict__ y) {
+                                         T *__restrict__ y, const uint8_t *__restrict__ bcn = nullptr) {
   const TileBox tb = tile_box(a, tile);
   const int oX = 2 * tb.nxt + (tb.xend ? 1 : 0);
   const int oY = 2 * tb.nyt + (tb.yend ? 1 : 0);
@@ -1194,8 +1196,10 @@ __device__ __forceinline__ void face_sum(const TileArgs &a, long tile, const T *
           acc[2] += src[2];
         }
     const long n = (long)I + a.X * (long)J + a.XY * (long)K;
+    const unsigned m = kSkip ? (unsigned)bcn[n] : 0u;
 #pragma unroll
-    for (int l = 0; l < 3; l++) y[3 * n + l] += acc[l];
+    for (int l = 0; l < 3; l++)
+      if (!kSkip || !((m >> l) & 1u)) y[3 * n + l] += acc[l];
   }
 }
 
@@ -1204,11 +1208,11 @@ __device__ __forceinline__ void face_sum(const TileArgs &a, long tile, const T *
 // wave would walk one dependent load/store round after another.
 constexpr int kFaceThreads = 256;
 
-template <typename T>
+template <typename T, bool kSkip = false>
 __global__ void __launch_bounds__(kFaceThreads)
     a11_face_kernel(TileArgs a, const T *__restrict__ fbx, const T *__restrict__ fby,
-                    const T *__restrict__ fbz, T *__restrict__ y) {
-  face_sum<T>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y);
+                    const T *__restrict__ fbz, T *__restrict__ y, const uint8_t *__restrict__ bcn = nullptr) {
+  face_sum<T, kSkip>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
 }
 
 // ---------------------------------------------------------------------------
@@ -1263,6 +1267,8 @@ __global__ void bc_copy_batch_kernel(const BoxDesc *__restrict__ boxes, const T 
   }
 }
 
+#include "a11_lane.h"
+
 TileArgs tile_args(const ptmf_op_s *op) {
   const Box &b = op->box;
   TileArgs a;
@@ -1277,7 +1283,175 @@ TileArgs tile_args(const ptmf_op_s *op) {
   return a;
 }
 
+// The lane kernel's decomposition of box b in precision T; false where the tile
+// kernel runs instead (as it does on a mesh that is not rectilinear, or with a
+// tiling, variant or tiles per work-group of the caller's choice): with arrays
+// past the 32-bit offsets of the lane kernel, in FP32 with more than 64 elements in a
+// direction (there the tile kernel's FP32 interpolation of the coordinates
+// rounds the Jacobian off by more than 1e-5, and the two kernels would differ
+// by that), and where the tile kernel is faster.
+// The costs are microseconds per round of one wave on each of the 1024 SIMDs,
+// times the layers a wave marches through.  Measured at 64^3 with the chip
+// full, FP64: 18.1 us per layer of 64 elements (lane) and 14.6 us per layer of
+// 20 (tile); FP32, two waves per SIMD: 19.6 and 12.6 us for both, 13 and 10.5
+// us with one; the lane kernel's first and last planes add 0.45 of a layer.
+// So the tile kernel keeps the small boxes that it takes in one round (16^3:
+// 13.5 us against 19.3 us), and the lane kernel has the rest (45 x 37 x 29:
+// 25.7 us against 50.1 us, 64^3: 79.6 against 178 us, 128^3 MatMult 707
+// against 1480 us; FP32 20.7 against 25.5 and 48 against 82 us).
+template <typename T>
+double lane_rounds(long waves, double one, double two) {
+  const long r = (waves + 1023) / 1024;
+  return sizeof(T) == 8 ? one * (double)r : two * (double)(r / 2) + one * (double)(r % 2);
+}
+
+template <typename T>
+bool lane_plan(const Box &b, const Tiling &t, TileArgs &a) {
+  constexpr bool f64 = sizeof(T) == 8;
+  if (!f64 && std::max(b.mx, std::max(b.my, b.mz)) > 64) return false;
+  a.mx = b.mx; a.my = b.my; a.mz = b.mz;
+  a.X = b.X; a.XY = b.X * b.Y; a.nel = b.nel;
+  a.TX = a.TY = kLT;
+  a.ntx = (b.mx + kLT - 1) / kLT;
+  a.nty = (b.my + kLT - 1) / kLT;
+  const long txy = (long)a.ntx * a.nty;
+  double best = 1e300;
+  for (int zc = 1; zc <= b.mz && zc <= kLMaxZ; zc++) {
+    const long nt = txy * ((b.mz + zc - 1) / zc);
+    const double cost = (zc + 0.45) * lane_rounds<T>(nt, f64 ? 18.1 : 13.0, 19.6);
+    if (cost < best) {
+      best = cost;
+      a.ZC = zc;
+      a.ntiles = nt;
+    }
+  }
+  if (best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 12.6)) return false;
+  a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
+  a.fbz_n = kLRows * kLRows;
+  return 8 * 3 * b.nnodes < (1L << 32) && 8 * 27 * b.nel < (1L << 32) &&
+         8 * face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) < (1L << 32);
+}
+
+// the same for an operator with face buffers of fb_doubles
+template <typename T>
+bool lane_tiles(const ptmf_op_s *op, long fb_doubles, TileArgs &a) {
+  return op->rect && op->tiling_default && op->wg_tiles == 1 && lane_plan<T>(op->box, op->tiling, a) &&
+         face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= fb_doubles;
+}
+
+// Is the mesh rectilinear?  Axis lines of the three directions first (mid
+// nodes halfway between their neighbours, ax = 2 / h per element), then every
+// node against the lines.  "Equal" is to 4 units of rounding of the largest
+// coordinate of the direction: what a mesh generator's own rounding leaves,
+// and what the general kernel's interpolation of the coordinates rounds off
+// anyway.  *bad is set when a check fails.
+__global__ void __launch_bounds__(256)
+    rect_axes_kernel(int mx, int my, int mz, long X, long XY, const double *__restrict__ xc, double *__restrict__ a64,
+                     float *__restrict__ a32, double *__restrict__ tol, int *__restrict__ bad) {
+  __shared__ double red[256];
+  const int m[3] = {mx, my, mz};
+  const long stride[3] = {3, 3 * X, 3 * XY};
+  for (int d = 0, first = 0; d < 3; first += m[d], d++) {
+    double big = 0.0;
+    for (int i = threadIdx.x; i <= 2 * m[d]; i += 256) big = fmax(big, fabs(xc[stride[d] * i + d]));
+    red[threadIdx.x] = big;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
+      __syncthreads();
+    }
+    const double t = 4.0 * 2.220446049250313e-16 * red[0];
+    __syncthreads();
+    if (threadIdx.x == 0) tol[d] = t;
+    for (int e = threadIdx.x; e < m[d]; e += 256) {
+      const double *x = xc + stride[d] * (2 * e) + d;
+      const double x0 = x[0], x1 = x[stride[d]], x2 = x[2 * stride[d]], h = x2 - x0;
+      if (!(fabs(x1 - 0.5 * (x0 + x2)) <= t) || !(fabs(h) > 64.0 * t) || !isfinite(h)) *bad = 1;
+      a64[first + e] = 2.0 / h;
+      a32[first + e] = (float)(2.0 / h);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256)
+    rect_check_kernel(long n, int X, int Y, const double *__restrict__ xc, const double *__restrict__ tol,
+                      int *__restrict__ bad) {
+  const double t0 = tol[0], t1 = tol[1], t2 = tol[2];
+  bool off = false;
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    const int r = (int)(i / X), I = (int)(i - (long)r * X), K = r / Y, J = r - K * Y;
+    const double *x = xc + 3 * i;
+    off |= !(fabs(x[0] - xc[3L * I]) <= t0) || !(fabs(x[1] - xc[3L * X * J + 1]) <= t1) ||
+           !(fabs(x[2] - xc[3L * X * Y * K + 2]) <= t2);
+  }
+  if (__any(off) && (threadIdx.x & 63) == 0) *bad = 1;
+}
+
+// per tile column of the lane kernel and node plane: 1 if one of the tile's
+// nodes in the plane has a Dirichlet dof
+__global__ void __launch_bounds__(64)
+    bc_plane_kernel(int mx, int my, int ntx, long X, long XY, long Z, const uint8_t *__restrict__ bcn,
+                    uint8_t *__restrict__ flags) {
+  const long col = blockIdx.x / Z, P = blockIdx.x - col * Z;
+  const int tx = (int)(col % ntx), ty = (int)(col / ntx);
+  const int x0 = kLT * tx, y0 = kLT * ty, wX = 2 * min(kLT, mx - x0) + 1, wY = 2 * min(kLT, my - y0) + 1;
+  unsigned any = 0;
+  for (int t = threadIdx.x; t < wX * wY; t += 64) any |= bcn[2 * x0 + t % wX + X * (2 * y0 + t / wX) + XY * P];
+  any = __any(any != 0);
+  if (threadIdx.x == 0) flags[blockIdx.x] = any ? 1 : 0;
+}
+
 }  // namespace
+
+int alloc_lane_data(ptmf_op_s *op) {
+  // one allocation: 2 / h in FP64 (and three tolerances) and FP32, the
+  // classification's flag, the plane flags
+  const Box &b = op->box;
+  const long na = b.mx + b.my + b.mz;
+  const long planes = (long)((b.mx + kLT - 1) / kLT) * ((b.my + kLT - 1) / kLT) * b.Z;
+  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) + planes));
+  op->ax32 = (float *)(op->ax64 + na + 3);
+  op->rect_bad = (int *)(op->ax32 + na);
+  op->bcplane = (uint8_t *)(op->rect_bad + 1);
+  return PTMF_OK;
+}
+
+int mark_dirichlet_planes(ptmf_op_s *op) {
+  const Box &b = op->box;
+  const int ntx = (b.mx + kLT - 1) / kLT, nty = (b.my + kLT - 1) / kLT;
+  const long n = (long)ntx * nty * b.Z;
+  bc_plane_kernel<<<dim3((unsigned)n), 64, 0, op->stream>>>(b.mx, b.my, ntx, b.X, b.X * b.Y, b.Z, op->bcnode,
+                                                            op->bcplane);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
+int classify_mesh(ptmf_op_s *op) {
+  const Box &b = op->box;
+  const long na = b.mx + b.my + b.mz;
+  op->rect = 0;
+  PTMF_TRY(launch_fill<int>(op->rect_bad, 0, 1, op->stream));
+  rect_axes_kernel<<<1, 256, 0, op->stream>>>(b.mx, b.my, b.mz, b.X, b.X * b.Y, op->d64.coords, op->ax64, op->ax32,
+                                              op->ax64 + na, op->rect_bad);
+  long nb = (b.nnodes + 255) / 256;
+  if (nb > 8192) nb = 8192;
+  rect_check_kernel<<<dim3((unsigned)nb), 256, 0, op->stream>>>(b.nnodes, (int)b.X, (int)b.Y, op->d64.coords,
+                                                               op->ax64 + na, op->rect_bad);
+  PTMF_HIP(hipGetLastError());
+  int bad = 1;
+  PTMF_HIP(hipMemcpyAsync(&bad, op->rect_bad, sizeof(int), hipMemcpyDeviceToHost, op->stream));
+  PTMF_HIP(hipStreamSynchronize(op->stream));
+  op->rect = !bad;
+  return PTMF_OK;
+}
+
+long lane_face_doubles(const Box &b, const Tiling &t) {
+  TileArgs a;
+  long n = 0;
+  if (lane_plan<double>(b, t, a)) n = face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles);
+  if (lane_plan<float>(b, t, a)) n = std::max(n, face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles));
+  return n;
+}
 
 long face_buffer_doubles(int TX, int TY, int ZC, long ntiles) {
   const long per = (long)(2 * TY + 1) * (2 * ZC + 1) + (long)(2 * TX + 1) * (2 * ZC + 1) +
@@ -1411,7 +1585,7 @@ int eta_tiled_in_place(ptmf_op_s *op) {
 // is allocated on the way (the stored-geometry and coloured variants, which
 // build tables of their own or need no face buffers, give way to the z-march).
 template <typename T>
-int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, bool noalloc = false) {
+int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long fb_doubles, bool noalloc = false) {
   const OpData<T> &d = *(const OpData<T> *)(sizeof(T) == 8 ? (const void *)&op->d64
                                                            : (const void *)&op->d32);
   const Tiling &tl = op->tiling;
@@ -1431,6 +1605,27 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, bool n
     }
     PTMF_HIP(hipGetLastError());
     if (faces == 1) PTMF_TRY(launch_bc_copy<T>(op->bcidx, op->nbc, x, y, op->stream));
+    return PTMF_OK;
+  }
+  TileArgs la;
+  if (variant == 0 && lane_tiles<T>(op, fb_doubles, la)) {
+    const T *ax = sizeof(T) == 8 ? (const T *)op->ax64 : (const T *)op->ax32;
+    T *fbx = fb, *fby = fbx + 3 * la.fbx_n * la.ntiles, *fbz = fby + 3 * la.fby_n * la.ntiles;
+    const dim3 grid((unsigned)la.ntiles);
+    if (faces == 2)
+      a11_lane_kernel<T, false><<<grid, dim3(64), 0, op->stream>>>(la, ax, d.eta, op->bcnode, op->bcplane, x, y, fbx,
+                                                                         fby, fbz);
+    else
+      a11_lane_kernel<T, true><<<grid, dim3(64), 0, op->stream>>>(la, ax, d.eta, op->bcnode, op->bcplane, x, y, fbx,
+                                                                         fby, fbz);
+    PTMF_HIP(hipGetLastError());
+    if (faces) {
+      if (faces == 1)
+        a11_face_kernel<T, true><<<grid, dim3(kFaceThreads), 0, op->stream>>>(la, fbx, fby, fbz, y, op->bcnode);
+      else
+        a11_face_kernel<T><<<grid, dim3(kFaceThreads), 0, op->stream>>>(la, fbx, fby, fbz, y);
+      PTMF_HIP(hipGetLastError());
+    }
     return PTMF_OK;
   }
   const TileArgs a = tile_args(op);
@@ -1470,7 +1665,7 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, bool n
 
 template <typename T>
 int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, int faces) {
-  return launch_a11_mult_fb<T>(op, x, y, faces, (T *)op->faces);
+  return launch_a11_mult_fb<T>(op, x, y, faces, (T *)op->faces, op->faces_doubles);
 }
 
 template <typename T>
@@ -1784,5 +1979,5 @@ extern "C" int ptmf_a11_mult_noalloc(ptmf_op op, const double *x, double *y) {
              need, kScratchDoubles);
   double *fb = nullptr;
   PTMF_TRY(scratch_address(dev, &fb));
-  return ptmf::launch_a11_mult_fb<double>(op, x, y, 1, fb, true);
+  return ptmf::launch_a11_mult_fb<double>(op, x, y, 1, fb, kScratchDoubles, true);
 }

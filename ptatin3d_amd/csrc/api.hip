@@ -4,6 +4,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "ptmf_internal.h"
@@ -157,6 +158,7 @@ int ptmf_op_create(int mx, int my, int mz, ptmf_op *out) {
   alloc((void **)&op->d32.coords, sizeof(float) * 3 * b.nnodes);
   alloc((void **)&op->d32.eta, sizeof(float) * 27 * b.nel);
   alloc((void **)&op->bcnode, sizeof(uint8_t) * b.nnodes);
+  if (st == PTMF_OK) st = ptmf::alloc_lane_data(op);
   if (st == PTMF_OK) {
     hipError_t e = hipGetDevice(&op->device);
     if (e == hipSuccess) e = hipStreamCreate(&op->stream);
@@ -167,8 +169,9 @@ int ptmf_op_create(int mx, int my, int mz, ptmf_op *out) {
   if (st == PTMF_OK) st = ptmf_memset(op->bcnode, 0, b.nnodes);
   if (st == PTMF_OK) {
     op->tiling = ptmf::choose_tiling(mx, my, mz);
-    op->faces_doubles = ptmf::face_buffer_doubles(op->tiling.TX, op->tiling.TY, op->tiling.ZC,
-                                                  op->tiling.ntiles);
+    op->faces_doubles = std::max(ptmf::face_buffer_doubles(op->tiling.TX, op->tiling.TY, op->tiling.ZC,
+                                                           op->tiling.ntiles),
+                                 ptmf::lane_face_doubles(b, op->tiling));
     st = ptmf_malloc(&op->faces, sizeof(double) * op->faces_doubles);
   }
   if (st != PTMF_OK) {
@@ -198,6 +201,7 @@ int ptmf_op_destroy(ptmf_op *pop) {
   (void)hipFree(op->pa_bad);
   (void)hipFree(op->et64);
   (void)hipFree(op->et32);
+  (void)hipFree(op->ax64);
   if (op->ev0) (void)hipEventDestroy(op->ev0);
   if (op->ev1) (void)hipEventDestroy(op->ev1);
   if (op->stream) (void)hipStreamDestroy(op->stream);
@@ -229,6 +233,8 @@ int ptmf_op_set_tiling(ptmf_op op, int TX, int TY, int ZC) {
     op->faces_doubles = need;
   }
   op->tiling = t;
+  const ptmf::Tiling def = ptmf::choose_tiling(b.mx, b.my, b.mz);
+  op->tiling_default = TX == def.TX && TY == def.TY && ZC == def.ZC;
   return op->has_eta ? ptmf::prepare_eta_tiled(op) : PTMF_OK;
 }
 
@@ -282,6 +288,7 @@ int ptmf_op_set_coordinates(ptmf_op op, const double *coords) {
   for (long i = 0; i < n; i++) c32[i] = (float)coords[i];
   PTMF_HIP(hipMemcpy(op->d64.coords, coords, sizeof(double) * n, hipMemcpyHostToDevice));
   PTMF_HIP(hipMemcpy(op->d32.coords, c32.data(), sizeof(float) * n, hipMemcpyHostToDevice));
+  PTMF_TRY(ptmf::classify_mesh(op));
   op->has_coords = 1;
   op->state++;
   return PTMF_OK;
@@ -359,6 +366,7 @@ int ptmf_op_set_dirichlet(ptmf_op op, const unsigned char *mask) {
     PTMF_TRY(ptmf_malloc((void **)&op->bcidx, sizeof(long) * op->nbc));
     PTMF_HIP(hipMemcpy(op->bcidx, idx.data(), sizeof(long) * op->nbc, hipMemcpyHostToDevice));
   }
+  PTMF_TRY(ptmf::mark_dirichlet_planes(op));
   op->has_bc = 1;
   op->state++;
   return PTMF_OK;

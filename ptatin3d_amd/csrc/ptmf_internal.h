@@ -96,12 +96,20 @@ struct ptmf_op_s {
   uint8_t *bcnode = nullptr;      // per-node Dirichlet bits (bit d: dof d)
   long *bcidx = nullptr;          // compact list of Dirichlet dofs
   long nbc = 0;
+  uint8_t *bcplane = nullptr;     // per 8 x 8 tile column and node plane: any Dirichlet dof
   int has_coords = 0, has_eta = 0, has_bc = 0;
   unsigned long state = 0;        // bumped by every coefficient change
   int device = 0;                 // device the operator was created on
   hipStream_t stream = nullptr;   // stream all work of this operator runs on
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   ptmf::Tiling tiling;
+  int tiling_default = 1;         // the tiling is choose_tiling's own
+  // rectilinear mesh (element faces normal to the axes): 2 / h per element of
+  // the mx columns, my rows and mz layers
+  int rect = 0;
+  double *ax64 = nullptr;         // holds ax32, rect_bad and bcplane too
+  float *ax32 = nullptr;
+  int *rect_bad = nullptr;
   int variant = 0;  // MatMult kernel: 0 z-march, 1 software-pipelined, 2 stored geometry, 3 coloured
   int wg_tiles = 1;  // tiles (one wave each) per work-group of the variant-0 z-march: 1, 2 or 4
   // stored quadrature-point geometry of variant 2 (per precision), valid for
@@ -160,6 +168,16 @@ int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, int faces);
 // build (or rebuild) the FP64 tile-ordered viscosity for the current
 // coefficients and tiling (allocates; set-up time)
 int prepare_eta_tiled(ptmf_op_s *op);
+// the operator's data of the lane kernel (freed through op->ax64)
+int alloc_lane_data(ptmf_op_s *op);
+// set-up: op->rect and op->ax* from the operator's coordinates
+int classify_mesh(ptmf_op_s *op);
+// face buffers of the lane kernel on box b with the default tiling t (0: it
+// does not run there); part of every operator's allocation, whatever its mesh,
+// so that new coordinates never move the buffers
+long lane_face_doubles(const Box &b, const Tiling &t);
+// set-up: op->bcplane from the operator's Dirichlet bits
+int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>
 int launch_fill(T *x, T v, long n, hipStream_t s);
 template <typename T>
