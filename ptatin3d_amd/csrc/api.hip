@@ -171,7 +171,7 @@ int ptmf_op_create(int mx, int my, int mz, ptmf_op *out) {
     op->tiling = ptmf::choose_tiling(mx, my, mz);
     op->faces_doubles = std::max(ptmf::face_buffer_doubles(op->tiling.TX, op->tiling.TY, op->tiling.ZC,
                                                            op->tiling.ntiles),
-                                 ptmf::lane_face_doubles(b, op->tiling));
+                                 std::max(ptmf::lane_face_doubles(b, op->tiling), ptmf::couple_face_doubles(b)));
     st = ptmf_malloc(&op->faces, sizeof(double) * op->faces_doubles);
   }
   if (st != PTMF_OK) {
@@ -467,9 +467,7 @@ int ptmf_schur_mass_blocks(ptmf_op op, double *Me) {
 int ptmf_a12_mult(ptmf_op op, const double *p, double *yu) {
   PTMF_TRY(check_ready(op, false, true));
   PTMF_CHECK(p && yu, PTMF_ERR_ARG, "a12_mult: null");
-  PTMF_TRY(ptmf::launch_fill<double>(yu, 0.0, 3 * op->box.nnodes, op->stream));
   PTMF_TRY(ptmf::launch_a12(op, p, yu));
-  PTMF_TRY(ptmf::launch_bc_set<double>(op->bcidx, op->nbc, 0.0, yu, op->stream));
   PTMF_HIP(hipStreamSynchronize(op->stream));
   return PTMF_OK;
 }

@@ -1,5 +1,5 @@
-// elem.hip -- per-element Q2 kernels other than the A11 apply: the A11
-// diagonal and the pressure-velocity couplings B (A12) and B^T (A21).
+// elem.hip -- per-element Q2 kernels: the A11 diagonal and its l1 row sums, the
+// Schur blocks and the power-law viscosity.
 //
 // Layout of a work-group: 64 lanes, 2 elements, lanes 32h + q (q < 27) own
 // quadrature point q of element h, lanes 32h + n (n < 27) own node n in the
@@ -275,109 +275,6 @@ __global__ void __launch_bounds__(128)
     }
     const long node = elem_node(mx, my, X, XY, e, a);
     atomicAdd(&l1[3 * node + c], sum);
-  }
-}
-
-// ---- B p: yu[3n+c] += sum_q -w detJ (d_c N_n) p_h(x_q)
-// (MFStokesWrapper_A12, stokes_operators_mf.c:788-856 with
-// MatMultMF_Stokes_MixedFEM3d_A12, stokes_q2p1_mf_operators_def.c:423-516)
-__global__ void __launch_bounds__(64)
-    a12_kernel(int mx, int my, int mz, long nel, long X, long XY, int color, const double *__restrict__ xc,
-               const double *__restrict__ p, double *__restrict__ yu) {
-  __shared__ double sx[kEPB][27][3];
-  __shared__ double sG[kEPB][27][10];
-  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
-  bool live;  // one parity class per launch: plain read-add-write below
-  const long e = class_element(mx, my, mz, color, (long)blockIdx.x * kEPB + h, live);
-  if (t < 27) {
-    const long node = elem_node(mx, my, X, XY, e, t);
-    for (int d = 0; d < 3; d++) sx[h][t][d] = xc[3 * node + d];
-  }
-  __syncthreads();
-  if (t < 27) {
-    QpGeom g;
-    qp_geometry(sx[h], t, g);
-    double Np[4];
-    p1_basis(sx[h], g.xq, Np);
-    const double ph = Np[0] * p[4 * e] + Np[1] * p[4 * e + 1] + Np[2] * p[4 * e + 2] +
-                      Np[3] * p[4 * e + 3];
-    for (int r = 0; r < 3; r++)
-      for (int s = 0; s < 3; s++) sG[h][t][3 * r + s] = g.G[r][s];
-    sG[h][t][9] = -g.wdet * ph;
-  }
-  __syncthreads();
-  if (t < 27 && live) {
-    LaneTab T;
-    lane_tab_node(t, T);
-    double acc[3] = {0, 0, 0};
-#pragma unroll 1
-    for (int qc = 0; qc < 3; qc++) {
-      const double bk = pick3(qc, T.B[2][0], T.B[2][1], T.B[2][2]), dk = pick3(qc, T.D[2][0], T.D[2][1], T.D[2][2]);
-#pragma unroll
-      for (int qb = 0; qb < 3; qb++)
-#pragma unroll
-        for (int qa = 0; qa < 3; qa++) {
-          const double *G = sG[h][qa + 3 * qb + 9 * qc];
-          const double gr[3] = {T.D[0][qa] * T.B[1][qb] * bk, T.B[0][qa] * T.D[1][qb] * bk,
-                                T.B[0][qa] * T.B[1][qb] * dk};
-#pragma unroll
-          for (int k = 0; k < 3; k++)
-            acc[k] += G[9] * (G[3 * k] * gr[0] + G[3 * k + 1] * gr[1] + G[3 * k + 2] * gr[2]);
-        }
-    }
-    const long node = elem_node(mx, my, X, XY, e, t);
-    for (int c = 0; c < 3; c++) yu[3 * node + c] += acc[c];
-  }
-}
-
-// ---- B^T u: yp[4e+i] = sum_q -w detJ NIp_i div u_h(x_q), u Dirichlet-masked
-// (MFStokesWrapper_A21, stokes_operators_mf.c:858-933 with
-// MatMultMF_Stokes_MixedFEM3d_A21, stokes_q2p1_mf_operators_def.c:517-538)
-__global__ void __launch_bounds__(64)
-    a21_kernel(int mx, int my, long nel, long X, long XY, const double *__restrict__ xc,
-               const uint8_t *__restrict__ bcn, const double *__restrict__ u,
-               double *__restrict__ yp) {
-  __shared__ double sx[kEPB][27][3];
-  __shared__ double su[kEPB][27][3];
-  __shared__ double sr[kEPB][32][4];
-  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
-  long e = (long)blockIdx.x * kEPB + h;
-  const bool live = e < nel;
-  if (!live) e = nel - 1;
-  if (t < 27) {
-    const long node = elem_node(mx, my, X, XY, e, t);
-    const unsigned m = bcn[node];
-    for (int d = 0; d < 3; d++) {
-      sx[h][t][d] = xc[3 * node + d];
-      su[h][t][d] = ((m >> d) & 1u) ? 0.0 : u[3 * node + d];
-    }
-  }
-  __syncthreads();
-  double val[4] = {0, 0, 0, 0};
-  if (t < 27) {
-    QpGeom g;
-    qp_geometry(sx[h], t, g);
-    double Np[4];
-    p1_basis(sx[h], g.xq, Np);
-    double div = 0.0;
-    LaneTab T;
-    lane_tab_qp(t, T);
-#pragma unroll
-    for (int n = 0; n < 27; n++) {
-      double gr[3];
-      tab_grad(T, n % 3, (n / 3) % 3, n / 9, gr);
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-        div += su[h][n][k] * (g.G[k][0] * gr[0] + g.G[k][1] * gr[1] + g.G[k][2] * gr[2]);
-    }
-    for (int i = 0; i < 4; i++) val[i] = -g.wdet * Np[i] * div;
-  }
-  for (int i = 0; i < 4; i++) sr[h][t][i] = val[i];
-  __syncthreads();
-  if (t < 4 && live) {
-    double s = 0.0;
-    for (int q = 0; q < 27; q++) s += sr[h][q][t];
-    yp[4 * e + t] = s;
   }
 }
 
@@ -694,30 +591,6 @@ int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, doubl
   powerlaw_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.nel, b.X, b.X * b.Y,
                                                                      op->d64.coords, u, B, nexp, eta_min,
                                                                      eta_max, eta);
-  PTMF_HIP(hipGetLastError());
-  return PTMF_OK;
-}
-
-int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
-  PTMF_TRY(init_constants());
-  const Box &b = op->box;
-  for (int color = 0; color < 8; color++) {
-    const long ncol = class_count(b, color);
-    if (ncol == 0) continue;
-    const long nblk = (ncol + kEPB - 1) / kEPB;
-    a12_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.mz, b.nel, b.X, b.X * b.Y,
-                                                                   color, op->d64.coords, p, yu);
-    PTMF_HIP(hipGetLastError());
-  }
-  return PTMF_OK;
-}
-
-int launch_a21(const ptmf_op_s *op, const double *u, double *yp) {
-  PTMF_TRY(init_constants());
-  const Box &b = op->box;
-  const long nblk = (b.nel + kEPB - 1) / kEPB;
-  a21_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(
-      b.mx, b.my, b.nel, b.X, b.X * b.Y, op->d64.coords, op->bcnode, u, yp);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

@@ -176,6 +176,7 @@ int classify_mesh(ptmf_op_s *op);
 // does not run there); part of every operator's allocation, whatever its mesh,
 // so that new coordinates never move the buffers
 long lane_face_doubles(const Box &b, const Tiling &t);
+long couple_face_doubles(const Box &b);  // of launch_a12
 // set-up: op->bcplane from the operator's Dirichlet bits
 int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>
@@ -204,6 +205,7 @@ int launch_a11_diag(const ptmf_op_s *op, double *d);
 int launch_a11_l1(const ptmf_op_s *op, double *d);
 int launch_schur_blocks(const ptmf_op_s *op, double *Me, double *Minv);
 int launch_schur_apply(const ptmf_op_s *op, const double *Minv, const double *rp, double *yp);
+// yu = B p, Dirichlet rows 0
 int launch_a12(const ptmf_op_s *op, const double *p, double *yu);
 // Multifrontal Cholesky of a level operator given as its 125-point 3x3-block
 // stencil S (device, S[((o*9)+3r+c)*N + m] = A(3m+r, 3(m+off_o)+c), SPD with
