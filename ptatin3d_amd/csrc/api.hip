@@ -202,6 +202,7 @@ int ptmf_op_destroy(ptmf_op *pop) {
   (void)hipFree(op->et64);
   (void)hipFree(op->et32);
   (void)hipFree(op->ax64);
+  (void)hipFree(op->points);
   if (op->ev0) (void)hipEventDestroy(op->ev0);
   if (op->ev1) (void)hipEventDestroy(op->ev1);
   if (op->stream) (void)hipStreamDestroy(op->stream);

@@ -10,6 +10,8 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include <mutex>
+
 #include "ptmf.h"
 
 namespace ptmf {
@@ -130,6 +132,8 @@ struct ptmf_op_s {
   long faces_doubles = 0;
   double *host_stage = nullptr;   // device staging for the host-array entry points
   double *host_stage2 = nullptr;
+  double *points = nullptr;       // point projection: 18 sums per element, then the nodal field
+  std::mutex points_mu;
 };
 
 // Error plumbing: every entry point returns a ptmf status code.
