@@ -1183,13 +1183,14 @@ bool lane_tiles(const ptmf_op_s *op, long fb_doubles, TileArgs &a) {
 // node against the lines.  "Equal" is to 4 units of rounding of the largest
 // coordinate of the direction: what a mesh generator's own rounding leaves,
 // and what the general kernel's interpolation of the coordinates rounds off
-// anyway.  *bad is set when a check fails.
+// anyway.  *bad is cleared, and set when a check fails.
 __global__ void __launch_bounds__(256)
     rect_axes_kernel(int mx, int my, int mz, long X, long XY, const double *__restrict__ xc, double *__restrict__ a64,
                      float *__restrict__ a32, double *__restrict__ tol, int *__restrict__ bad) {
   __shared__ double red[256];
   const int m[3] = {mx, my, mz};
   const long stride[3] = {3, 3 * X, 3 * XY};
+  if (threadIdx.x == 0) *bad = 0;
   for (int d = 0, first = 0; d < 3; first += m[d], d++) {
     double big = 0.0;
     for (int i = threadIdx.x; i <= 2 * m[d]; i += 256) big = fmax(big, fabs(xc[stride[d] * i + d]));
@@ -1269,7 +1270,6 @@ int classify_mesh(ptmf_op_s *op) {
   const Box &b = op->box;
   const long na = b.mx + b.my + b.mz;
   op->rect = 0;
-  PTMF_TRY(launch_fill<int>(op->rect_bad, 0, 1, op->stream));
   rect_axes_kernel<<<1, 256, 0, op->stream>>>(b.mx, b.my, b.mz, b.X, b.X * b.Y, op->d64.coords, op->ax64, op->ax32,
                                               op->ax64 + na, op->rect_bad);
   long nb = (b.nnodes + 255) / 256;
@@ -1419,6 +1419,22 @@ int eta_tiled_in_place(ptmf_op_s *op) {
   return PTMF_OK;
 }
 
+// the lane kernel (lane_tiles must hold) and its faces
+template <typename T, LaneBC kBC, bool kP>
+int launch_lane(const ptmf_op_s *op, const TileArgs &a, int faces, const T *x, const T *p, T *y, T *yp, T *fb) {
+  const T *ax = sizeof(T) == 8 ? (const T *)op->ax64 : (const T *)op->ax32;
+  const T *eta = sizeof(T) == 8 ? (const T *)op->d64.eta : (const T *)op->d32.eta;
+  T *fbx = fb, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
+  const dim3 grid((unsigned)a.ntiles);
+  a11_lane_kernel<T, kBC, kP><<<grid, dim3(64), 0, op->stream>>>(a, ax, eta, op->bcnode, op->bcplane, x, p, y, yp, fbx,
+                                                                   fby, fbz);
+  PTMF_HIP(hipGetLastError());
+  if (!faces) return PTMF_OK;
+  a11_face_kernel<T, kBC == kLaneCopy><<<grid, dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y, op->bcnode);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
 // The MatMult's kernels with the face buffers at fb (the operator's own, or
 // the static scratch of the allocation-free entry point).  noalloc: nothing
 // is allocated on the way (the stored-geometry and coloured variants, which
@@ -1448,24 +1464,8 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
   }
   TileArgs la;
   if (variant == 0 && lane_tiles<T>(op, fb_doubles, la)) {
-    const T *ax = sizeof(T) == 8 ? (const T *)op->ax64 : (const T *)op->ax32;
-    T *fbx = fb, *fby = fbx + 3 * la.fbx_n * la.ntiles, *fbz = fby + 3 * la.fby_n * la.ntiles;
-    const dim3 grid((unsigned)la.ntiles);
-    if (faces == 2)
-      a11_lane_kernel<T, kLaneSums><<<grid, dim3(64), 0, op->stream>>>(la, ax, d.eta, op->bcnode, op->bcplane, x, y, fbx,
-                                                                         fby, fbz);
-    else
-      a11_lane_kernel<T, kLaneCopy><<<grid, dim3(64), 0, op->stream>>>(la, ax, d.eta, op->bcnode, op->bcplane, x, y, fbx,
-                                                                         fby, fbz);
-    PTMF_HIP(hipGetLastError());
-    if (faces) {
-      if (faces == 1)
-        a11_face_kernel<T, true><<<grid, dim3(kFaceThreads), 0, op->stream>>>(la, fbx, fby, fbz, y, op->bcnode);
-      else
-        a11_face_kernel<T><<<grid, dim3(kFaceThreads), 0, op->stream>>>(la, fbx, fby, fbz, y);
-      PTMF_HIP(hipGetLastError());
-    }
-    return PTMF_OK;
+    if (faces == 2) return launch_lane<T, kLaneSums, false>(op, la, faces, x, nullptr, y, nullptr, fb);
+    return launch_lane<T, kLaneCopy, false>(op, la, faces, x, nullptr, y, nullptr, fb);
   }
   const TileArgs a = tile_args(op);
   const long ntiles = tl.ntiles;
@@ -1515,10 +1515,16 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   PTMF_CHECK(tl.TX * tl.TY <= kEPW && (2 * tl.TX + 1) * (2 * tl.TY + 1) <= kWinNodes && tl.ZC > 0,
              PTMF_ERR_ARG, "stokes: invalid tiling %d x %d x %d", tl.TX, tl.TY, tl.ZC);
   PTMF_CHECK(op->faces != nullptr, PTMF_ERR_NOT_SETUP, "stokes: face buffers not allocated");
+  const long nu = 3 * op->box.nnodes;
+  // (by lane_plan's rule for the MatMult: at 24^3 both take 42 us, at 28^3 the
+  // lane kernel 41 us and the tile kernel 62 us, and further apart above)
+  TileArgs la;
+  if (lane_tiles<T>(op, op->faces_doubles, la))
+    return launch_lane<T, kLaneCopy, true>(op, la, 1, x, x + nu, y, y + nu, (T *)op->faces);
   PTMF_TRY(ensure_eta_tiled<T>(op));
   const T *et = sizeof(T) == 8 ? (const T *)op->et64 : (const T *)op->et32;
   const TileArgs a = tile_args(op);
-  const long ntiles = tl.ntiles, nu = 3 * op->box.nnodes;
+  const long ntiles = tl.ntiles;
   T *fbx = (T *)op->faces, *fby = fbx + 3 * a.fbx_n * ntiles, *fbz = fby + 3 * a.fby_n * ntiles;
   stokes_tile_kernel<T><<<dim3((unsigned)ntiles), dim3(64), 0, op->stream>>>(
       a, d.coords, et, op->bcnode, x, x + nu, y, y + nu, fbx, fby, fbz);

@@ -21,6 +21,11 @@
 // same kernel with its loads in flight across the stress stage took 130 us,
 // with 40 scratch moves 156 us).  So every load is issued before a forward
 // stage and used up at its end, where few registers are live.
+//
+// The saddle-point product runs the same way: the couplings add some 10
+// instructions a point, the pressure basis being that of the unit cube, and 66
+// AGPRs (96 x 96 x 48 MatMult 171 us, the tile kernel's 485 us; 28^3 41 and 62
+// us).
 
 // per-lane constants of a rectilinear element: the collocation coefficients
 // of the two in-plane directions scaled by 2 / h, and the Jacobian determinant
@@ -58,9 +63,12 @@ __device__ __forceinline__ void ldot_t(int a, const T c[3], T v, T &y0, T &y1, T
 
 // Stress at the plane's points and its transposed derivatives:
 // out[k][l][3j+i] += the plane's part of (A11_e u)(node (i, j, k), component l)
-template <typename T, int c>
+// kP: of the saddle-point product.  The pressure basis of a rectilinear element
+// is {1, xi / 2, eta / 2, zeta / 2}; pc: its coefficients, the last three times
+// s / 2; acc += the plane's part of (A21_e u), the last three over s / 2.
+template <typename T, int c, bool kP>
 __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const LaneGeom<T> &g, const T et[9],
-                                            T out[3][3][9]) {
+                                            T out[3][3][9], const T pc[4], T acc[4]) {
   const T d0 = (T)kD[c][0] * g.az, d1 = (T)kD[c][1] * g.az, d2 = (T)kD[c][2] * g.az;
   T W[3][9];
 #pragma unroll
@@ -79,11 +87,28 @@ __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const La
         G[1][l] = ldot<T>(b, g.cy, U[l][a], U[l][3 + a], U[l][6 + a]);
         G[2][l] = Z[l][p];
       }
-      const T t = et[p] * ((T)(kW[a] * kW[b] * kW[c]) * g.vol), t2 = t + t;
+      const T wv = (T)(kW[a] * kW[b] * kW[c]) * g.vol, t = et[p] * wv, t2 = t + t;
       T sg[3][3];
-      sg[0][0] = t2 * G[0][0];
-      sg[1][1] = t2 * G[1][1];
-      sg[2][2] = t2 * G[2][2];
+      if constexpr (kP) {
+        T pq = pc[0];
+        if (a != 1) pq += a == 0 ? -pc[1] : pc[1];
+        if (b != 1) pq += b == 0 ? -pc[2] : pc[2];
+        if (c != 1) pq += c == 0 ? -pc[3] : pc[3];
+        const T wp = wv * pq, wd = wv * (G[0][0] + G[1][1] + G[2][2]);
+        acc[0] -= wd;
+        if (a != 1) acc[1] += a == 0 ? wd : -wd;
+        if (b != 1) acc[2] += b == 0 ? wd : -wd;
+        if (c != 1) acc[3] += c == 0 ? wd : -wd;
+#pragma unroll
+        for (int i = 0; i < 4; i++) asm volatile("" : "+v"(acc[i]));
+        sg[0][0] = t2 * G[0][0] - wp;
+        sg[1][1] = t2 * G[1][1] - wp;
+        sg[2][2] = t2 * G[2][2] - wp;
+      } else {
+        sg[0][0] = t2 * G[0][0];
+        sg[1][1] = t2 * G[1][1];
+        sg[2][2] = t2 * G[2][2];
+      }
       sg[0][1] = sg[1][0] = t * (G[0][1] + G[1][0]);
       sg[0][2] = sg[2][0] = t * (G[0][2] + G[2][0]);
       sg[1][2] = sg[2][1] = t * (G[1][2] + G[2][1]);
@@ -104,11 +129,13 @@ __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const La
 // element sums.  bcp: per tile column and node plane, whether the tile's nodes
 // there have a Dirichlet dof.  ax: 2 / h of the mx element columns, the my
 // rows and the mz layers.
-template <typename T, LaneBC kBC>
+// kP: the saddle-point product with p, yp the pressures (4 per element).
+template <typename T, LaneBC kBC, bool kP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
     a11_lane_kernel(TileArgs a, const T *__restrict__ ax, const T *__restrict__ eta,
                     const uint8_t *__restrict__ bcn, const uint8_t *__restrict__ bcp, const T *__restrict__ u,
-                    T *__restrict__ y, T *__restrict__ fbx, T *__restrict__ fby, T *__restrict__ fbz) {
+                    const T *__restrict__ p, T *__restrict__ y, T *__restrict__ yp, T *__restrict__ fbx,
+                    T *__restrict__ fby, T *__restrict__ fbz) {
   // five plane slots: the layer's three planes and the next layer's two
   __shared__ T sm[5 * kLSlot];
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
@@ -176,7 +203,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     // The loads of a plane are in flight during its forward stage only: held
     // through the stress stage, the compiler would wait for each of them at
     // once to move it out of the registers that stage needs.
-    T et[9], r[kLBatch], U[3][9], Z[3][9];
+    T et[9], r[kLBatch], U[3][9], Z[3][9], pc[4], acc[4] = {T(0), T(0), T(0), T(0)};
+    const long e4 = 4 * (tb.x0 + (long)a.mx * (tb.y0 + (long)a.my * ek)) + 4 * (q.cx + a.mx * q.cy);
+    if constexpr (kP) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) pc[i] = p[e4 + i];
+    }
     int lq = q.li;
     auto forward = [&](auto c) {
       constexpr int C = decltype(c)::value;
@@ -190,7 +222,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     lane_rows_load<T, 0>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 0>());
     lane_rows_store<T, 0>(r, q, s3, s4);
-    lane_stress<T, 0>(U, Z, g, et, out);
+    if constexpr (kP) {
+#pragma unroll
+      for (int i = 1; i < 4; i++) pc[i] *= (T)(0.5 * kS);
+    }
+    lane_stress<T, 0, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
     // the node values are read again per quadrature plane, not held: an
     // index the compiler knows nothing about keeps it from merging the reads
@@ -200,7 +236,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     lane_rows_load<T, 1>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 1>());
     lane_rows_store<T, 1>(r, q, s3, s4);
-    lane_stress<T, 1>(U, Z, g, et, out);
+    lane_stress<T, 1, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
     asm volatile("" : "+v"(lq));
 #pragma unroll
@@ -208,8 +244,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     lane_rows_load<T, 2>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 2>());
     lane_rows_store<T, 2>(r, q, s3, s4);
-    lane_stress<T, 2>(U, Z, g, et, out);
+    lane_stress<T, 2, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
+    if constexpr (kP) {
+      if (q.live) {
+        yp[e4] = acc[0];
+#pragma unroll
+        for (int i = 1; i < 4; i++) yp[e4 + i] = (T)(0.5 * kS) * acc[i];
+      }
+    }
     if (more && ((bits >> (2 * kz + 3)) & 1)) lane_rows_mask<T>(s3, q, a.X, mask(nn));
     if (more && ((bits >> (2 * kz + 4)) & 1)) lane_rows_mask<T>(s4, q, a.X, mask(nn + 1));
     __syncthreads();

@@ -12,8 +12,8 @@ import pytest
 from oracle import oracle as O
 from ptatin3d_amd import fields as F
 from ptatin3d_amd._lib import DeviceArray, call
-from ptatin3d_amd.multigrid import GMG, default_options
-from ptatin3d_amd.operators import MatA11MF
+from ptatin3d_amd.multigrid import GMG, default_options, stokes_solve_timed
+from ptatin3d_amd.operators import MatA11MF, MatStokesMF
 
 from conftest import rel_inf
 
@@ -135,3 +135,49 @@ def test_lane_smoother_takes_dirichlet_rows_itself(gpu):
     mg.smooth(3, db, dx, 3, True)
     assert rel_inf(dx.download(), p[-1]) <= 1e-12
     mg.destroy()
+
+
+@pytest.mark.parametrize("m", [b for b, prec in BOXES if prec == 64])
+def test_lane_saddle_point_parity(gpu, m):
+    """MatMult_MFStokes_A with one lane per element = oracle A11 + A12 and A21."""
+    coords, eta, bc, u = _case(m, 9)
+    p = np.random.default_rng(10).uniform(-1.0, 1.0, 4 * m[0] * m[1] * m[2])
+    A = MatStokesMF(*m).setup(coords, eta, bc)
+    yu, yp = A.stokes_host(u, p)
+    ou = O.a11_matmult(*m, coords, eta, bc, u) + O.a12_matmult(*m, coords, bc, p)
+    op = O.a21_matmult(*m, coords, bc, u)
+    assert rel_inf(yu, ou) <= 1e-12
+    assert rel_inf(yp, op) <= 1e-12
+    d = bc.astype(bool)
+    assert np.array_equal(yu[d], u[d])
+    A.set_tiles_per_group(2)  # the tile kernel on the same operator
+    yu, yp = A.stokes_host(u, p)
+    assert rel_inf(yu, ou) <= 1e-12
+    assert rel_inf(yp, op) <= 1e-12
+    A.destroy()
+
+
+def test_lane_saddle_point_in_fp32_preconditioner(gpu):
+    """The FP32 velocity preconditioner forms its A12 product with the FP32
+    saddle-point kernel.  Its rounding, 1e-5 of the product, cannot show in a
+    Krylov method's iterations to 1e-6 but for one at either end; a wrong
+    product does."""
+    m = (40, 32, 32)
+    rng = np.random.default_rng(12)
+    coords = F.box_coords(*m)
+    eta = F.eta_loguniform(m[0] * m[1] * m[2], 0.1, 10.0, rng)
+    its = []
+    for prec in (64, 32):
+        mg = GMG(*m, 3)
+        mg.set_coordinates(coords)
+        mg.set_viscosity(2, eta)
+        mg.coarsen_viscosity()
+        mg.set_dirichlet_all_faces()
+        mg.setup(default_options(smoother_precision=prec))
+        mg.stokes_setup()
+        bu, bp = F.smooth_body_force(coords, *m), np.zeros(4 * m[0] * m[1] * m[2])
+        out = stokes_solve_timed(mg, bu, bp, rtol=1e-6, maxit=200, restart=60)
+        assert out[3] <= 1e-6 * np.linalg.norm(bu) * 1.5
+        its.append(out[2])
+        mg.destroy()
+    assert abs(its[0] - its[1]) <= 1, its
