@@ -440,9 +440,7 @@ int ptmf_op_synchronize(ptmf_op op) {
 int ptmf_a11_diagonal(ptmf_op op, double *d) {
   PTMF_TRY(check_ready(op, true, true));
   PTMF_CHECK(d, PTMF_ERR_ARG, "a11_diagonal: null");
-  PTMF_TRY(ptmf::launch_fill<double>(d, 0.0, 3 * op->box.nnodes, op->stream));
   PTMF_TRY(ptmf::launch_a11_diag(op, d));
-  PTMF_TRY(ptmf::launch_bc_set<double>(op->bcidx, op->nbc, 1.0, d, op->stream));
   PTMF_HIP(hipStreamSynchronize(op->stream));
   return PTMF_OK;
 }

@@ -32,26 +32,11 @@ __device__ __forceinline__ double pick3(int i, double v0, double v1, double v2) 
   return i == 0 ? v0 : (i == 1 ? v1 : v2);
 }
 
-// The 1-D tables as one lane sees them, in registers.  A lane that owns
-// quadrature point (qa, qb, qc) holds rows: B[d][r] = kB[q_d][r]; a lane that
-// owns node (i, j, k) holds columns: B[d][a] = kB[a][n_d].  tab_grad(T, x, y,
-// z) is then the reference gradient of the (node, point) pair whose other
-// index is (x, y, z), with static register indices when x, y, z are
-// compile-time (unrolled loops).
+// The columns of the 1-D tables of a lane that owns node (i, j, k), in
+// registers: B[d][a] = kB[a][n_d].
 struct LaneTab {
   double B[3][3], D[3][3];
 };
-
-__device__ __forceinline__ void lane_tab_qp(int q, LaneTab &T) {
-  const int qd[3] = {q % 3, (q / 3) % 3, q / 9};
-#pragma unroll
-  for (int d = 0; d < 3; d++)
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-      T.B[d][r] = pick3(qd[d], kB[0][r], kB[1][r], kB[2][r]);
-      T.D[d][r] = pick3(qd[d], kD[0][r], kD[1][r], kD[2][r]);
-    }
-}
 
 __device__ __forceinline__ void lane_tab_node(int n, LaneTab &T) {
   const int nd[3] = {n % 3, (n / 3) % 3, n / 9};
@@ -62,12 +47,6 @@ __device__ __forceinline__ void lane_tab_node(int n, LaneTab &T) {
       T.B[d][a] = pick3(nd[d], kB[a][0], kB[a][1], kB[a][2]);
       T.D[d][a] = pick3(nd[d], kD[a][0], kD[a][1], kD[a][2]);
     }
-}
-
-__device__ __forceinline__ void tab_grad(const LaneTab &T, int x, int y, int z, double gr[3]) {
-  gr[0] = T.D[0][x] * T.B[1][y] * T.B[2][z];
-  gr[1] = T.B[0][x] * T.D[1][y] * T.B[2][z];
-  gr[2] = T.B[0][x] * T.B[1][y] * T.D[2][z];
 }
 
 __device__ void qp_geometry(const double (*xe)[3], int q, QpGeom &g) {
@@ -146,61 +125,6 @@ __device__ __forceinline__ void p1_basis(const double (*xe)[3], const double xq[
   const double L[3] = {xe[14][0] - xe[12][0], xe[16][1] - xe[10][1], xe[22][2] - xe[4][2]};
   Np[0] = 1.0;
   for (int d = 0; d < 3; d++) Np[1 + d] = (xq[d] - (1.0 / 27.0) * avg[d]) / L[d];
-}
-
-// ---- diag(A11): d[3n+c] += sum_q w detJ eta (|grad N_n|^2 + (d_c N_n)^2)
-// (MFStokesWrapper_diagA11, stokes_operators_mf.c:67-131 with
-// MatMultMF_Stokes_MixedFEM3d_diagB11, stokes_q2p1_mf_operators_diag_def.c:120-205)
-__global__ void __launch_bounds__(64)
-    a11_diag_kernel(int mx, int my, int mz, long nel, long X, long XY, int color, const double *__restrict__ xc,
-                    const double *__restrict__ eta, double *__restrict__ dg) {
-  __shared__ double sx[kEPB][27][3];
-  __shared__ double sG[kEPB][27][10];
-  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
-  // elements of one parity class: their sums go in with plain read-add-write
-  bool live;
-  const long e = class_element(mx, my, mz, color, (long)blockIdx.x * kEPB + h, live);
-  if (t < 27) {
-    const long node = elem_node(mx, my, X, XY, e, t);
-    for (int d = 0; d < 3; d++) sx[h][t][d] = xc[3 * node + d];
-  }
-  __syncthreads();
-  if (t < 27) {
-    QpGeom g;
-    qp_geometry(sx[h], t, g);
-    for (int r = 0; r < 3; r++)
-      for (int s = 0; s < 3; s++) sG[h][t][3 * r + s] = g.G[r][s];
-    sG[h][t][9] = g.wdet * eta[(long)t * nel + e];
-  }
-  __syncthreads();
-  if (t < 27 && live) {
-    LaneTab T;
-    lane_tab_node(t, T);
-    double acc[3] = {0, 0, 0};
-    // one quadrature plane per trip (the unrolled 9 points keep their
-    // geometry loads in registers; all 27 at once would spill)
-#pragma unroll 1
-    for (int qc = 0; qc < 3; qc++) {
-      const double bk = pick3(qc, T.B[2][0], T.B[2][1], T.B[2][2]), dk = pick3(qc, T.D[2][0], T.D[2][1], T.D[2][2]);
-#pragma unroll
-      for (int qb = 0; qb < 3; qb++)
-#pragma unroll
-        for (int qa = 0; qa < 3; qa++) {
-          const double *G = sG[h][qa + 3 * qb + 9 * qc];
-          const double gr[3] = {T.D[0][qa] * T.B[1][qb] * bk, T.B[0][qa] * T.D[1][qb] * bk,
-                                T.B[0][qa] * T.B[1][qb] * dk};
-          double gp[3];
-#pragma unroll
-          for (int k = 0; k < 3; k++) gp[k] = G[3 * k] * gr[0] + G[3 * k + 1] * gr[1] + G[3 * k + 2] * gr[2];
-          const double s = G[9];
-          const double g2 = gp[0] * gp[0] + gp[1] * gp[1] + gp[2] * gp[2];
-#pragma unroll
-          for (int c = 0; c < 3; c++) acc[c] += s * (g2 + gp[c] * gp[c]);
-        }
-    }
-    const long node = elem_node(mx, my, X, XY, e, t);
-    for (int c = 0; c < 3; c++) dg[3 * node + c] += acc[c];
-  }
 }
 
 // ---- l1 row sums of A11 with the MatMult's boundary handling, an upper
@@ -466,57 +390,6 @@ __global__ void schur_apply_kernel(long nel, const double *__restrict__ Minv, co
   }
 }
 
-// ---- strain-rate-dependent viscosity at the quadrature points:
-// eta = clip(B * max(eII, 1e-17)^(1/n - 1)), eII = sqrt(0.5 D:D), D = sym(grad u)
-// (ComputeStrainRate3d / ComputeSecondInvariant3d, stokes_rheology_vp_std.c:85-148;
-// the VISCOUS_ARRHENIUS_2 power law, stokes_rheology_vp_std.c:437-461, with the
-// prefactor B per quadrature point).  Element-major input B and output eta.
-__global__ void __launch_bounds__(64)
-    powerlaw_kernel(int mx, int my, long nel, long X, long XY, const double *__restrict__ xc,
-                    const double *__restrict__ u, const double *__restrict__ B, double nexp, double eta_min,
-                    double eta_max, double *__restrict__ eta) {
-  __shared__ double sx[kEPB][27][3];
-  __shared__ double su[kEPB][27][3];
-  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
-  long e = (long)blockIdx.x * kEPB + h;
-  const bool live = e < nel;
-  if (!live) e = nel - 1;
-  if (t < 27) {
-    const long node = elem_node(mx, my, X, XY, e, t);
-    for (int d = 0; d < 3; d++) {
-      sx[h][t][d] = xc[3 * node + d];
-      su[h][t][d] = u[3 * node + d];
-    }
-  }
-  __syncthreads();
-  if (t < 27 && live) {
-    QpGeom g;
-    qp_geometry(sx[h], t, g);
-    double L[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // L[l][k] = d u_l / d x_k
-    LaneTab T;
-    lane_tab_qp(t, T);
-#pragma unroll
-    for (int n = 0; n < 27; n++) {
-      double gr[3], gp[3];
-      tab_grad(T, n % 3, (n / 3) % 3, n / 9, gr);
-      for (int k = 0; k < 3; k++) gp[k] = g.G[k][0] * gr[0] + g.G[k][1] * gr[1] + g.G[k][2] * gr[2];
-      for (int l = 0; l < 3; l++)
-        for (int k = 0; k < 3; k++) L[l][k] += su[h][n][l] * gp[k];
-    }
-    double sum = 0.0;
-    for (int l = 0; l < 3; l++)
-      for (int k = 0; k < 3; k++) {
-        const double dlk = 0.5 * (L[l][k] + L[k][l]);
-        sum += dlk * dlk;
-      }
-    double sr = sqrt(0.5 * sum);
-    if (sr < 1.0e-17) sr = 1.0e-17;
-    double v = B[27 * e + t] * pow(sr, 1.0 / nexp - 1.0);
-    v = fmin(fmax(v, eta_min), eta_max);
-    eta[27 * e + t] = v;
-  }
-}
-
 int init_constants() {
   static bool done = false;
   if (done) return PTMF_OK;
@@ -528,20 +401,6 @@ int init_constants() {
 }
 
 }  // namespace
-
-int launch_a11_diag(const ptmf_op_s *op, double *d) {
-  PTMF_TRY(init_constants());
-  const Box &b = op->box;
-  for (int color = 0; color < 8; color++) {
-    const long ncol = class_count(b, color);
-    if (ncol == 0) continue;
-    const long nblk = (ncol + kEPB - 1) / kEPB;
-    a11_diag_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(
-        b.mx, b.my, b.mz, b.nel, b.X, b.X * b.Y, color, op->d64.coords, op->d64.eta, d);
-    PTMF_HIP(hipGetLastError());
-  }
-  return PTMF_OK;
-}
 
 int launch_a11_l1(const ptmf_op_s *op, double *d) {
   PTMF_TRY(init_constants());
@@ -579,18 +438,6 @@ int launch_schur_apply(const ptmf_op_s *op, const double *Minv, const double *rp
   long nb = (n + 255) / 256;
   if (nb > 65536) nb = 65536;
   schur_apply_kernel<<<dim3((unsigned)nb), dim3(256), 0, op->stream>>>(op->box.nel, Minv, rp, yp);
-  PTMF_HIP(hipGetLastError());
-  return PTMF_OK;
-}
-
-int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, double nexp, double eta_min,
-                    double eta_max, double *eta) {
-  PTMF_TRY(init_constants());
-  const Box &b = op->box;
-  const long nblk = (b.nel + kEPB - 1) / kEPB;
-  powerlaw_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.nel, b.X, b.X * b.Y,
-                                                                     op->d64.coords, u, B, nexp, eta_min,
-                                                                     eta_max, eta);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

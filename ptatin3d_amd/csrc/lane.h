@@ -281,7 +281,8 @@ __device__ __forceinline__ void lane_window(T *w, bool moreX, bool moreY, const 
 enum LaneBC {
   kLaneSums,  // left as the element sums
   kLaneCopy,  // y = x
-  kLaneZero   // y = 0
+  kLaneZero,  // y = 0
+  kLaneOne    // y = 1
 };
 
 // Writes a completed node plane P: the tile's own nodes to y (or, on the
@@ -316,7 +317,7 @@ __device__ __forceinline__ void lane_flush(const TileArgs &a, const LaneTile &q,
       for (int j = 0; j < kLRows; j++) {
         const unsigned row = X * (unsigned)min(j, nyo - 1);
         m[j] = b.load((unsigned)il, row);
-        xv[j] = kBC == kLaneCopy ? xb.load(S * (unsigned)lane, 3 * S * row) : T(0);
+        xv[j] = kBC == kLaneCopy ? xb.load(S * (unsigned)lane, 3 * S * row) : T(kBC == kLaneOne ? 1 : 0);
       }
       __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the first is used
 #pragma unroll

@@ -1,0 +1,45 @@
+"""The diagonal of A11 and the power-law viscosity with one lane per element, at
+the sizes where they can go wrong: partial 8 x 8 tiles in either direction, one
+to many layers a chunk and a shorter last one, one element, Dirichlet dofs
+inside the box, sheared elements (the diagonal's mixed products are large) and
+velocities at rest.
+
+Tolerance: 1e-12 relative to the oracle, the FP64 bar of both operators."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from ptatin3d_amd import fields as F
+from ptatin3d_amd._lib import DeviceArray
+from ptatin3d_amd.operators import MatA11MF
+
+from conftest import rel_inf
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [(1, 1, 1), (8, 1, 2), (9, 5, 4), (17, 9, 11), (8, 8, 70), (30, 28, 33)])
+def test_diagonal_and_powerlaw_parity(gpu, m):
+    rng = np.random.default_rng(4)
+    E = m[0] * m[1] * m[2]
+    coords = F.perturb_interior(F.box_coords(*m), *m, 0.1, rng).reshape(-1, 3)
+    coords[:, 0] += 0.7 * coords[:, 1] - 0.4 * coords[:, 2]
+    coords = coords.reshape(-1)
+    bc = F.dirichlet_all_faces(*m)
+    bc[rng.integers(0, bc.size, bc.size // 20)] = 1
+    eta = F.eta_loguniform(E, 1e-2, 1e2, rng)
+    A = MatA11MF(*m).setup(coords, eta, bc)
+    d = A.diagonal_host()
+    assert rel_inf(d, O.a11_diagonal(*m, coords, eta, bc)) <= 1e-12
+    assert np.all(d[bc.astype(bool)] == 1.0)
+    assert np.array_equal(d, A.diagonal_host())  # no atomics: repeats are bit-identical
+
+    u, B = rng.uniform(-1.0, 1.0, (F.nnodes(*m), 3)), 10.0 ** rng.uniform(-2.0, 2.0, 27 * E)
+    u[: u.shape[0] // 3] = 0.0  # at rest: the floor of the strain rate
+    ref = O.powerlaw_eta(*m, coords, u.reshape(-1), B, 3.0, 1e-3, 1e3)
+    du, dB, de = DeviceArray.from_host(u.reshape(-1)), DeviceArray.from_host(B), DeviceArray(27 * E)
+    A.powerlaw_viscosity(du, dB, 3.0, 1e-3, 1e3, de)
+    assert rel_inf(de.download(), ref) <= 1e-12
+    A.powerlaw_viscosity(du, dB, 3.0, 1e-3, 1e3, dB)  # in place
+    assert np.array_equal(dB.download(), de.download())
+    A.destroy()
