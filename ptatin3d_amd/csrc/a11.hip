@@ -1047,11 +1047,33 @@ __global__ void __launch_bounds__(64)
 // wave would walk one dependent load/store round after another.
 constexpr int kFaceThreads = 256;
 
-template <typename T, bool kSkip = false>
+template <typename T>
 __global__ void __launch_bounds__(kFaceThreads)
     a11_face_kernel(TileArgs a, const T *__restrict__ fbx, const T *__restrict__ fby,
-                    const T *__restrict__ fbz, T *__restrict__ y, const uint8_t *__restrict__ bcn = nullptr) {
-  face_sum<T, kSkip>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
+                    const T *__restrict__ fbz, T *__restrict__ y) {
+  face_sum<T>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y);
+}
+
+// The same with the Dirichlet rows y = x, which the face sums leave alone: the
+// work-groups past the tiles copy them, beside the others' face sums and not
+// after them (64^3: 15 us for the faces alone and for both, a launch of its own
+// took 5 us more; copied by the lane kernel as it writes the other rows 16 us).
+constexpr int kCopyGroup = 8 * kFaceThreads;  // rows per work-group
+template <typename T>
+__global__ void __launch_bounds__(kFaceThreads)
+    a11_face_copy_kernel(TileArgs a, const T *__restrict__ fbx, const T *__restrict__ fby, const T *__restrict__ fbz,
+                         T *__restrict__ y, const uint8_t *__restrict__ bcn, const long *__restrict__ bcidx, long nbc,
+                         const T *__restrict__ x) {
+  if (blockIdx.x < a.ntiles) {
+    face_sum<T, true>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
+    return;
+  }
+  const long i0 = (long)kCopyGroup * (blockIdx.x - a.ntiles);
+#pragma unroll
+  for (int k = 0; k < kCopyGroup / kFaceThreads; k++) {
+    const long i = i0 + kFaceThreads * k + threadIdx.x;
+    if (i < nbc) y[bcidx[i]] = x[bcidx[i]];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1130,14 +1152,14 @@ TileArgs tile_args(const ptmf_op_s *op) {
 // rounds the Jacobian off by more than 1e-5, and the two kernels would differ
 // by that), and where the tile kernel is faster.
 // The costs are microseconds per round of one wave on each of the 1024 SIMDs,
-// times the layers a wave marches through.  Measured at 64^3 with the chip
-// full, FP64: 18.1 us per layer of 64 elements (lane) and 14.6 us per layer of
-// 20 (tile); FP32, two waves per SIMD: 19.6 and 12.6 us for both, 13 and 10.5
-// us with one; the lane kernel's first and last planes add 0.45 of a layer.
-// So the tile kernel keeps the small boxes that it takes in one round (16^3:
-// 13.5 us against 19.3 us), and the lane kernel has the rest (45 x 37 x 29:
-// 25.7 us against 50.1 us, 64^3: 79.6 against 178 us, 128^3 MatMult 707
-// against 1480 us; FP32 20.7 against 25.5 and 48 against 82 us).
+// times the layers a wave marches through.  Measured on boxes from 8^3 to
+// 96 x 96 x 48, FP64: 14 us per layer of 64 elements (lane) and 14.6 us per
+// layer of 20 (tile); FP32, two waves per SIMD: 14.2 and 15.7 us for both, 10 and
+// 10.5 us with one; the lane kernel's first and last planes add 0.57 (0.45) of a
+// layer.  So the tile kernel keeps the boxes that it takes in one round (16^3:
+// 13.5 us against 15.6 us; 20^3: 15.6 and 16.0 us), and the lane kernel has the
+// rest (28^3: 17.8 us against 33.6 us, FP32 13.7 and 17.2 us; 48 x 48 x 32: 32
+// and 71 us, FP32 18 and 31 us; 64^3: 63 and 178 us, FP32 35 and 82 us).
 template <typename T>
 double lane_rounds(long waves, double one, double two) {
   const long r = (waves + 1023) / 1024;
@@ -1157,14 +1179,14 @@ bool lane_plan(const Box &b, const Tiling &t, TileArgs &a) {
   double best = 1e300;
   for (int zc = 1; zc <= b.mz && zc <= kLMaxZ; zc++) {
     const long nt = txy * ((b.mz + zc - 1) / zc);
-    const double cost = (zc + 0.45) * lane_rounds<T>(nt, f64 ? 18.1 : 13.0, 19.6);
+    const double cost = (zc + (f64 ? 0.57 : 0.45)) * lane_rounds<T>(nt, f64 ? 14.0 : 10.0, 14.2);
     if (cost < best) {
       best = cost;
       a.ZC = zc;
       a.ntiles = nt;
     }
   }
-  if (best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 12.6)) return false;
+  if (best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 15.7)) return false;
   a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
   a.fbz_n = kLRows * kLRows;
   // byte offsets of the 27 quadrature points' viscosities and of 17 node rows
@@ -1227,32 +1249,32 @@ __global__ void __launch_bounds__(256)
   if (__any(off) && (threadIdx.x & 63) == 0) *bad = 1;
 }
 
-// per tile column of the lane kernel and node plane: 1 if one of the tile's
-// nodes in the plane has a Dirichlet dof
+// lane_bc_word of every tile column of the lane kernels and node plane
 __global__ void __launch_bounds__(64)
-    bc_plane_kernel(int mx, int my, int ntx, long X, long XY, long Z, const uint8_t *__restrict__ bcn,
-                    uint8_t *__restrict__ flags) {
+    bc_word_kernel(int mx, int my, int ntx, long X, long XY, long Z, const uint8_t *__restrict__ bcn,
+                   unsigned *__restrict__ words) {
   const long col = blockIdx.x / Z, P = blockIdx.x - col * Z;
   const int tx = (int)(col % ntx), ty = (int)(col / ntx);
   const int x0 = kLT * tx, y0 = kLT * ty, wX = 2 * min(kLT, mx - x0) + 1, wY = 2 * min(kLT, my - y0) + 1;
-  unsigned any = 0;
-  for (int t = threadIdx.x; t < wX * wY; t += 64) any |= bcn[2 * x0 + t % wX + X * (2 * y0 + t / wX) + XY * P];
-  any = __any(any != 0);
-  if (threadIdx.x == 0) flags[blockIdx.x] = any ? 1 : 0;
+  const int il = threadIdx.x / 3, d = threadIdx.x - 3 * il;
+  unsigned w = 0;
+  if (il < wX)
+    for (int j = 0; j < wY; j++) w |= ((bcn[2 * x0 + il + X * (2 * y0 + j) + XY * P] >> d) & 1u) << j;
+  words[64L * blockIdx.x + threadIdx.x] = w;
 }
 
 }  // namespace
 
 int alloc_lane_data(ptmf_op_s *op) {
   // one allocation: 2 / h in FP64 (and three tolerances) and FP32, the
-  // classification's flag, the plane flags
+  // classification's flag, the Dirichlet words
   const Box &b = op->box;
   const long na = b.mx + b.my + b.mz;
   const long planes = (long)((b.mx + kLT - 1) / kLT) * ((b.my + kLT - 1) / kLT) * b.Z;
-  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) + planes));
+  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) + 64 * sizeof(unsigned) * planes));
   op->ax32 = (float *)(op->ax64 + na + 3);
   op->rect_bad = (int *)(op->ax32 + na);
-  op->bcplane = (uint8_t *)(op->rect_bad + 1);
+  op->bcword = (unsigned *)(op->rect_bad + 1);
   return PTMF_OK;
 }
 
@@ -1260,8 +1282,8 @@ int mark_dirichlet_planes(ptmf_op_s *op) {
   const Box &b = op->box;
   const int ntx = (b.mx + kLT - 1) / kLT, nty = (b.my + kLT - 1) / kLT;
   const long n = (long)ntx * nty * b.Z;
-  bc_plane_kernel<<<dim3((unsigned)n), 64, 0, op->stream>>>(b.mx, b.my, ntx, b.X, b.X * b.Y, b.Z, op->bcnode,
-                                                            op->bcplane);
+  PTMF_CHECK(n < (1L << 31), PTMF_ERR_ARG, "set_dirichlet: mesh too large");
+  bc_word_kernel<<<dim3((unsigned)n), 64, 0, op->stream>>>(b.mx, b.my, ntx, b.X, b.X * b.Y, b.Z, op->bcnode, op->bcword);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }
@@ -1419,18 +1441,31 @@ int eta_tiled_in_place(ptmf_op_s *op) {
   return PTMF_OK;
 }
 
+// the face sums and the Dirichlet rows
+template <typename T>
+int launch_face_copy(const ptmf_op_s *op, const TileArgs &a, const T *fbx, const T *fby, const T *fbz, const T *x,
+                     T *y) {
+  const long groups = a.ntiles + (op->nbc + kCopyGroup - 1) / kCopyGroup;
+  PTMF_CHECK(groups < (1L << 31), PTMF_ERR_ARG, "a11: mesh too large (%ld work-groups)", groups);
+  a11_face_copy_kernel<T><<<dim3((unsigned)groups), dim3(kFaceThreads), 0, op->stream>>>(
+      a, fbx, fby, fbz, y, op->bcnode, op->bcidx, op->nbc, x);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
 // the lane kernel (lane_tiles must hold) and its faces
-template <typename T, LaneBC kBC, bool kP>
+template <typename T, bool kP>
 int launch_lane(const ptmf_op_s *op, const TileArgs &a, int faces, const T *x, const T *p, T *y, T *yp, T *fb) {
   const T *ax = sizeof(T) == 8 ? (const T *)op->ax64 : (const T *)op->ax32;
   const T *eta = sizeof(T) == 8 ? (const T *)op->d64.eta : (const T *)op->d32.eta;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
-  const dim3 grid((unsigned)a.ntiles);
-  a11_lane_kernel<T, kBC, kP><<<grid, dim3(64), 0, op->stream>>>(a, ax, eta, op->bcnode, op->bcplane, x, p, y, yp, fbx,
-                                                                   fby, fbz);
+  a11_lane_kernel<T, kP><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, ax, eta, op->bcword, x, p, y, yp, fbx,
+                                                                               fby, fbz);
   PTMF_HIP(hipGetLastError());
-  if (!faces) return PTMF_OK;
-  a11_face_kernel<T, kBC == kLaneCopy><<<grid, dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y, op->bcnode);
+  if (faces == 1)
+    PTMF_TRY(launch_face_copy<T>(op, a, fbx, fby, fbz, x, y));
+  else if (faces)
+    a11_face_kernel<T><<<dim3((unsigned)a.ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }
@@ -1463,10 +1498,8 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
     return PTMF_OK;
   }
   TileArgs la;
-  if (variant == 0 && lane_tiles<T>(op, fb_doubles, la)) {
-    if (faces == 2) return launch_lane<T, kLaneSums, false>(op, la, faces, x, nullptr, y, nullptr, fb);
-    return launch_lane<T, kLaneCopy, false>(op, la, faces, x, nullptr, y, nullptr, fb);
-  }
+  if (variant == 0 && lane_tiles<T>(op, fb_doubles, la))
+    return launch_lane<T, false>(op, la, faces, x, nullptr, y, nullptr, fb);
   const TileArgs a = tile_args(op);
   const long ntiles = tl.ntiles;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * ntiles, *fbz = fby + 3 * a.fby_n * ntiles;
@@ -1494,10 +1527,10 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
           a, d.coords, et, op->bcnode, x, y, fbx, fby, fbz);
   }
   PTMF_HIP(hipGetLastError());
+  if (faces == 1) return launch_face_copy<T>(op, a, fbx, fby, fbz, x, y);
   if (faces) {
     a11_face_kernel<T><<<dim3((unsigned)ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y);
     PTMF_HIP(hipGetLastError());
-    if (faces == 1) PTMF_TRY(launch_bc_copy<T>(op->bcidx, op->nbc, x, y, op->stream));
   }
   return PTMF_OK;
 }
@@ -1520,7 +1553,7 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   // lane kernel 41 us and the tile kernel 62 us, and further apart above)
   TileArgs la;
   if (lane_tiles<T>(op, op->faces_doubles, la))
-    return launch_lane<T, kLaneCopy, true>(op, la, 1, x, x + nu, y, y + nu, (T *)op->faces);
+    return launch_lane<T, true>(op, la, 1, x, x + nu, y, y + nu, (T *)op->faces);
   PTMF_TRY(ensure_eta_tiled<T>(op));
   const T *et = sizeof(T) == 8 ? (const T *)op->et64 : (const T *)op->et32;
   const TileArgs a = tile_args(op);
@@ -1529,10 +1562,7 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   stokes_tile_kernel<T><<<dim3((unsigned)ntiles), dim3(64), 0, op->stream>>>(
       a, d.coords, et, op->bcnode, x, x + nu, y, y + nu, fbx, fby, fbz);
   PTMF_HIP(hipGetLastError());
-  a11_face_kernel<T><<<dim3((unsigned)ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y);
-  PTMF_HIP(hipGetLastError());
-  PTMF_TRY(launch_bc_copy<T>(op->bcidx, op->nbc, x, y, op->stream));
-  return PTMF_OK;
+  return launch_face_copy<T>(op, a, fbx, fby, fbz, x, y);
 }
 
 int launch_stokes_mult(ptmf_op_s *op, const double *x, double *y) { return launch_stokes_mult_t<double>(op, x, y); }

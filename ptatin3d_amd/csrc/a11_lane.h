@@ -125,26 +125,22 @@ __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const La
     lane_field_t<T, c>(W[l], Z[l], d0, d1, d2, out[0][l], out[1][l], out[2][l]);
 }
 
-// kBC: Dirichlet rows y = x (the face pass leaves them alone) or left as the
-// element sums.  bcp: per tile column and node plane, whether the tile's nodes
-// there have a Dirichlet dof.  ax: 2 / h of the mx element columns, the my
-// rows and the mz layers.
+// Dirichlet rows are left as the element sums.  bcw: lane_bc_word's.  ax: 2 / h
+// of the mx element columns, the my rows and the mz layers.
 // kP: the saddle-point product with p, yp the pressures (4 per element).
-template <typename T, LaneBC kBC, bool kP>
+template <typename T, bool kP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
     a11_lane_kernel(TileArgs a, const T *__restrict__ ax, const T *__restrict__ eta,
-                    const uint8_t *__restrict__ bcn, const uint8_t *__restrict__ bcp, const T *__restrict__ u,
-                    const T *__restrict__ p, T *__restrict__ y, T *__restrict__ yp, T *__restrict__ fbx,
+                    const unsigned *__restrict__ bcw, const T *__restrict__ u, const T *__restrict__ p,
+                    T *__restrict__ y, T *__restrict__ yp, T *__restrict__ fbx,
                     T *__restrict__ fby, T *__restrict__ fbz) {
   // five plane slots: the layer's three planes and the next layer's two
   __shared__ T sm[5 * kLSlot];
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
-  const unsigned long long bits = lane_bc_bits(a, q, bcp);
   // 2 / hz of the chunk's layers, one per lane
   const T szs = ax[a.mx + a.my + tb.z0 + min(q.lane, tb.nzt - 1)];
   auto plane = [&](int P) { return LaneBuf<T>(u + 3 * lane_node(a, tb, P)); };
-  auto mask = [&](int P) { return LaneBuf<uint8_t>(bcn + lane_node(a, tb, P)); };
 
   LaneGeom<T> g;
   const T sx = ax[tb.x0 + q.cx], sy = ax[a.mx + tb.y0 + q.cy];
@@ -158,18 +154,23 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
   {
     const LaneBuf<T> v0 = plane(2 * tb.z0), v1 = plane(2 * tb.z0 + 1), v2 = plane(2 * tb.z0 + 2);
     T r0[kLBatch], r1[kLBatch], r2[kLBatch];
+    const unsigned m0 = lane_bc_word(a, q, bcw, 2 * tb.z0), m1 = lane_bc_word(a, q, bcw, 2 * tb.z0 + 1),
+                   m2 = lane_bc_word(a, q, bcw, 2 * tb.z0 + 2);
     lane_rows_load<T, 0>(r0, q, a.X, v0, v1);
     lane_rows_load<T, 1>(r1, q, a.X, v0, v1);
+    lane_rows_mask<T, 0>(r0, m0, m1);
     lane_rows_store<T, 0>(r0, q, sm, sm + kLSlot);
     lane_rows_load<T, 2>(r2, q, a.X, v0, v1);
+    lane_rows_mask<T, 1>(r1, m0, m1);
     lane_rows_store<T, 1>(r1, q, sm, sm + kLSlot);
     lane_rows_load<T, 0, kLRows>(r0, q, a.X, v2, v2);
     lane_rows_load<T, 1, kLRows>(r1, q, a.X, v2, v2);
+    lane_rows_mask<T, 2>(r2, m0, m1);
     lane_rows_store<T, 2>(r2, q, sm, sm + kLSlot);
+    lane_rows_mask<T, 0, kLRows>(r0, m2, 0u);
     lane_rows_store<T, 0, kLRows>(r0, q, sm + 2 * kLSlot, nullptr);
+    lane_rows_mask<T, 1, kLRows>(r1, m2, 0u);
     lane_rows_store<T, 1, kLRows>(r1, q, sm + 2 * kLSlot, nullptr);
-    for (int k = 0; k < 3; k++)
-      if ((bits >> k) & 1) lane_rows_mask<T>(sm + k * kLSlot, q, a.X, mask(2 * tb.z0 + k));
   }
   T out[3][3][9];
 #pragma unroll
@@ -184,9 +185,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     const int ek = tb.z0 + kz;
     auto place = [&](int k) { return sm + kLSlot * (slot + k >= 5 ? slot + k - 5 : slot + k); };
     T *const s0 = place(0), *const s1 = place(1), *const s2 = place(2), *const s3 = place(3), *const s4 = place(4);
-    const bool more = kz + 1 < tb.nzt;
     // (the last layer of the chunk loads its own planes again, into free slots)
-    const int nn = more ? 2 * ek + 3 : 2 * ek + 1;
+    const int nn = kz + 1 < tb.nzt ? 2 * ek + 3 : 2 * ek + 1;
     const LaneBuf<T> v1 = plane(nn), v2 = plane(nn + 1);
     const LaneBuf<T> eta_k(eta + tb.x0 + (long)a.mx * (tb.y0 + (long)a.my * ek));
     const T sz = __shfl(szs, kz);
@@ -219,8 +219,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     };
 #pragma unroll
     for (int p = 0; p < 9; p++) et[p] = eta_k.load(oe, qs * p);
+    const unsigned m3 = lane_bc_word(a, q, bcw, nn), m4 = lane_bc_word(a, q, bcw, nn + 1);
     lane_rows_load<T, 0>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 0>());
+    lane_rows_mask<T, 0>(r, m3, m4);
     lane_rows_store<T, 0>(r, q, s3, s4);
     if constexpr (kP) {
 #pragma unroll
@@ -235,6 +237,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     for (int p = 0; p < 9; p++) et[p] = eta_k.load(oe, qs * (9 + p));
     lane_rows_load<T, 1>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 1>());
+    lane_rows_mask<T, 1>(r, m3, m4);
     lane_rows_store<T, 1>(r, q, s3, s4);
     lane_stress<T, 1, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
@@ -243,6 +246,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     for (int p = 0; p < 9; p++) et[p] = eta_k.load(oe, qs * (18 + p));
     lane_rows_load<T, 2>(r, q, a.X, v1, v2);
     forward(std::integral_constant<int, 2>());
+    lane_rows_mask<T, 2>(r, m3, m4);
     lane_rows_store<T, 2>(r, q, s3, s4);
     lane_stress<T, 2, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
@@ -253,20 +257,18 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
         for (int i = 1; i < 4; i++) yp[e4 + i] = (T)(0.5 * kS) * acc[i];
       }
     }
-    if (more && ((bits >> (2 * kz + 3)) & 1)) lane_rows_mask<T>(s3, q, a.X, mask(nn));
-    if (more && ((bits >> (2 * kz + 4)) & 1)) lane_rows_mask<T>(s4, q, a.X, mask(nn + 1));
     __syncthreads();
     // the planes 2 ek and 2 ek + 1 are complete: their slots become windows
     lane_window<T>(s0 + q.lw, q.moreX, q.moreY, out[0]);
     lane_window<T>(s1 + q.lw, q.moreX, q.moreY, out[1]);
     __syncthreads();
-    lane_flush<T, kBC, false>(a, q, 2 * ek, s0, (bits >> (2 * kz)) & 1, u, bcn, y, fbx, fby, fbz);
-    lane_flush<T, kBC, false>(a, q, 2 * ek + 1, s1, (bits >> (2 * kz + 1)) & 1, u, bcn, y, fbx, fby, fbz);
+    lane_flush<T, kLaneSums, false>(a, q, 2 * ek, s0, 0u, y, fbx, fby, fbz);
+    lane_flush<T, kLaneSums, false>(a, q, 2 * ek + 1, s1, 0u, y, fbx, fby, fbz);
     __syncthreads();
     slot = slot + 2 >= 5 ? slot - 3 : slot + 2;
   }
   T *const top = sm + kLSlot * slot;
   lane_window<T>(top + q.lw, q.moreX, q.moreY, out[2]);
   __syncthreads();
-  lane_flush<T, kBC, true>(a, q, 2 * (tb.z0 + tb.nzt), top, (bits >> (2 * tb.nzt)) & 1, u, bcn, y, fbx, fby, fbz);
+  lane_flush<T, kLaneSums, true>(a, q, 2 * (tb.z0 + tb.nzt), top, 0u, y, fbx, fby, fbz);
 }

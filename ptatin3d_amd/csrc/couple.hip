@@ -145,18 +145,17 @@ __device__ __forceinline__ void a21_plane(const double X[3][9], const double XZ[
 }
 
 __global__ void __launch_bounds__(64)
-    a21_lane_kernel(TileArgs a, const double *__restrict__ xc, const uint8_t *__restrict__ bcn,
-                    const uint8_t *__restrict__ bcp, const double *__restrict__ u, double *__restrict__ yp) {
+    a21_lane_kernel(TileArgs a, const double *__restrict__ xc, const unsigned *__restrict__ bcw,
+                    const double *__restrict__ u, double *__restrict__ yp) {
   __shared__ double sm[2 * 6 * kLPlane + 6 * kOdd];
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
-  const unsigned long long bits = lane_bc_bits(a, q, bcp);
   double *const s1 = sm + 2 * 6 * kLPlane;
   PlaneRows r1, r2;
   {
     const long n = lane_node(a, tb, 2 * tb.z0);
     r2.load(q, a.X, xc + 3 * n, u + 3 * n);
-    if (bits & 1) r2.mask(q, a.X, bcn + n);
+    r2.mask(lane_bc_word(a, q, bcw, 2 * tb.z0));
     r2.store<kLPlane>(q, sm);
   }
   for (int kz = 0; kz < tb.nzt; kz++) {
@@ -165,6 +164,7 @@ __global__ void __launch_bounds__(64)
     const long n1 = lane_node(a, tb, 2 * ek + 1), n2 = n1 + a.XY;
     const long nc = n1 + a.X * (2 * q.cy + 1) + 2 * q.cx + 1;  // the element's centre
     double ctr[6];
+    const unsigned m1 = lane_bc_word(a, q, bcw, 2 * ek + 1), m2 = lane_bc_word(a, q, bcw, 2 * ek + 2);
     r1.load(q, a.X, xc + 3 * n1, u + 3 * n1);
     r2.load(q, a.X, xc + 3 * n2, u + 3 * n2);
 #pragma unroll
@@ -172,13 +172,13 @@ __global__ void __launch_bounds__(64)
       ctr[f] = xc[3 * nc + f];
       ctr[3 + f] = u[3 * nc + f];
     }
-    if ((bits >> (2 * kz + 1)) & 1) {
-      const unsigned m = bcn[nc];
-      r1.mask(q, a.X, bcn + n1);
+    r1.mask(m1);
+    if (__ballot(m1 != 0u) != 0) {
 #pragma unroll
-      for (int f = 0; f < 3; f++) ctr[3 + f] = ((m >> f) & 1u) ? 0.0 : ctr[3 + f];
+      for (int f = 0; f < 3; f++)  // the lane that holds the centre's entry of its row knows
+        ctr[3 + f] = ((__shfl(m1, 3 * (2 * q.cx + 1) + f) >> (2 * q.cy + 1)) & 1u) ? 0.0 : ctr[3 + f];
     }
-    if ((bits >> (2 * kz + 2)) & 1) r2.mask(q, a.X, bcn + n2);
+    r2.mask(m2);
     r1.store<kOdd>(q, s1);
     r2.store<kLPlane>(q, s2);
     __syncthreads();
@@ -223,8 +223,7 @@ int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
 int launch_a21(const ptmf_op_s *op, const double *u, double *yp) {
   const TileArgs a = lane_args(op->box, 1024, 0.2);
   PTMF_CHECK(a.ntiles < (1L << 31), PTMF_ERR_ARG, "a21: mesh too large (%ld tiles)", a.ntiles);
-  a21_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, op->d64.coords, op->bcnode, op->bcplane, u,
-                                                                         yp);
+  a21_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, op->d64.coords, op->bcword, u, yp);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

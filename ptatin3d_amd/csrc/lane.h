@@ -17,7 +17,7 @@ namespace {
 constexpr int kLT = 8;     // elements per tile side
 constexpr int kLRow = 9;   // row stride of a node class
 constexpr int kLRows = 17; // node rows and columns of a tile
-constexpr int kLMaxZ = 31; // element layers of a chunk (63 node planes: one bit each of a 64-bit mask)
+constexpr int kLMaxZ = 31; // element layers of a chunk, at most
 // The nodes of a tile plane are stored by the parity of their indices, so a
 // lane's node (i, j) lies at a constant offset from the lane's own index and
 // neighbouring lanes read neighbouring words: class (i & 1) + 2 (j & 1).
@@ -157,26 +157,25 @@ __device__ __forceinline__ void lane_rows_store(const T r[kLBatch], const LaneTi
   }
 }
 
-// zeroes the Dirichlet dofs of a stored plane (bcn: from its first node of the tile)
-template <typename T>
-__device__ __forceinline__ void lane_rows_mask(T *p, const LaneTile &q, long X, const LaneBuf<uint8_t> &bcn) {
-  unsigned m[kLRows];
-#pragma unroll
-  for (int j = 0; j < kLRows; j++) m[j] = bcn.load(q.tn, (unsigned)X * (unsigned)min(j, q.last));
-  __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the first is used
-#pragma unroll
-  for (int j = 0; j < kLRows; j++)
-    if ((m[j] >> q.d) & 1u) p[(j & 1 ? q.od : q.ev) + kLRow * (j >> 1)] = T(0);
+// Dirichlet dofs of the tile's node plane P as the lane that holds entry t of
+// its rows sees them: bit j for row j, none for lanes past the rows' entries.
+// One word a plane: a byte per node would be 17 loads, waited for behind every
+// store in flight.
+__device__ __forceinline__ unsigned lane_bc_word(const TileArgs &a, const LaneTile &q, const unsigned *__restrict__ bcw,
+                                                 int P) {
+  return (bcw + 64 * ((2L * a.mz + 1) * (q.tb.tx + (long)a.ntx * q.tb.ty) + P))[q.lane];
 }
 
-// per tile column and node plane: 1 if one of the tile's nodes there has a
-// Dirichlet dof; as bit P - 2 z0 of the chunk's planes (one vector load for the
-// whole chunk, at most 63 planes: a byte load per plane would be waited for
-// together with every store in flight)
-__device__ __forceinline__ unsigned long long lane_bc_bits(const TileArgs &a, const LaneTile &q,
-                                                           const uint8_t *__restrict__ bcp) {
-  const uint8_t *fl = bcp + (2L * a.mz + 1) * (q.tb.tx + (long)a.ntx * q.tb.ty) + 2 * q.tb.z0;
-  return __ballot(fl[min(q.lane, 2 * q.tb.nzt)] != 0);
+// the Dirichlet dofs of a batch of rows to zero (m1, m2: the planes' words)
+template <typename T, int kB, int kN = 2 * kLRows>
+__device__ __forceinline__ void lane_rows_mask(T r[kLBatch], unsigned m1, unsigned m2) {
+  if (__ballot((m1 | m2) != 0u) == 0) return;
+#pragma unroll
+  for (int k = 0; k < kLBatch; k++) {
+    const int h = kB * kLBatch + k, j = h % kLRows;
+    if (h >= kN) continue;
+    r[k] = (((h >= kLRows ? m2 : m1) >> j) & 1u) ? T(0) : r[k];
+  }
 }
 
 // One component at quadrature plane c of an element: V at the plane's 9 points
@@ -280,17 +279,15 @@ __device__ __forceinline__ void lane_window(T *w, bool moreX, bool moreY, const 
 // Dirichlet rows of a flushed plane
 enum LaneBC {
   kLaneSums,  // left as the element sums
-  kLaneCopy,  // y = x
   kLaneZero,  // y = 0
   kLaneOne    // y = 1
 };
 
 // Writes a completed node plane P: the tile's own nodes to y (or, on the
 // tile's top plane, kTop, to the z face), the upper x face column and y face
-// row.  dirichlet: the plane holds Dirichlet dofs.
+// row.  m: the plane's lane_bc_word.
 template <typename T, LaneBC kBC, bool kTop>
-__device__ __forceinline__ void lane_flush(const TileArgs &a, const LaneTile &q, int P, const T *win, bool dirichlet,
-                                           const T *__restrict__ x, const uint8_t *__restrict__ bcn,
+__device__ __forceinline__ void lane_flush(const TileArgs &a, const LaneTile &q, int P, const T *win, unsigned m,
                                            T *__restrict__ y, T *__restrict__ fbx, T *__restrict__ fby,
                                            T *__restrict__ fbz) {
   constexpr unsigned S = sizeof(T);
@@ -308,20 +305,9 @@ __device__ __forceinline__ void lane_flush(const TileArgs &a, const LaneTile &q,
     T v[kLRows];
 #pragma unroll
     for (int j = 0; j < kLRows; j++) v[j] = (j & 1) ? odd[kLRow * (j >> 1)] : even[kLRow * (j >> 1)];
-    if (kBC != kLaneSums && dirichlet && !zface) {
-      const LaneBuf<uint8_t> b(bcn + n0);
-      const LaneBuf<T> xb(kBC == kLaneCopy ? x + 3 * n0 : nullptr);
-      unsigned m[kLRows];
-      T xv[kLRows];
+    if (kBC != kLaneSums && !zface && __ballot(m != 0u) != 0) {
 #pragma unroll
-      for (int j = 0; j < kLRows; j++) {
-        const unsigned row = X * (unsigned)min(j, nyo - 1);
-        m[j] = b.load((unsigned)il, row);
-        xv[j] = kBC == kLaneCopy ? xb.load(S * (unsigned)lane, 3 * S * row) : T(kBC == kLaneOne ? 1 : 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the first is used
-#pragma unroll
-      for (int j = 0; j < kLRows; j++) v[j] = ((m[j] >> q.d) & 1u) ? xv[j] : v[j];
+      for (int j = 0; j < kLRows; j++) v[j] = ((m >> j) & 1u) ? T(kBC == kLaneOne ? 1 : 0) : v[j];
     }
     auto rows = [&](const LaneBuf<T> &w, unsigned rs) {
       const unsigned o = S * (unsigned)lane;

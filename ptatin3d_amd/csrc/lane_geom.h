@@ -71,14 +71,10 @@ struct PlaneRows {
       p[(j & 1 ? od : ev) + kLRow * (j >> 1) + 3 * S] = u[j];
     }
   }
-  __device__ __forceinline__ void mask(const LaneTile &q, long X, const uint8_t *bcn) {
-    const LaneBuf<uint8_t> b(bcn);
-    unsigned m[kLRows];
+  __device__ __forceinline__ void mask(unsigned m) {  // the plane's lane_bc_word
+    if (__ballot(m != 0u) == 0) return;
 #pragma unroll
-    for (int j = 0; j < kLRows; j++) m[j] = b.load(q.tn, (unsigned)X * (unsigned)min(j, q.last));
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < kLRows; j++) u[j] = ((m[j] >> q.d) & 1u) ? 0.0 : u[j];
+    for (int j = 0; j < kLRows; j++) u[j] = ((m >> j) & 1u) ? 0.0 : u[j];
   }
 };
 
@@ -94,13 +90,12 @@ struct PlaneRows {
 // loaded behind the forward stages.
 template <typename Op>
 __global__ void __launch_bounds__(64)
-    node_lane_kernel(TileArgs a, Op op, const double *__restrict__ xc, const uint8_t *__restrict__ bcn,
-                     const uint8_t *__restrict__ bcp, double *__restrict__ y, double *__restrict__ fbx,
+    node_lane_kernel(TileArgs a, Op op, const double *__restrict__ xc, const unsigned *__restrict__ bcw,
+                     double *__restrict__ y, double *__restrict__ fbx,
                      double *__restrict__ fby, double *__restrict__ fbz) {
   __shared__ double sm[5 * kLSlot];
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
-  const unsigned long long bits = lane_bc_bits(a, q, bcp);
   auto plane = [&](int P) { return LaneBuf<double>(xc + 3 * lane_node(a, tb, P)); };
   {
     const LaneBuf<double> v0 = plane(2 * tb.z0), v1 = plane(2 * tb.z0 + 1), v2 = plane(2 * tb.z0 + 2);
@@ -122,6 +117,7 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
     for (int n = 0; n < 9; n++) out[2][l][n] = 0.0;
 
+  unsigned m0 = 0, m1 = 0, m2 = 0;
   int slot = 0;  // of plane 2 ek; its successors follow modulo 5
   for (int kz = 0; kz < tb.nzt; kz++) {
     const int ek = tb.z0 + kz;
@@ -159,9 +155,13 @@ __global__ void __launch_bounds__(64)
     lane_pin<double>(out);
     asm volatile("" : "+v"(lq));
     op.template load<2>();
+    m0 = lane_bc_word(a, q, bcw, 2 * ek);
+    m1 = lane_bc_word(a, q, bcw, 2 * ek + 1);
+    m2 = lane_bc_word(a, q, bcw, 2 * ek + 2);
     lane_rows_load<double, 2>(r, q, a.X, v1, v2);
     plane_fields<2>(s0 + lq, s1 + lq, s2 + lq, X, Z);
     lane_rows_store<double, 2>(r, q, s3, s4);
+    asm volatile("" : "+v"(m0), "+v"(m1), "+v"(m2));
     op.template plane<2>(X, Z, out);
     lane_pin<double>(out);
     op.finish(out[0]);
@@ -170,8 +170,8 @@ __global__ void __launch_bounds__(64)
     lane_window<double>(s0 + q.lw, q.moreX, q.moreY, out[0]);
     lane_window<double>(s1 + q.lw, q.moreX, q.moreY, out[1]);
     __syncthreads();
-    lane_flush<double, Op::kBC, false>(a, q, 2 * ek, s0, (bits >> (2 * kz)) & 1, nullptr, bcn, y, fbx, fby, fbz);
-    lane_flush<double, Op::kBC, false>(a, q, 2 * ek + 1, s1, (bits >> (2 * kz + 1)) & 1, nullptr, bcn, y, fbx, fby,
+    lane_flush<double, Op::kBC, false>(a, q, 2 * ek, s0, m0, y, fbx, fby, fbz);
+    lane_flush<double, Op::kBC, false>(a, q, 2 * ek + 1, s1, m1, y, fbx, fby,
                                          fbz);
     __syncthreads();
     slot = slot + 2 >= 5 ? slot - 3 : slot + 2;
@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(64)
   op.finish(out[2]);
   lane_window<double>(top + q.lw, q.moreX, q.moreY, out[2]);
   __syncthreads();
-  lane_flush<double, Op::kBC, true>(a, q, 2 * (tb.z0 + tb.nzt), top, (bits >> (2 * tb.nzt)) & 1, nullptr, bcn, y, fbx,
+  lane_flush<double, Op::kBC, true>(a, q, 2 * (tb.z0 + tb.nzt), top, m2, y, fbx,
                                       fby, fbz);
 }
 
@@ -198,8 +198,8 @@ int launch_node_lane(const ptmf_op_s *op, const TileArgs &a, const Op &nodal, do
   PTMF_CHECK(face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= op->faces_doubles && a.ntiles < (1L << 31),
              PTMF_ERR_ARG, "mesh too large (%ld tiles)", a.ntiles);
   double *fbx = (double *)op->faces, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
-  node_lane_kernel<Op><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, nodal, op->d64.coords, op->bcnode,
-                                                                              op->bcplane, y, fbx, fby, fbz);
+  node_lane_kernel<Op><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, nodal, op->d64.coords, op->bcword, y,
+                                                                              fbx, fby, fbz);
   PTMF_HIP(hipGetLastError());
   node_face_kernel<<<dim3((unsigned)a.ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y, op->bcnode);
   PTMF_HIP(hipGetLastError());

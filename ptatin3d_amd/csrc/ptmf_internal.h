@@ -98,7 +98,7 @@ struct ptmf_op_s {
   uint8_t *bcnode = nullptr;      // per-node Dirichlet bits (bit d: dof d)
   long *bcidx = nullptr;          // compact list of Dirichlet dofs
   long nbc = 0;
-  uint8_t *bcplane = nullptr;     // per 8 x 8 tile column and node plane: any Dirichlet dof
+  unsigned *bcword = nullptr;     // Dirichlet dofs per 8 x 8 tile column, node plane and lane (lane.h)
   int has_coords = 0, has_eta = 0, has_bc = 0;
   unsigned long state = 0;        // bumped by every coefficient change
   int device = 0;                 // device the operator was created on
@@ -109,7 +109,7 @@ struct ptmf_op_s {
   // rectilinear mesh (element faces normal to the axes): 2 / h per element of
   // the mx columns, my rows and mz layers
   int rect = 0;
-  double *ax64 = nullptr;         // holds ax32, rect_bad and bcplane too
+  double *ax64 = nullptr;         // holds ax32, rect_bad and bcword too
   float *ax32 = nullptr;
   int *rect_bad = nullptr;
   int variant = 0;  // MatMult kernel: 0 z-march, 1 software-pipelined, 2 stored geometry, 3 coloured
@@ -181,7 +181,7 @@ int classify_mesh(ptmf_op_s *op);
 // so that new coordinates never move the buffers
 long lane_face_doubles(const Box &b, const Tiling &t);
 long couple_face_doubles(const Box &b);  // of launch_a12
-// set-up: op->bcplane from the operator's Dirichlet bits
+// set-up: op->bcword from the operator's Dirichlet bits
 int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>
 int launch_fill(T *x, T v, long n, hipStream_t s);
