@@ -1076,19 +1076,45 @@ __global__ void __launch_bounds__(kFaceThreads)
   }
 }
 
+#include "a11_col.h"
+
 // ---------------------------------------------------------------------------
-// Batched MatMult: many independent boxes in one launch per stage.  A work
-// item is (box, tile); every box has its own tiling, coefficients, Dirichlet
-// data and face buffers (BoxDesc, in device memory).
+// Batched MatMult: many independent boxes in one launch per stage.  Every box
+// takes the column kernel or, too large for it or tiled by the caller, the tile
+// kernel.  A work item is (box, tile), or (box, wave) and then (box, 256 nodes);
+// every box has its own sizes, coefficients, Dirichlet data and buffers
+// (BoxDesc, in device memory).
 // ---------------------------------------------------------------------------
 struct BoxDesc {
   TileArgs a;
-  const void *xc, *eta;  // coordinates and tile-ordered viscosity of the precision
+  ColArgs c;
+  const void *xc, *eta;  // coordinates; viscosity, tile-ordered for the tile kernel
   const uint8_t *bcn;
   const long *bcidx;
-  long nbc;
-  void *fbx, *fby, *fbz;
+  long nbc;              // 0 for the column kernel, whose sums copy the Dirichlet rows
+  void *fbx, *fby, *fbz; // fbx: the element sums of the column kernel
 };
+
+template <typename T>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+    a11_col_batch_kernel(const BoxDesc *__restrict__ boxes, const int2 *__restrict__ work, long nwork,
+                         const T *const *__restrict__ xs, const int *__restrict__ active) {
+  __shared__ T sm[18][64];
+  const int2 w = work[xcd_tile(blockIdx.x, nwork)];
+  if (active && !active[w.x]) return;  // whole work-group: the box is idle
+  const BoxDesc &d = boxes[w.x];
+  col_wave<T>(d.c, (unsigned)w.y, (const T *)d.xc, (const T *)d.eta, d.bcn, xs[w.x], (T *)d.fbx, sm);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kColSumThreads)
+    col_sum_batch_kernel(const BoxDesc *__restrict__ boxes, const int2 *__restrict__ work, long nwork,
+                         const T *const *__restrict__ xs, T *const *__restrict__ ys, const int *__restrict__ active) {
+  const int2 w = work[xcd_tile(blockIdx.x, nwork)];
+  if (active && !active[w.x]) return;
+  const BoxDesc &d = boxes[w.x];
+  col_node<T>(d.c, (unsigned)(w.y * kColSumThreads) + threadIdx.x, (const T *)d.fbx, ys[w.x], d.bcn, xs[w.x]);
+}
 
 template <typename T>
 __global__ void __launch_bounds__(64)
@@ -1160,14 +1186,33 @@ TileArgs tile_args(const ptmf_op_s *op) {
 // 13.5 us against 15.6 us; 20^3: 15.6 and 16.0 us), and the lane kernel has the
 // rest (28^3: 17.8 us against 33.6 us, FP32 13.7 and 17.2 us; 48 x 48 x 32: 32
 // and 71 us, FP32 18 and 31 us; 64^3: 63 and 178 us, FP32 35 and 82 us).
+//
+// The column kernel (a11_col.h) has the boxes of up to 100,000 elements, whose
+// element sums fit 64 MiB, on meshes that are not rectilinear (MatMult against
+// the tile kernel's: 8^3 9.2 and 18.4 us, 24^3 20 and 24 us, 45 x 37 x 29 44 and
+// 62 us, 48 x 48 x 32 62 and 82 us, FP32 41 and 43 us; 64 x 64 x 32 in FP32 70
+// and 68 us), and the small rectilinear ones: its MatMult takes 8.5 + E / 1333 us
+// (FP32 7.5 + E / 2222), the lane kernel's that of its kernel above, rounded up
+// for a chip not full, and 1 us (5.5 us): 24^3 20 against 21 us, 32^3 32 against
+// 27 us; FP32 14 against 18 us, 24 against 22 us.
+constexpr long kColDoubles = 8L << 20;
+
+template <typename T>
+double col_cost(long nel) {
+  return sizeof(T) == 8 ? 8.5 + 0.75e-3 * (double)nel : 7.5 + 0.45e-3 * (double)nel;
+}
+
 template <typename T>
 double lane_rounds(long waves, double one, double two) {
   const long r = (waves + 1023) / 1024;
   return sizeof(T) == 8 ? one * (double)r : two * (double)(r / 2) + one * (double)(r % 2);
 }
 
+// kernel: the one the lane kernel would take the place of
+enum LaneOther { kOtherTile, kOtherCol };
+
 template <typename T>
-bool lane_plan(const Box &b, const Tiling &t, TileArgs &a) {
+bool lane_plan(const Box &b, const Tiling &t, LaneOther other, TileArgs &a) {
   constexpr bool f64 = sizeof(T) == 8;
   if (!f64 && std::max(b.mx, std::max(b.my, b.mz)) > 64) return false;
   a.mx = b.mx; a.my = b.my; a.mz = b.mz;
@@ -1186,7 +1231,8 @@ bool lane_plan(const Box &b, const Tiling &t, TileArgs &a) {
       a.ntiles = nt;
     }
   }
-  if (best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 15.7)) return false;
+  if (other == kOtherTile && best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 15.7)) return false;
+  if (other == kOtherCol && best + (f64 ? 1.0 : 5.5) >= col_cost<T>(b.nel)) return false;
   a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
   a.fbz_n = kLRows * kLRows;
   // byte offsets of the 27 quadrature points' viscosities and of 17 node rows
@@ -1195,9 +1241,21 @@ bool lane_plan(const Box &b, const Tiling &t, TileArgs &a) {
 
 // the same for an operator with face buffers of fb_doubles
 template <typename T>
-bool lane_tiles(const ptmf_op_s *op, long fb_doubles, TileArgs &a) {
-  return op->rect && op->tiling_default && op->wg_tiles == 1 && lane_plan<T>(op->box, op->tiling, a) &&
+bool lane_tiles(const ptmf_op_s *op, long fb_doubles, LaneOther other, TileArgs &a) {
+  return op->rect && op->tiling_default && op->wg_tiles == 1 && lane_plan<T>(op->box, op->tiling, other, a) &&
          face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= fb_doubles;
+}
+
+long col_doubles(const Box &b) { return 81 * b.nel <= kColDoubles ? 81 * b.nel : 0; }
+
+ColArgs col_args(const Box &b) {
+  const unsigned ne = (unsigned)b.nel;
+  return ColArgs{(unsigned)b.mx, (unsigned)b.my, (unsigned)b.mz, ne, (ne + kColElems - 1) / kColElems};
+}
+
+// the column kernel, with a buffer of fb_doubles, where the lane kernel is not chosen
+bool col_box(const ptmf_op_s *op, long fb_doubles) {
+  return op->tiling_default && op->wg_tiles == 1 && col_doubles(op->box) > 0 && col_doubles(op->box) <= fb_doubles;
 }
 
 // Is the mesh rectilinear?  Axis lines of the three directions first (mid
@@ -1309,9 +1367,9 @@ int classify_mesh(ptmf_op_s *op) {
 long lane_face_doubles(const Box &b, const Tiling &t) {
   TileArgs a;
   long n = 0;
-  if (lane_plan<double>(b, t, a)) n = face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles);
-  if (lane_plan<float>(b, t, a)) n = std::max(n, face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles));
-  return n;
+  if (lane_plan<double>(b, t, kOtherTile, a)) n = face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles);
+  if (lane_plan<float>(b, t, kOtherTile, a)) n = std::max(n, face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles));
+  return std::max(n, col_doubles(b));
 }
 
 long face_buffer_doubles(int TX, int TY, int ZC, long ntiles) {
@@ -1470,6 +1528,21 @@ int launch_lane(const ptmf_op_s *op, const TileArgs &a, int faces, const T *x, c
   return PTMF_OK;
 }
 
+template <typename T>
+int launch_col(const ptmf_op_s *op, int faces, const T *x, T *y, T *es) {
+  const Box &b = op->box;
+  const OpData<T> &d = *(const OpData<T> *)(sizeof(T) == 8 ? (const void *)&op->d64 : (const void *)&op->d32);
+  const ColArgs a = col_args(b);
+  a11_col_kernel<T><<<dim3(a.nwaves), dim3(64), 0, op->stream>>>(a, d.coords, d.eta, op->bcnode, x, es);
+  PTMF_HIP(hipGetLastError());
+  if (!faces) return PTMF_OK;
+  const long groups = (b.nnodes + kColSumThreads - 1) / kColSumThreads;
+  col_sum_kernel<T><<<dim3((unsigned)groups), dim3(kColSumThreads), 0, op->stream>>>(a, es, y, op->bcnode,
+                                                                                     faces == 1 ? x : nullptr);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
 // The MatMult's kernels with the face buffers at fb (the operator's own, or
 // the static scratch of the allocation-free entry point).  noalloc: nothing
 // is allocated on the way (the stored-geometry and coloured variants, which
@@ -1498,8 +1571,10 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
     return PTMF_OK;
   }
   TileArgs la;
-  if (variant == 0 && lane_tiles<T>(op, fb_doubles, la))
+  const LaneOther other = col_box(op, fb_doubles) ? kOtherCol : kOtherTile;
+  if (variant == 0 && lane_tiles<T>(op, fb_doubles, other, la))
     return launch_lane<T, false>(op, la, faces, x, nullptr, y, nullptr, fb);
+  if (variant == 0 && col_box(op, fb_doubles)) return launch_col<T>(op, faces, x, y, fb);
   const TileArgs a = tile_args(op);
   const long ntiles = tl.ntiles;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * ntiles, *fbz = fby + 3 * a.fby_n * ntiles;
@@ -1552,7 +1627,7 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   // (by lane_plan's rule for the MatMult: at 24^3 both take 42 us, at 28^3 the
   // lane kernel 41 us and the tile kernel 62 us, and further apart above)
   TileArgs la;
-  if (lane_tiles<T>(op, op->faces_doubles, la))
+  if (lane_tiles<T>(op, op->faces_doubles, kOtherTile, la))
     return launch_lane<T, true>(op, la, 1, x, x + nu, y, y + nu, (T *)op->faces);
   PTMF_TRY(ensure_eta_tiled<T>(op));
   const T *et = sizeof(T) == 8 ? (const T *)op->et64 : (const T *)op->et32;
@@ -1590,9 +1665,11 @@ struct ptmf_batch_s {
   // device data, rebuilt when the operators' tilings or buffers change
   ptmf::BoxDesc *dbox[2] = {nullptr, nullptr};
   std::vector<unsigned char> hbox[2];
+  // (box, tile) of the tile kernel, then (box, wave) and (box, node block) of
+  // the column kernel
   int2 *dwork = nullptr;
-  long nwork = 0;
-  std::vector<int> key;  // TX, TY, ZC, ntiles per operator of the current work list
+  long nwork = 0, ncol = 0, nsum = 0;
+  std::vector<int> key;  // TX, TY, ZC, ntiles, column kernel per operator of the current work list
   void **dxy[2] = {nullptr, nullptr};  // device arrays of x and y pointers, per precision
   std::vector<const void *> hxy[2];
   long maxnbc = 0;
@@ -1605,22 +1682,30 @@ template <typename T>
 int batch_prepare_boxes(ptmf_batch_s *b) {
   const int ip = sizeof(T) == 8 ? 0 : 1;
   const int n = (int)b->ops.size();
-  // work list of (box, tile)
+  // work lists
+  auto col = [](const ptmf_op_s *op) { return op->variant == 0 && ptmf::col_box(op, op->faces_doubles); };
   std::vector<int> key;
   for (ptmf_op op : b->ops) {
     const ptmf::Tiling &t = op->tiling;
-    key.insert(key.end(), {t.TX, t.TY, t.ZC, (int)t.ntiles});
+    key.insert(key.end(), {t.TX, t.TY, t.ZC, (int)t.ntiles, col(op) ? 1 : 0});
   }
   if (key != b->key) {
     std::vector<int2> work;
-    for (int i = 0; i < n; i++)
-      for (long t = 0; t < b->ops[i]->tiling.ntiles; t++) work.push_back(make_int2(i, (int)t));
-    PTMF_CHECK(!work.empty() && work.size() < (1UL << 31), PTMF_ERR_ARG, "batch: %zu tiles", work.size());
+    auto add = [&](bool column, auto &&count) {
+      const size_t first = work.size();
+      for (int i = 0; i < n; i++)
+        if (col(b->ops[i]) == column)
+          for (long t = 0, m = count(b->ops[i]); t < m; t++) work.push_back(make_int2(i, (int)t));
+      return (long)(work.size() - first);
+    };
+    b->nwork = add(false, [](ptmf_op op) { return op->tiling.ntiles; });
+    b->ncol = add(true, [](ptmf_op op) { return (op->box.nel + ptmf::kColElems - 1) / ptmf::kColElems; });
+    b->nsum = add(true, [](ptmf_op op) { return (op->box.nnodes + ptmf::kColSumThreads - 1) / ptmf::kColSumThreads; });
+    PTMF_CHECK(!work.empty() && work.size() < (1UL << 31), PTMF_ERR_ARG, "batch: %zu work items", work.size());
     (void)hipFree(b->dwork);
     b->dwork = nullptr;
     PTMF_HIP(hipMalloc((void **)&b->dwork, sizeof(int2) * work.size()));
     PTMF_HIP(hipMemcpy(b->dwork, work.data(), sizeof(int2) * work.size(), hipMemcpyHostToDevice));
-    b->nwork = (long)work.size();
     b->key = key;
   }
   // per-box descriptors of this precision
@@ -1630,8 +1715,9 @@ int batch_prepare_boxes(ptmf_batch_s *b) {
     ptmf_op op = b->ops[i];
     PTMF_CHECK(op->has_coords && op->has_eta && op->has_bc, PTMF_ERR_NOT_SETUP,
                "batch: operator %d: MF operator not setup", i);
-    PTMF_TRY(ptmf::ensure_eta_tiled<T>(op));
     ptmf::BoxDesc &d = box[i];
+    memset((void *)&d, 0, sizeof(d));  // (compared bytewise)
+    if (!col(op)) PTMF_TRY(ptmf::ensure_eta_tiled<T>(op));
     d.a = ptmf::tile_args(op);
     const ptmf::OpData<T> &od = *(const ptmf::OpData<T> *)(ip == 0 ? (const void *)&op->d64 : (const void *)&op->d32);
     d.xc = od.coords;
@@ -1643,7 +1729,12 @@ int batch_prepare_boxes(ptmf_batch_s *b) {
     d.fbx = fb;
     d.fby = fb + 3 * d.a.fbx_n * d.a.ntiles;
     d.fbz = (T *)d.fby + 3 * d.a.fby_n * d.a.ntiles;
-    if (op->nbc > b->maxnbc) b->maxnbc = op->nbc;
+    if (col(op)) {
+      d.c = ptmf::col_args(op->box);
+      d.eta = od.eta;
+      d.nbc = 0;
+    }
+    if (d.nbc > b->maxnbc) b->maxnbc = d.nbc;
   }
   // the tile-ordered viscosity is built on each operator's own stream
   for (ptmf_op op : b->ops) PTMF_HIP(hipStreamSynchronize(op->stream));
@@ -1678,12 +1769,21 @@ int batch_prepare(ptmf_batch_s *b, const void *const *x, void *const *y) {
   return PTMF_OK;
 }
 
-// the three batched stages on device tables of x and y pointers
+// the batched stages on device tables of x and y pointers
 template <typename T>
 int batch_launch_tables(ptmf_batch_s *b, const T *const *xs, T *const *ys, hipStream_t s,
                         const int *active = nullptr) {
   const int ip = sizeof(T) == 8 ? 0 : 1;
   const int n = (int)b->ops.size();
+  if (b->ncol > 0) {
+    const int2 *work = b->dwork + b->nwork;
+    ptmf::a11_col_batch_kernel<T><<<dim3((unsigned)b->ncol), dim3(64), 0, s>>>(b->dbox[ip], work, b->ncol, xs, active);
+    PTMF_HIP(hipGetLastError());
+    ptmf::col_sum_batch_kernel<T><<<dim3((unsigned)b->nsum), dim3(ptmf::kColSumThreads), 0, s>>>(
+        b->dbox[ip], work + b->ncol, b->nsum, xs, ys, active);
+    PTMF_HIP(hipGetLastError());
+  }
+  if (b->nwork == 0) return PTMF_OK;
   ptmf::a11_tile_batch_kernel<T><<<dim3((unsigned)b->nwork), dim3(64), 0, s>>>(b->dbox[ip], b->dwork, b->nwork, xs,
                                                                               ys, active);
   PTMF_HIP(hipGetLastError());
