@@ -1047,16 +1047,9 @@ __global__ void __launch_bounds__(64)
 // wave would walk one dependent load/store round after another.
 constexpr int kFaceThreads = 256;
 
-template <typename T>
-__global__ void __launch_bounds__(kFaceThreads)
-    a11_face_kernel(TileArgs a, const T *__restrict__ fbx, const T *__restrict__ fby,
-                    const T *__restrict__ fbz, T *__restrict__ y) {
-  face_sum<T>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y);
-}
-
-// The same with the Dirichlet rows y = x, which the face sums leave alone: the
-// work-groups past the tiles copy them, beside the others' face sums and not
-// after them (64^3: 15 us for the faces alone and for both, a launch of its own
+// It adds the face sums and, in the work-groups past the tiles, copies the
+// Dirichlet rows y = x, which the face sums leave alone: beside
+// the others' face sums and not after them (64^3: 15 us for the faces alone and for both, a launch of its own
 // took 5 us more; copied by the lane kernel as it writes the other rows 16 us).
 constexpr int kCopyGroup = 8 * kFaceThreads;  // rows per work-group
 template <typename T>
@@ -1074,6 +1067,92 @@ __global__ void __launch_bounds__(kFaceThreads)
     const long i = i0 + kFaceThreads * k + threadIdx.x;
     if (i < nbc) y[bcidx[i]] = x[bcidx[i]];
   }
+}
+
+// RowUpdates by what they read besides b: nothing (a residual), dinv, or dinv
+// and prev
+enum UpdateKind { kUpResidual, kUpFirst, kUpStep };
+
+// One row: all it reads is requested before any of it is used (out may be prev
+// or the element sums, the same row of them).
+template <typename T, UpdateKind kUp>
+struct UpdateRow {
+  T b, x, dinv, prev;
+  unsigned m;
+  __device__ __forceinline__ void load(const RowUpdate<T> &up, long i, const T *__restrict__ x_, unsigned bits) {
+    m = bits;
+    b = up.b[i];
+    x = x_[i];
+    if (kUp != kUpResidual) dinv = up.dinv[i];
+    if (kUp == kUpStep) prev = up.prev[i];
+  }
+  __device__ __forceinline__ void store(const RowUpdate<T> &up, long i, unsigned d, T sum) const {
+    T o = b - (((m >> d) & 1u) ? x : sum);
+    if (kUp != kUpResidual) o = up.os * (o * dinv);
+    if (kUp == kUpStep) o += up.om1 * prev;
+    if (kUp != kUpResidual) o += up.om * x;
+    if (up.out64) ((double *)up.out)[i] = (double)o;
+    else ((T *)up.out)[i] = o;
+  }
+};
+
+// A RowUpdate with the face sums added on the way: one pass over the vectors in
+// place of the face pass and the update (FP64 32^3: 8.0 us, apart 14.2 us; 48 x
+// 48 x 32 FP32 10.0 and 16 us; 64^3 47 us, apart 44 us but one launch more).
+// Bound by memory: up to five vectors in and one out.  A thread takes one row of
+// the two node planes 2 ek and 2 ek + 1 of an element layer (of the top layer:
+// three): its place in the tiles is worked out once, and all loads of both are
+// in flight together (all planes of a tile layer two at a time: 56 us).  Each
+// XCD has a slab of its own, as in the element kernel (52 us without).  r: the
+// element kernel's sums.
+template <typename T, UpdateKind kUp>
+__global__ void __launch_bounds__(256)
+    a11_update_kernel(TileArgs a, unsigned gx, const T *__restrict__ fbx, const T *__restrict__ fby,
+                      const T *__restrict__ fbz, const T *r, const uint8_t *__restrict__ bcn, const T *__restrict__ x,
+                      RowUpdate<T> up) {
+  const unsigned blk = (unsigned)xcd_tile(blockIdx.x, gridDim.x), ek = blk / gx;
+  const unsigned t = (blk - ek * gx) * 256u + threadIdx.x, X = (unsigned)a.X;
+  if (t >= 3u * (unsigned)a.XY) return;
+  const unsigned m = t / 3u, d = t - 3u * m, J = m / X, I = m - J * X;
+  const int tx = min((int)(I / (2u * a.TX)), a.ntx - 1), ty = min((int)(J / (2u * a.TY)), a.nty - 1);
+  const int il = (int)I - 2 * a.TX * tx, jl = (int)J - 2 * a.TY * ty;
+  const bool hx = tx > 0 && il == 0, hy = ty > 0 && jl == 0;
+  const int tz = (int)ek / a.ZC, k0 = 2 * ((int)ek - a.ZC * tz);
+  const int sx = 3 * (2 * a.TY + 1), sy = 3 * (2 * a.TX + 1);
+  const long tile = tx + (long)a.ntx * (ty + (long)a.nty * tz), below = (long)a.ntx * a.nty;
+  // the neighbours' upper faces at this row, in the order of face_sum
+  const T *const p0 = fbx + 3 * ((tile - 1 - a.ntx) * a.fbx_n + 2 * a.TY) + d,
+                 *const p1 = fby + 3 * ((tile - a.ntx) * a.fby_n + il) + d,
+                 *const p2 = fbx + 3 * ((tile - 1) * a.fbx_n + jl) + d;
+  auto faces = [&](long kx, long ky) {
+    const T v0 = hx && hy ? p0[kx] : T(0), v1 = hy ? p1[ky] : T(0), v2 = hx ? p2[kx] : T(0);
+    return v0 + v1 + v2;
+  };
+  const long n0 = m + a.XY * (2L * ek);
+  auto planes = [&](auto first, auto count) {
+    constexpr int kF = decltype(first)::value, kN = decltype(count)::value;
+    UpdateRow<T, kUp> u[kN];
+    T s[kN], f[kN];
+#pragma unroll
+    for (int p = 0; p < kN; p++) {
+      const long n = n0 + a.XY * (kF + p);
+      s[p] = r[3 * n + d];
+      u[p].load(up, 3 * n + d, x, bcn[n]);
+      f[p] = T(0);
+    }
+    if (kF == 0 && k0 == 0 && tz > 0)  // the tiles below
+      f[0] = faces(2L * a.ZC * sx - 3 * below * a.fbx_n, 2L * a.ZC * sy - 3 * below * a.fby_n) +
+             fbz[3 * ((tile - below) * a.fbz_n + il + (long)(2 * a.TX + 1) * jl) + d];
+    if (hx || hy) {
+#pragma unroll
+      for (int p = 0; p < kN; p++) f[p] += faces((long)sx * (k0 + kF + p), (long)sy * (k0 + kF + p));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < kN; p++) u[p].store(up, 3 * (n0 + a.XY * (kF + p)) + d, d, s[p] + f[p]);
+  };
+  planes(std::integral_constant<int, 0>(), std::integral_constant<int, 2>());
+  if ((int)ek == a.mz - 1) planes(std::integral_constant<int, 2>(), std::integral_constant<int, 1>());
 }
 
 #include "a11_col.h"
@@ -1511,34 +1590,62 @@ int launch_face_copy(const ptmf_op_s *op, const TileArgs &a, const T *fbx, const
   return PTMF_OK;
 }
 
-// the lane kernel (lane_tiles must hold) and its faces
+template <typename T, typename F>
+void with_kind(const RowUpdate<T> &up, F &&f) {
+  if (!up.dinv) f(std::integral_constant<UpdateKind, kUpResidual>());
+  else if (!up.prev) f(std::integral_constant<UpdateKind, kUpFirst>());
+  else f(std::integral_constant<UpdateKind, kUpStep>());
+}
+
+// what follows the element kernel: nothing (its timing alone), the MatMult's face
+// sums and Dirichlet rows, or a RowUpdate
+enum Finish { kFinNone, kFinMult, kFinUpdate };
+
+template <typename T>
+int finish_rows(const ptmf_op_s *op, const TileArgs &a, Finish fin, const RowUpdate<T> *up, const T *fbx, const T *fby,
+                const T *fbz, const T *x, T *y) {
+  if (fin == kFinNone) return PTMF_OK;
+  if (fin == kFinMult) return launch_face_copy<T>(op, a, fbx, fby, fbz, x, y);
+  PTMF_CHECK(3 * a.XY < (1L << 32) - 256, PTMF_ERR_ARG, "a11: mesh too large (%ld nodes in a plane)", a.XY);
+  const long gx = (3 * a.XY + 255) / 256;
+  PTMF_CHECK(gx * a.mz < (1L << 31), PTMF_ERR_ARG, "a11: mesh too large (%ld work-groups)", gx * a.mz);
+  with_kind(*up, [&](auto k) {
+    a11_update_kernel<T, decltype(k)::value><<<dim3((unsigned)(gx * a.mz)), dim3(256), 0, op->stream>>>(
+        a, (unsigned)gx, fbx, fby, fbz, y, op->bcnode, x, *up);
+  });
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
+// the lane kernel (lane_tiles must hold) and what follows
 template <typename T, bool kP>
-int launch_lane(const ptmf_op_s *op, const TileArgs &a, int faces, const T *x, const T *p, T *y, T *yp, T *fb) {
+int launch_lane(const ptmf_op_s *op, const TileArgs &a, Finish fin, const RowUpdate<T> *up, const T *x, const T *p, T *y,
+                T *yp, T *fb) {
   const T *ax = sizeof(T) == 8 ? (const T *)op->ax64 : (const T *)op->ax32;
   const T *eta = sizeof(T) == 8 ? (const T *)op->d64.eta : (const T *)op->d32.eta;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
   a11_lane_kernel<T, kP><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, ax, eta, op->bcword, x, p, y, yp, fbx,
                                                                                fby, fbz);
   PTMF_HIP(hipGetLastError());
-  if (faces == 1)
-    PTMF_TRY(launch_face_copy<T>(op, a, fbx, fby, fbz, x, y));
-  else if (faces)
-    a11_face_kernel<T><<<dim3((unsigned)a.ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y);
-  PTMF_HIP(hipGetLastError());
-  return PTMF_OK;
+  return finish_rows<T>(op, a, fin, up, fbx, fby, fbz, x, y);
 }
 
 template <typename T>
-int launch_col(const ptmf_op_s *op, int faces, const T *x, T *y, T *es) {
+int launch_col(const ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T *x, T *y, T *es) {
   const Box &b = op->box;
   const OpData<T> &d = *(const OpData<T> *)(sizeof(T) == 8 ? (const void *)&op->d64 : (const void *)&op->d32);
   const ColArgs a = col_args(b);
   a11_col_kernel<T><<<dim3(a.nwaves), dim3(64), 0, op->stream>>>(a, d.coords, d.eta, op->bcnode, x, es);
   PTMF_HIP(hipGetLastError());
-  if (!faces) return PTMF_OK;
+  if (fin == kFinNone) return PTMF_OK;
   const long groups = (b.nnodes + kColSumThreads - 1) / kColSumThreads;
-  col_sum_kernel<T><<<dim3((unsigned)groups), dim3(kColSumThreads), 0, op->stream>>>(a, es, y, op->bcnode,
-                                                                                     faces == 1 ? x : nullptr);
+  if (fin == kFinMult)
+    col_sum_kernel<T><<<dim3((unsigned)groups), dim3(kColSumThreads), 0, op->stream>>>(a, es, y, op->bcnode, x);
+  else
+    with_kind(*up, [&](auto k) {
+      col_update_kernel<T, decltype(k)::value>
+          <<<dim3((unsigned)groups), dim3(kColSumThreads), 0, op->stream>>>(a, es, op->bcnode, x, *up);
+    });
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }
@@ -1548,7 +1655,8 @@ int launch_col(const ptmf_op_s *op, int faces, const T *x, T *y, T *es) {
 // is allocated on the way (the stored-geometry and coloured variants, which
 // build tables of their own or need no face buffers, give way to the z-march).
 template <typename T>
-int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long fb_doubles, bool noalloc = false) {
+int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T *x, T *y, T *fb, long fb_doubles,
+                       bool noalloc = false) {
   const OpData<T> &d = *(const OpData<T> *)(sizeof(T) == 8 ? (const void *)&op->d64
                                                            : (const void *)&op->d32);
   const Tiling &tl = op->tiling;
@@ -1567,14 +1675,17 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
           b.mx, b.my, b.mz, b.nel, b.X, b.X * b.Y, color, d.coords, d.eta, op->bcnode, x, y);
     }
     PTMF_HIP(hipGetLastError());
-    if (faces == 1) PTMF_TRY(launch_bc_copy<T>(op->bcidx, op->nbc, x, y, op->stream));
-    return PTMF_OK;
+    TileArgs one = tile_args(op);  // (a single tile: no faces)
+    one.TX = b.mx; one.TY = b.my; one.ZC = b.mz;
+    one.ntx = one.nty = 1;
+    one.ntiles = 0;
+    return finish_rows<T>(op, one, fin, up, nullptr, nullptr, nullptr, x, y);
   }
   TileArgs la;
   const LaneOther other = col_box(op, fb_doubles) ? kOtherCol : kOtherTile;
   if (variant == 0 && lane_tiles<T>(op, fb_doubles, other, la))
-    return launch_lane<T, false>(op, la, faces, x, nullptr, y, nullptr, fb);
-  if (variant == 0 && col_box(op, fb_doubles)) return launch_col<T>(op, faces, x, y, fb);
+    return launch_lane<T, false>(op, la, fin, up, x, nullptr, y, nullptr, fb);
+  if (variant == 0 && col_box(op, fb_doubles)) return launch_col<T>(op, fin, up, x, y, fb);
   const TileArgs a = tile_args(op);
   const long ntiles = tl.ntiles;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * ntiles, *fbz = fby + 3 * a.fby_n * ntiles;
@@ -1602,17 +1713,17 @@ int launch_a11_mult_fb(ptmf_op_s *op, const T *x, T *y, int faces, T *fb, long f
           a, d.coords, et, op->bcnode, x, y, fbx, fby, fbz);
   }
   PTMF_HIP(hipGetLastError());
-  if (faces == 1) return launch_face_copy<T>(op, a, fbx, fby, fbz, x, y);
-  if (faces) {
-    a11_face_kernel<T><<<dim3((unsigned)ntiles), dim3(kFaceThreads), 0, op->stream>>>(a, fbx, fby, fbz, y);
-    PTMF_HIP(hipGetLastError());
-  }
-  return PTMF_OK;
+  return finish_rows<T>(op, a, fin, up, fbx, fby, fbz, x, y);
 }
 
 template <typename T>
-int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, int faces) {
-  return launch_a11_mult_fb<T>(op, x, y, faces, (T *)op->faces, op->faces_doubles);
+int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, bool whole) {
+  return launch_a11_mult_fb<T>(op, whole ? kFinMult : kFinNone, nullptr, x, y, (T *)op->faces, op->faces_doubles);
+}
+
+template <typename T>
+int launch_a11_update(ptmf_op_s *op, const T *x, T *r, const RowUpdate<T> &up) {
+  return launch_a11_mult_fb<T>(op, kFinUpdate, &up, x, r, (T *)op->faces, op->faces_doubles);
 }
 
 template <typename T>
@@ -1628,7 +1739,7 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   // lane kernel 41 us and the tile kernel 62 us, and further apart above)
   TileArgs la;
   if (lane_tiles<T>(op, op->faces_doubles, kOtherTile, la))
-    return launch_lane<T, true>(op, la, 1, x, x + nu, y, y + nu, (T *)op->faces);
+    return launch_lane<T, true>(op, la, kFinMult, nullptr, x, x + nu, y, y + nu, (T *)op->faces);
   PTMF_TRY(ensure_eta_tiled<T>(op));
   const T *et = sizeof(T) == 8 ? (const T *)op->et64 : (const T *)op->et32;
   const TileArgs a = tile_args(op);
@@ -1650,8 +1761,10 @@ int prepare_eta_tiled(ptmf_op_s *op) { return ensure_eta_tiled<double>(op); }
 
 template int launch_a11<double>(const ptmf_op_s *, const double *, double *, bool);
 template int launch_a11<float>(const ptmf_op_s *, const float *, float *, bool);
-template int launch_a11_mult<double>(ptmf_op_s *, const double *, double *, int);
-template int launch_a11_mult<float>(ptmf_op_s *, const float *, float *, int);
+template int launch_a11_mult<double>(ptmf_op_s *, const double *, double *, bool);
+template int launch_a11_mult<float>(ptmf_op_s *, const float *, float *, bool);
+template int launch_a11_update<double>(ptmf_op_s *, const double *, double *, const RowUpdate<double> &);
+template int launch_a11_update<float>(ptmf_op_s *, const float *, float *, const RowUpdate<float> &);
 
 }  // namespace ptmf
 
@@ -1954,5 +2067,5 @@ extern "C" int ptmf_a11_mult_noalloc(ptmf_op op, const double *x, double *y) {
              need, kScratchDoubles);
   double *fb = nullptr;
   PTMF_TRY(scratch_address(dev, &fb));
-  return ptmf::launch_a11_mult_fb<double>(op, x, y, 1, fb, kScratchDoubles, true);
+  return ptmf::launch_a11_mult_fb<double>(op, ptmf::kFinMult, nullptr, x, y, fb, kScratchDoubles, true);
 }

@@ -225,8 +225,7 @@ __device__ __forceinline__ void col_sum(const ColArgs &a, unsigned I, unsigned J
       }
 }
 
-// node n of y from the element sums.  x: Dirichlet rows y = x (nullptr: sums
-// there too)
+// node n of y from the element sums, Dirichlet rows y = x
 constexpr int kColSumThreads = 256;
 template <typename T>
 __device__ __forceinline__ void col_node(const ColArgs &a, unsigned n, const T *__restrict__ es, T *__restrict__ y,
@@ -236,7 +235,7 @@ __device__ __forceinline__ void col_node(const ColArgs &a, unsigned n, const T *
   if (K > 2 * a.mz) return;
   T sum[3];
   col_sum<T>(a, I, J, K, es, sum);
-  const unsigned m = x ? (unsigned)bcn[n] : 0u;
+  const unsigned m = bcn[n];
 #pragma unroll
   for (int l = 0; l < 3; l++) y[3 * (long)n + l] = ((m >> l) & 1u) ? x[3 * (long)n + l] : sum[l];
 }
@@ -246,4 +245,21 @@ __global__ void __launch_bounds__(kColSumThreads)
     col_sum_kernel(ColArgs a, const T *__restrict__ es, T *__restrict__ y, const uint8_t *__restrict__ bcn,
                    const T *__restrict__ x) {
   col_node<T>(a, blockIdx.x * (unsigned)kColSumThreads + threadIdx.x, es, y, bcn, x);
+}
+
+// the same with a RowUpdate of the row
+template <typename T, UpdateKind kUp>
+__global__ void __launch_bounds__(kColSumThreads)
+    col_update_kernel(ColArgs a, const T *__restrict__ es, const uint8_t *__restrict__ bcn, const T *__restrict__ x,
+                      RowUpdate<T> up) {
+  const unsigned n = blockIdx.x * (unsigned)kColSumThreads + threadIdx.x, X = 2 * a.mx + 1, Y = 2 * a.my + 1;
+  const unsigned r = n / X, I = n - r * X, K = r / Y, J = r - K * Y;
+  if (K > 2 * a.mz) return;
+  UpdateRow<T, kUp> u[3];
+#pragma unroll
+  for (int l = 0; l < 3; l++) u[l].load(up, 3 * (long)n + l, x, bcn[n]);
+  T sum[3];
+  col_sum<T>(a, I, J, K, es, sum);
+#pragma unroll
+  for (int l = 0; l < 3; l++) u[l].store(up, 3 * (long)n + l, l, sum[l]);
 }

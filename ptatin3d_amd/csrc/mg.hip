@@ -158,30 +158,6 @@ __global__ void k_cheb_first(long n, const Tb *__restrict__ b, const T *__restri
   }
 }
 
-// p_kp1 = (omega scale) dinv (b - A p_k) + (1 - omega) p_km1 + omega p_k;
-// with bcn (per-node Dirichlet bits) the Dirichlet rows of A p_k are taken as
-// p_k (the MatMult's y = x), so Apk may hold the element sums there
-// pkp1 may be pkm1 (the step overwrites the iterate before last in place);
-// pkm1 == nullptr stands for a zero iterate.  To: the type the new iterate
-// is stored in (the FP64 output of an FP32 V-cycle's last step: the step
-// and the cast in one pass).
-template <typename T, typename To = T>
-__global__ void k_cheb_step(long n, const T *__restrict__ b, const T *__restrict__ Apk,
-                            const T *__restrict__ dinv, const T *pkm1,
-                            const T *__restrict__ pk, T os, T om1, T om, To *pkp1,
-                            const uint8_t *__restrict__ bcn = nullptr) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    T ap = Apk[i];
-    if (bcn) {
-      const long nd = i / 3;
-      if ((bcn[nd] >> (int)(i - 3 * nd)) & 1u) ap = pk[i];
-    }
-    const T z = (b[i] - ap) * dinv[i];
-    const T prev = pkm1 ? pkm1[i] : T(0);
-    pkp1[i] = (To)(os * z + om1 * prev + om * pk[i]);
-  }
-}
-
 // partial sums of the dot products <V_j, w>, j in [j0, j0 + nk), nk <= 8,
 // one value per block: part[j * gridDim.x + block]
 __global__ void k_mdot_partial(long n, int j0, int nk, const double *const *__restrict__ V,
@@ -833,7 +809,7 @@ __global__ void k_q1_point_nodes(int mx, int my, int mz, const double *__restric
 // sums are reduced through LDS.
 // kCheb: the Chebyshev-Jacobi step is applied to the product as it is
 // formed, pkp1 = os dinv (b - A x) + om1 pkm1 + om x (x = p_k), and y is not
-// written (the same arithmetic as the product followed by k_cheb_step);
+// written (the same arithmetic as the product followed by the step);
 // pkp1 may be pkm1 (in place), pkm1 == nullptr stands for zero.
 constexpr int kStNodes = 16;
 template <typename T, bool kCheb = false>
@@ -1205,7 +1181,10 @@ int cheb(ptmf_mg_s *mg, MGLevel &L, const T *b, T *x, int its, bool nonzero, con
   // V-cycle may be captured into a graph).
   T *prev = nullptr, *cur = p[0];
   PTMF_CHECK(!b64 || !nonzero, PTMF_ERR_ARG, "cheb: an FP64 right-hand side needs a zero initial guess");
-  if (nonzero) {
+  if (nonzero && !L.galerkin) {
+    PTMF_TRY(launch_a11_update<T>(L.op, x, r, RowUpdate<T>{b, dinv, nullptr, (T)scale, T(0), T(1), cur, false}));
+    prev = x;
+  } else if (nonzero) {
     PTMF_TRY(matmult<T>(L, x, r));
     k_cheb_first<T><<<nblocks(n), kBS, 0, s>>>(n, b, r, x, dinv, (T)scale, cur);
     prev = x;
@@ -1229,17 +1208,13 @@ int cheb(ptmf_mg_s *mg, MGLevel &L, const T *b, T *x, int its, bool nonzero, con
       k_stencil_apply<T, true><<<dim3((unsigned)nb), dim3(25 * kStNodes), 0, L.op->stream>>>(
           bx.X, bx.Y, bx.Z, S, cur, r, b, dinv, prev, (T)(omega * scale), (T)(1.0 - omega), (T)omega, out);
     } else {
-      // MatMult without its Dirichlet-copy launch; the update takes y = x there
-      PTMF_TRY(launch_a11_mult<T>(L.op, cur, r, 2));
-      if (x64 && i == its - 1) {
-        // the last step stores the result in FP64
-        k_cheb_step<T, double><<<nblocks(n), kBS, 0, s>>>(n, b, r, dinv, prev, cur, (T)(omega * scale),
-                                                           (T)(1.0 - omega), (T)omega, x64, L.op->bcnode);
-        PTMF_HIP(hipGetLastError());
-        return PTMF_OK;
-      }
-      k_cheb_step<T><<<nblocks(n), kBS, 0, s>>>(n, b, r, dinv, prev, cur, (T)(omega * scale), (T)(1.0 - omega),
-                                                 (T)omega, out, L.op->bcnode);
+      // p_kp1 = (omega scale) dinv (b - A p_k) + (1 - omega) p_km1 + omega p_k
+      // with the MatMult's last pass; the last step may store the result in FP64
+      const bool last64 = x64 && i == its - 1;
+      PTMF_TRY(launch_a11_update<T>(L.op, cur, r,
+                                    RowUpdate<T>{b, dinv, prev, (T)(omega * scale), (T)(1.0 - omega), (T)omega,
+                                                 last64 ? (void *)x64 : (void *)out, last64}));
+      if (last64) return PTMF_OK;
     }
     PTMF_HIP(hipGetLastError());
     c[0] = c[1];
@@ -1295,9 +1270,13 @@ int vcycle(ptmf_mg_s *mg, int l, int lc, const T *b, T *x, const double *b64 = n
   // pre-smooth from zero
   PTMF_TRY(cheb<T>(mg, L, b, x, mg->opt.pre_its, false, b64));
   // residual and restriction
-  PTMF_TRY(matmult<T>(L, x, r));
-  k_residual<T><<<nblocks(L.n), kBS, 0, s>>>(L.n, b, r, r);
-  PTMF_HIP(hipGetLastError());
+  if (!L.galerkin) {
+    PTMF_TRY(launch_a11_update<T>(L.op, x, r, RowUpdate<T>{b, nullptr, nullptr, T(1), T(0), T(0), r, false}));
+  } else {
+    PTMF_TRY(matmult<T>(L, x, r));
+    k_residual<T><<<nblocks(L.n), kBS, 0, s>>>(L.n, b, r, r);
+    PTMF_HIP(hipGetLastError());
+  }
   PTMF_TRY(restrict_<T>(mg, l, r, bc));
   // coarse correction vanishing on the Dirichlet dofs: the coarse Dirichlet
   // rows are identities, so a nonzero restricted residual there would act as

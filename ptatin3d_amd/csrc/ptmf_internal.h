@@ -164,11 +164,22 @@ namespace ptmf {
 template <typename T>
 int launch_a11(const ptmf_op_s *op, const T *u, T *y, bool mask_columns);
 // MatMult_MFStokes_A11: y = A11 mask(x) on free rows, y = x on Dirichlet rows.
-// faces: 1 the whole MatMult; 0 the element (tile) kernel alone, for timing;
-// 2 without the Dirichlet rows (left as the element sums), for a consumer
-// that takes y = x there itself.
+// whole: false for the element kernel alone, for timing
 template <typename T>
-int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, int faces);
+int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, bool whole);
+// A row update in place of the product itself: out = os dinv (b - A x) + om1 prev
+// + om x, the second term left out with prev nullptr; with dinv nullptr the
+// residual b - A x alone.  out (FP64 where out64) may be prev or r but not x.
+template <typename T>
+struct RowUpdate {
+  const T *b, *dinv, *prev;
+  T os, om1, om;
+  void *out;
+  bool out64;
+};
+// r: work vector
+template <typename T>
+int launch_a11_update(ptmf_op_s *op, const T *x, T *r, const RowUpdate<T> &up);
 // build (or rebuild) the FP64 tile-ordered viscosity for the current
 // coefficients and tiling (allocates; set-up time)
 int prepare_eta_tiled(ptmf_op_s *op);
