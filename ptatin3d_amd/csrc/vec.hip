@@ -34,14 +34,31 @@ __global__ void __launch_bounds__(256) copy16_kernel(const uint4 *__restrict__ x
     y[i] = x[i];
 }
 
-// element-major [27e+q] -> quadrature-point-major [q*nel+e], FP64 and FP32
-__global__ void eta_qpmajor_kernel(long nel, const double *__restrict__ em, double *__restrict__ q64,
-                                   float *__restrict__ q32) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < 27 * nel; t += (long)gridDim.x * blockDim.x) {
-    const long q = t / nel, e = t - q * nel;
-    const double v = em[27 * e + q];
-    q64[t] = v;
-    q32[t] = (float)v;
+// element-major [27e+q] -> quadrature-point-major [q*nel+e], FP64 and FP32.
+// Bound by memory (44 bytes a value in all): 64 elements at a time are turned
+// round in LDS, so that both sides move in whole lines (48^3 11.2 us; read with a
+// stride of 27 values 20.5 us).
+constexpr int kEtaElems = 64;
+__global__ void __launch_bounds__(256) eta_qpmajor_kernel(long nel, const double *__restrict__ em,
+                                                          double *__restrict__ q64, float *__restrict__ q32) {
+  __shared__ double sm[27 * kEtaElems];
+  const long e0 = (long)kEtaElems * blockIdx.x;
+  const int ne = (int)min((long)kEtaElems, nel - e0);
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    const int t = 256 * k + threadIdx.x;
+    if (t < 27 * ne) sm[t] = em[27 * e0 + t];
+  }
+  __syncthreads();
+  const int e = threadIdx.x % kEtaElems;
+  if (e >= ne) return;
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    const int q = 256 / kEtaElems * k + threadIdx.x / kEtaElems;
+    if (q >= 27) break;
+    const double v = sm[27 * e + q];
+    q64[q * nel + e0 + e] = v;
+    q32[q * nel + e0 + e] = (float)v;
   }
 }
 
@@ -86,7 +103,9 @@ int launch_copy16(const void *x, void *y, long n16, hipStream_t s) {
 }
 
 int launch_eta_qpmajor(long nel, const double *em, double *q64, float *q32, hipStream_t s) {
-  eta_qpmajor_kernel<<<grid_for(27 * nel, 256), 256, 0, s>>>(nel, em, q64, q32);
+  const long nb = (nel + kEtaElems - 1) / kEtaElems;
+  if (nb >= (1L << 31)) return ptmf_set_error(PTMF_ERR_ARG, "viscosity: %ld elements", nel);
+  eta_qpmajor_kernel<<<dim3((unsigned)nb), 256, 0, s>>>(nel, em, q64, q32);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

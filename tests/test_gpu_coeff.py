@@ -43,3 +43,24 @@ def test_diagonal_and_powerlaw_parity(gpu, m):
     A.powerlaw_viscosity(du, dB, 3.0, 1e-3, 1e3, dB)  # in place
     assert np.array_equal(dB.download(), de.download())
     A.destroy()
+
+
+@pytest.mark.parametrize("m", [(1, 1, 1), (9, 7, 1), (8, 4, 2), (13, 5, 1), (11, 6, 9)])
+@pytest.mark.parametrize("tiling", [None, (4, 3, 2)])
+def test_viscosity_copies(gpu, m, tiling):
+    """The copies of a viscosity given on the device (63, 64, 65 elements and
+    others; partial tiles and chunks) are those of one given on the host: the
+    MatMults are bit-identical."""
+    rng = np.random.default_rng(6)
+    eta = F.eta_loguniform(m[0] * m[1] * m[2], 1e-2, 1e2, rng)
+    coords = F.perturb_interior(F.box_coords(*m), *m, 0.1, rng)
+    u = rng.uniform(-1.0, 1.0, 3 * F.nnodes(*m))
+    ops = [MatA11MF(*m).setup(coords, e, F.dirichlet_all_faces(*m)) for e in (eta, np.ones_like(eta))]
+    for A in ops:
+        if tiling:
+            A.set_tiling(*tiling)
+    ops[1].set_viscosity_device(DeviceArray.from_host(eta.reshape(-1)))
+    for prec in (64, 32):
+        assert np.array_equal(ops[0].mult_host(u, precision=prec), ops[1].mult_host(u, precision=prec))
+    for A in ops:
+        A.destroy()
