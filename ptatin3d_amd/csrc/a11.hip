@@ -1833,7 +1833,10 @@ int batch_prepare_boxes(ptmf_batch_s *b) {
                "batch: operator %d: MF operator not setup", i);
     ptmf::BoxDesc &d = box[i];
     memset((void *)&d, 0, sizeof(d));  // (compared bytewise)
-    if (!col(op)) PTMF_TRY(ptmf::ensure_eta_tiled<T>(op));
+    if (!col(op)) {
+      PTMF_TRY(ptmf::ensure_eta_tiled<T>(op));
+      PTMF_HIP(hipStreamSynchronize(op->stream));  // (built on the operator's own stream)
+    }
     d.a = ptmf::tile_args(op);
     const ptmf::OpData<T> &od = *(const ptmf::OpData<T> *)(ip == 0 ? (const void *)&op->d64 : (const void *)&op->d32);
     d.xc = od.coords;
@@ -1852,8 +1855,6 @@ int batch_prepare_boxes(ptmf_batch_s *b) {
     }
     if (d.nbc > b->maxnbc) b->maxnbc = d.nbc;
   }
-  // the tile-ordered viscosity is built on each operator's own stream
-  for (ptmf_op op : b->ops) PTMF_HIP(hipStreamSynchronize(op->stream));
   const size_t bytes = sizeof(ptmf::BoxDesc) * n;
   if (!b->dbox[ip]) PTMF_HIP(hipMalloc((void **)&b->dbox[ip], bytes));
   const unsigned char *raw = (const unsigned char *)box.data();
