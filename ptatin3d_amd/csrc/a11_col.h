@@ -173,15 +173,20 @@ __device__ __forceinline__ void col_wave(const ColArgs &a, unsigned wave, const 
       const T f2 = A[0][2] * S[0][l] + A[1][2] * S[1][l] + A[2][2] * S[2][l];
       // the level's slots of the forward fields are read by now
       sm[3 * l + k][lane] = f1;
-      w[3 * l + k] += col_mix_x<T>(f0, rx.ct) + ry.ct[0] * f1;
+      w[3 * l + k] += rx.ct[0] * f0;
+      w[3 * l + k] += rx.ct[1] * col_x<1>(f0);
+      w[3 * l + k] += rx.ct[2] * col_x<2>(f0);
+      w[3 * l + k] += ry.ct[0] * f1;
 #pragma unroll
       for (int q = 0; q < 3; q++)
         if (k != 1 || q != 1) w[3 * l + q] += (T)kC[k][q] * f2;
     }
     col_fence();
 #pragma unroll
-    for (int l = 0; l < 3; l++)
-      w[3 * l + k] += ry.ct[1] * sm[3 * l + k][n1] + ry.ct[2] * sm[3 * l + k][n2];
+    for (int l = 0; l < 3; l++) {
+      w[3 * l + k] += ry.ct[1] * sm[3 * l + k][n1];
+      w[3 * l + k] += ry.ct[2] * sm[3 * l + k][n2];
+    }
     col_fence();
   }
 #pragma unroll

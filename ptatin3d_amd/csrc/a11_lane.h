@@ -12,10 +12,10 @@
 // element's: no Jacobian, adjugate or division per point.
 //
 // What bounds it: instruction issue of the one (FP64) or two (FP32) waves per
-// SIMD that the registers allow.  FP64: 256 VGPRs + 150 AGPRs, about 4,900
-// vector instructions per layer of which 3,340 are FP64 arithmetic, VALU busy
-// 44 % of the wave's cycles.  64^3, MI355X: 79.6 us in FP64 (tile kernel 178
-// us), 48 us in FP32 (82 us).  The loads are the delicate part: a value that
+// SIMD that the registers allow.  FP64: 256 VGPRs + 168 AGPRs, about 4,200
+// vector instructions per layer of which 3,050 are FP64 arithmetic, VALU busy
+// 57 % of the wave's cycles, waiting 20 %.  64^3, MI355X: 62 us in FP64 (tile
+// kernel 178 us), 35 us in FP32 (82 us).  The loads are the delicate part: a value that
 // is still in flight when the registers run short is waited for at once, to
 // be moved to an accumulation register or to scratch, one round trip each (the
 // same kernel with its loads in flight across the stress stage took 130 us,
@@ -51,9 +51,8 @@ __device__ __forceinline__ void ldot_t(int a, const T c[3], T v, T &y0, T &y1, T
     y1 += c[1] * v;
     y2 -= c[2] * v;
   } else if (a == 1) {
-    const T t = c[2] * v;
-    y0 -= t;
-    y2 += t;
+    y0 -= c[2] * v;
+    y2 += c[2] * v;
   } else {
     y0 += c[2] * v;
     y1 -= c[1] * v;

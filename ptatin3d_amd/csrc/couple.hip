@@ -46,7 +46,7 @@ __device__ __forceinline__ void pressure_frame(const double *s0, const double *s
 //
 // Bound by instruction issue at one wave
 // per SIMD (4,100 FP64 instructions a layer of 64 elements, two thirds of the
-// kernel's): 64 x 48 x 40 in 57 us and 5 us of faces; one 27-lane group per
+// kernel's): 64 x 48 x 40 in 44 us and 11 us of faces; one 27-lane group per
 // element with atomic adds to y took 290 us.
 // ---------------------------------------------------------------------------
 struct A12Op {
@@ -117,7 +117,7 @@ struct A12Op {
 // element centres (a lane loads its own), so that a wave's 40,608 B let four
 // waves live on a CU.  A layer's rows are all in flight before the first is
 // stored: one exposed latency a layer, in place of five slots that would leave
-// two waves a CU.  Bound by instruction issue: 64 x 48 x 40 in 35 us (53 us at
+// two waves a CU.  Bound by instruction issue: 64 x 48 x 40 in 40 us (53 us at
 // three waves a CU with the centres in the slots); 27 lanes per element with a
 // reduction over them took 330 us.
 // ---------------------------------------------------------------------------

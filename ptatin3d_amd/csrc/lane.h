@@ -220,15 +220,18 @@ __device__ __forceinline__ void lane_field_t(const T W[9], const T Z[9], T d0, T
   interp_plane_t<T>(Z, Zn);
 #pragma unroll
   for (int n = 0; n < 9; n++) {
+    // (each term an addition to the sum: one operation apiece)
     if (c == 1) {
-      const T z = d2 * Zn[n];
-      o0[n] -= z;
+      o0[n] -= d2 * Zn[n];
       o1[n] += Wn[n];
-      o2[n] += z;
+      o2[n] += d2 * Zn[n];
     } else {
-      o0[n] += (T)kB[c][0] * Wn[n] + d0 * Zn[n];
-      o1[n] += (T)kB[c][1] * Wn[n] + d1 * Zn[n];
-      o2[n] += (T)kB[c][2] * Wn[n] + d2 * Zn[n];
+      o0[n] += (T)kB[c][0] * Wn[n];
+      o0[n] += d0 * Zn[n];
+      o1[n] += (T)kB[c][1] * Wn[n];
+      o1[n] += d1 * Zn[n];
+      o2[n] += (T)kB[c][2] * Wn[n];
+      o2[n] += d2 * Zn[n];
     }
   }
   __builtin_amdgcn_sched_barrier(0);

@@ -15,19 +15,18 @@ __device__ __forceinline__ T sel3(int c, double a0, double a1, double a2) {
 
 // 1-D operators written with the exact structure of the Gauss tables (the
 // compiler may not drop multiplications by exact zeros or ones under IEEE
-// rules): B = [[e+o, m, e-o], [0, 1, 0], [e-o, m, e+o]] with e = 0.3,
-// o = sqrt(3/5)/2, m = 0.4, evaluated in even/odd form (6 operations instead
-// of 9).  interp3: y = B x; interp3t: y = B^T x.
+// rules): B = [[a, m, b], [0, 1, 0], [b, m, a]] with a, b = e +- o, e = 0.3,
+// o = sqrt(3/5)/2, m = 0.4.  interp3: y = B x, in 5 operations; interp3t: y =
+// B^T x, in even/odd form in 6.
 constexpr double kBe = 0.5 * (kB[0][0] + kB[0][2]);
 constexpr double kBo = 0.5 * (kB[0][0] - kB[0][2]);
 
 template <typename T>
 __device__ __forceinline__ void interp3(T x0, T x1, T x2, T &y0, T &y1, T &y2) {
-  const T sm = x0 + x2, df = x0 - x2;
-  const T t = (T)kB[0][1] * x1 + (T)kBe * sm;
-  y0 = t + (T)kBo * df;
+  const T p = (T)kB[0][1] * x1, u = p + (T)kB[0][2] * x2, v = p + (T)kB[2][2] * x2;
+  y0 = u + (T)kB[0][0] * x0;
   y1 = x1;
-  y2 = t - (T)kBo * df;
+  y2 = v + (T)kB[2][0] * x0;
 }
 
 template <typename T>
