@@ -1052,26 +1052,32 @@ __global__ void __launch_bounds__(64)
 // wave would walk one dependent load/store round after another.
 constexpr int kFaceThreads = 256;
 
-// It adds the face sums and, in the work-groups past the tiles, copies the
-// Dirichlet rows y = x, which the face sums leave alone: beside
-// the others' face sums and not after them (64^3: 15 us for the faces alone and for both, a launch of its own
-// took 5 us more; copied by the lane kernel as it writes the other rows 16 us).
-constexpr int kCopyGroup = 8 * kFaceThreads;  // rows per work-group
+// It adds the face sums and copies the Dirichlet rows y = x, which the face sums
+// leave alone, in work-groups of their own: beside the sums and not after them
+// (64^3: 13 us for both, apart 5 us more; copied by the lane kernel as it writes
+// the other rows 16 us more).
+constexpr int kCopyGroup = 4 * kFaceThreads;  // rows per work-group
 template <typename T>
 __global__ void __launch_bounds__(kFaceThreads)
     a11_face_copy_kernel(TileArgs a, const T *__restrict__ fbx, const T *__restrict__ fby, const T *__restrict__ fbz,
                          T *__restrict__ y, const uint8_t *__restrict__ bcn, const long *__restrict__ bcidx, long nbc,
                          const T *__restrict__ x) {
-  if (blockIdx.x < a.ntiles) {
-    face_sum<T, true>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
+  // (the copies first: they are short, and the face sums fill up behind them)
+  const long g = (long)blockIdx.x - ((long)gridDim.x - a.ntiles);
+  if (g >= 0) {
+    face_sum<T, true>(a, xcd_tile(g, a.ntiles), fbx, fby, fbz, y, bcn);
     return;
   }
-  const long i0 = (long)kCopyGroup * (blockIdx.x - a.ntiles);
+  constexpr int kN = kCopyGroup / kFaceThreads;
+  const long i0 = (long)kCopyGroup * blockIdx.x + threadIdx.x;
+  long idx[kN];
+  T v[kN];
 #pragma unroll
-  for (int k = 0; k < kCopyGroup / kFaceThreads; k++) {
-    const long i = i0 + kFaceThreads * k + threadIdx.x;
-    if (i < nbc) y[bcidx[i]] = x[bcidx[i]];
-  }
+  for (int k = 0; k < kN; k++) idx[k] = bcidx[min(i0 + kFaceThreads * k, nbc - 1)];
+#pragma unroll
+  for (int k = 0; k < kN; k++) v[k] = x[idx[k]];
+#pragma unroll
+  for (int k = 0; k < kN; k++) y[idx[k]] = v[k];
 }
 
 // RowUpdates by what they read besides b: nothing (a residual), dinv, or dinv
@@ -1585,7 +1591,8 @@ int eta_tiled_in_place(ptmf_op_s *op) {
 template <typename T>
 int launch_face_copy(const ptmf_op_s *op, const TileArgs &a, const T *fbx, const T *fby, const T *fbz, const T *x,
                      T *y) {
-  const long groups = a.ntiles + (op->nbc + kCopyGroup - 1) / kCopyGroup;
+  // (whole rounds of the XCDs, so that each keeps its own tiles; a row copied twice is the same)
+  const long copies = 8 * ((op->nbc + 8 * kCopyGroup - 1) / (8 * kCopyGroup)), groups = a.ntiles + copies;
   PTMF_CHECK(groups < (1L << 31), PTMF_ERR_ARG, "a11: mesh too large (%ld work-groups)", groups);
   a11_face_copy_kernel<T><<<dim3((unsigned)groups), dim3(kFaceThreads), 0, op->stream>>>(
       a, fbx, fby, fbz, y, op->bcnode, op->bcidx, op->nbc, x);

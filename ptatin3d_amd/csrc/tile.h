@@ -145,33 +145,42 @@ __device__ __forceinline__ void face_sum(const TileArgs &a, long tile, const T *
       il = iz0 + r % w; jl = jz0 + r / w; kl = 0;
     }
     const int I = 2 * tb.x0 + il, J = 2 * tb.y0 + jl, K = 2 * tb.z0 + kl;
-    T acc[3] = {T(0), T(0), T(0)};
-    for (int dz = (kl == 0 && hz) ? -1 : 0; dz <= 0; dz++)
-      for (int dy = (jl == 0 && hy) ? -1 : 0; dy <= 0; dy++)
-        for (int dx = (il == 0 && hx) ? -1 : 0; dx <= 0; dx++) {
-          if (dx == 0 && dy == 0 && dz == 0) continue;
-          const long tp = (tb.tx + dx) + (long)a.ntx * ((tb.ty + dy) + (long)a.nty * (tb.tz + dz));
-          const int ilp = I - 2 * (tb.tx + dx) * a.TX, jlp = J - 2 * (tb.ty + dy) * a.TY,
-                    klp = K - 2 * (tb.tz + dz) * a.ZC;
-          const T *src;
-          if (dx == -1)
-            src = fbx + 3 * (tp * a.fbx_n + jlp + (long)(2 * a.TY + 1) * klp);
-          else if (dy == -1)
-            src = fby + 3 * (tp * a.fby_n + ilp + (long)(2 * a.TX + 1) * klp);
-          else
-            src = fbz + 3 * (tp * a.fbz_n + ilp + (long)(2 * a.TX + 1) * jlp);
-          acc[0] += src[0];
-          acc[1] += src[1];
-          acc[2] += src[2];
-        }
     const long n = (long)I + a.X * (long)J + a.XY * (long)K;
+    // all that the row needs is requested before any of it is used
     const unsigned m = kSkip ? (unsigned)bcn[n] : 0u;
+    T row[3], v[7][3];
 #pragma unroll
-    for (int l = 0; l < 3; l++)
-      if (!kSkip || !((m >> l) & 1u)) y[3 * n + l] += acc[l];
+    for (int l = 0; l < 3; l++) row[l] = y[3 * n + l];
+#pragma unroll
+    for (int s = 0; s < 7; s++) {  // the neighbours one tile on in x, y, z; lowest first
+      const int dx = s & 1 ? 0 : -1, dy = s & 2 ? 0 : -1, dz = s & 4 ? 0 : -1;
+      const bool has = (dx == 0 || (hx && il == 0)) && (dy == 0 || (hy && jl == 0)) && (dz == 0 || (hz && kl == 0));
+#pragma unroll
+      for (int l = 0; l < 3; l++) v[s][l] = T(0);
+      if (!has) continue;
+      const long tp = (tb.tx + dx) + (long)a.ntx * ((tb.ty + dy) + (long)a.nty * (tb.tz + dz));
+      const int ilp = I - 2 * (tb.tx + dx) * a.TX, jlp = J - 2 * (tb.ty + dy) * a.TY,
+                klp = K - 2 * (tb.tz + dz) * a.ZC;
+      const T *src;
+      if (dx == -1)
+        src = fbx + 3 * (tp * a.fbx_n + jlp + (long)(2 * a.TY + 1) * klp);
+      else if (dy == -1)
+        src = fby + 3 * (tp * a.fby_n + ilp + (long)(2 * a.TX + 1) * klp);
+      else
+        src = fbz + 3 * (tp * a.fbz_n + ilp + (long)(2 * a.TX + 1) * jlp);
+#pragma unroll
+      for (int l = 0; l < 3; l++) v[s][l] = src[l];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      T acc = v[0][l];
+#pragma unroll
+      for (int s = 1; s < 7; s++) acc += v[s][l];
+      if (!kSkip || !((m >> l) & 1u)) y[3 * n + l] = row[l] + acc;
+    }
   }
 }
-
 
 }  // namespace
 }  // namespace ptmf
