@@ -217,17 +217,28 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 template <typename T>
 __device__ __forceinline__ void col_sum(const ColArgs &a, unsigned I, unsigned J, unsigned K, const T *__restrict__ es,
                                         T sum[3]) {
-  const int x0 = (int)(I >> 1) - ((I & 1) ? 0 : 1), y0 = (int)(J >> 1) - ((J & 1) ? 0 : 1),
-            z0 = (int)(K >> 1) - ((K & 1) ? 0 : 1);
-  sum[0] = sum[1] = sum[2] = T(0);
-  for (int z = max(z0, 0); z <= min((int)(K >> 1), (int)a.mz - 1); z++)
-    for (int y = max(y0, 0); y <= min((int)(J >> 1), (int)a.my - 1); y++)
-      for (int x = max(x0, 0); x <= min((int)(I >> 1), (int)a.mx - 1); x++) {
-        const int i = (int)I - 2 * x, j = (int)J - 2 * y, k = (int)K - 2 * z;
-        const T *p = es + 3 * ((9 * k + j) * (long)a.ne + x + (long)a.mx * (y + (long)a.my * z)) + i;
+  T v[8][3];
 #pragma unroll
-        for (int l = 0; l < 3; l++) sum[l] += p[9 * l * (long)a.ne];
-      }
+  for (int s = 0; s < 8; s++) {  // all in flight together
+    const bool dx = s & 1, dy = s & 2, dz = s & 4;
+    const int x = (int)(I >> 1) - (dx ? 0 : 1), y = (int)(J >> 1) - (dy ? 0 : 1), z = (int)(K >> 1) - (dz ? 0 : 1);
+    const bool has = (dx ? x < (int)a.mx : !(I & 1) && x >= 0) && (dy ? y < (int)a.my : !(J & 1) && y >= 0) &&
+                     (dz ? z < (int)a.mz : !(K & 1) && z >= 0);
+#pragma unroll
+    for (int l = 0; l < 3; l++) v[s][l] = T(0);
+    if (!has) continue;
+    const int i = (int)I - 2 * x, j = (int)J - 2 * y, k = (int)K - 2 * z;
+    const T *p = es + 3 * ((9 * k + j) * (long)a.ne + x + (long)a.mx * (y + (long)a.my * z)) + i;
+#pragma unroll
+    for (int l = 0; l < 3; l++) v[s][l] = p[9 * l * (long)a.ne];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int l = 0; l < 3; l++) {
+    sum[l] = v[0][l];
+#pragma unroll
+    for (int s = 1; s < 8; s++) sum[l] += v[s][l];
+  }
 }
 
 // node n of y from the element sums, Dirichlet rows y = x
@@ -249,7 +260,7 @@ template <typename T>
 __global__ void __launch_bounds__(kColSumThreads)
     col_sum_kernel(ColArgs a, const T *__restrict__ es, T *__restrict__ y, const uint8_t *__restrict__ bcn,
                    const T *__restrict__ x) {
-  col_node<T>(a, blockIdx.x * (unsigned)kColSumThreads + threadIdx.x, es, y, bcn, x);
+  col_node<T>(a, (unsigned)xcd_tile(blockIdx.x, gridDim.x) * kColSumThreads + threadIdx.x, es, y, bcn, x);
 }
 
 // the same with a RowUpdate of the row
@@ -257,7 +268,8 @@ template <typename T, UpdateKind kUp>
 __global__ void __launch_bounds__(kColSumThreads)
     col_update_kernel(ColArgs a, const T *__restrict__ es, const uint8_t *__restrict__ bcn, const T *__restrict__ x,
                       RowUpdate<T> up) {
-  const unsigned n = blockIdx.x * (unsigned)kColSumThreads + threadIdx.x, X = 2 * a.mx + 1, Y = 2 * a.my + 1;
+  const unsigned n = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * kColSumThreads + threadIdx.x;
+  const unsigned X = 2 * a.mx + 1, Y = 2 * a.my + 1;
   const unsigned r = n / X, I = n - r * X, K = r / Y, J = r - K * Y;
   if (K > 2 * a.mz) return;
   UpdateRow<T, kUp> u[3];
