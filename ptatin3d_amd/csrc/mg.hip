@@ -81,43 +81,31 @@ __global__ void k_copy(long n, const T *__restrict__ x, T *__restrict__ y) {
     y[i] = x[i];
 }
 
-// Dense column-major product y = A x (A: n x m, leading dimension lda) in
-// two launches: each work-group forms the partial sums of kGvRows rows over
-// one chunk of kGvCols columns (x chunk staged in LDS, consecutive threads
-// read consecutive rows of a column), then the chunks are summed in a fixed
-// order, so the result is deterministic and no atomics are needed.
-constexpr int kGvRows = 256;
-constexpr int kGvCols = 512;
-
-__global__ void __launch_bounds__(kGvRows)
-    k_gemv_part(long n, long m, const double *__restrict__ A, long lda, const double *__restrict__ x,
-                double *__restrict__ part) {
-  __shared__ double xs[kGvCols];
-  const long j0 = (long)blockIdx.y * kGvCols;
-  const int nj = (int)(m - j0 < kGvCols ? m - j0 : kGvCols);
-  for (int t = threadIdx.x; t < nj; t += kGvRows) xs[t] = x[j0 + t];
-  __syncthreads();
-  const long i = (long)blockIdx.x * kGvRows + threadIdx.x;
+// y = A x of a dense symmetric matrix in full storage: one wave per row, read as
+// the column it equals, 512 contiguous bytes at a time, its lanes' sums added up
+// in a fixed order.  Bound by reading A (n = 2187: 38 MB in 14 us; a work-group of 256
+// rows per chunk of 512 columns left most of the chip idle, 67 us and a launch
+// for the chunks).
+__global__ void __launch_bounds__(kBS) k_symv(long n, const double *__restrict__ A, const double *__restrict__ x,
+                                              double *__restrict__ y) {
+  const long i = blockIdx.x * (long)(kBS / 64) + threadIdx.x / 64;
   if (i >= n) return;
-  const double *a = A + i + j0 * lda;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  int j = 0;
-  for (; j + 4 <= nj; j += 4) {
-    s0 += a[(long)j * lda] * xs[j];
-    s1 += a[(long)(j + 1) * lda] * xs[j + 1];
-    s2 += a[(long)(j + 2) * lda] * xs[j + 2];
-    s3 += a[(long)(j + 3) * lda] * xs[j + 3];
+  const int lane = threadIdx.x % 64;
+  const double *a = A + i * n;
+  constexpr int kU = 8;
+  double s[kU];
+#pragma unroll
+  for (int u = 0; u < kU; u++) s[u] = 0.0;
+  long j = lane;
+  for (; j + 64 * (kU - 1) < n; j += 64 * kU) {
+#pragma unroll
+    for (int u = 0; u < kU; u++) s[u] += a[j + 64 * u] * x[j + 64 * u];
   }
-  for (; j < nj; j++) s0 += a[(long)j * lda] * xs[j];
-  part[(long)blockIdx.y * n + i] = (s0 + s1) + (s2 + s3);
-}
-
-__global__ void k_gemv_sum(long n, int nchunks, const double *__restrict__ part, double *__restrict__ y) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int c = 0; c < nchunks; c++) s += part[(long)c * n + i];
-    y[i] = s;
-  }
+  for (; j < n; j += 64) s[0] += a[j] * x[j];
+  double t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) t += __shfl_xor(t, d);
+  if (lane == 0) y[i] = t;
 }
 
 // mirror the lower triangle of a column-major n x n matrix into its upper one
@@ -396,15 +384,23 @@ __global__ void k_prolong_add(int Xc, int Yc, int Xf, int Yf, int bpp, const T *
 // yc = P^T xf, gathered per coarse node from fine nodes 2i-1, 2i, 2i+1
 // (weights 1/2, 1, 1/2 per direction).  Launch as k_prolong_add, over the
 // coarse planes.
+// bcn: Dirichlet dofs of the coarse level to zero.  p: the first smoothing step
+// of the coarse level from zero, p = scale dinv yc.
 template <typename T>
 __global__ void k_restrict(int Xc, int Yc, int Xf, int Yf, int Zf, int bpp, const T *__restrict__ xf,
-                           T *__restrict__ yc) {
+                           T *__restrict__ yc, const uint8_t *__restrict__ bcn, const T *__restrict__ dinv, T scale,
+                           T *__restrict__ p) {
   const int q = xcd_item(blockIdx.x, gridDim.x);
   const int k = q / bpp;
   const int t = (q - k * bpp) * blockDim.x + threadIdx.x;
   if (t >= Xc * Yc) return;
-  const int j = t / Xc, i = t - j * Xc;
-  T s0 = 0, s1 = 0, s2 = 0;
+  const int j = t / Xc, i = t - j * Xc, node = t + Xc * Yc * k, g = 3 * node;
+  const unsigned m = bcn ? (unsigned)bcn[node] : 0u;
+  T d[3] = {0, 0, 0}, s[3] = {0, 0, 0};
+  if (p) {
+#pragma unroll
+    for (int l = 0; l < 3; l++) d[l] = dinv[g + l];
+  }
   for (int dk = -1; dk <= 1; dk++) {
     const int K = 2 * k + dk;
     if (K < 0 || K >= Zf) continue;
@@ -418,16 +414,17 @@ __global__ void k_restrict(int Xc, int Yc, int Xf, int Yf, int Zf, int bpp, cons
         if (I < 0 || I >= Xf) continue;
         const T w = (di == 0 ? T(1) : T(0.5)) * wj * wk;
         const int f = 3 * (I + Xf * (J + Yf * K));
-        s0 += w * xf[f];
-        s1 += w * xf[f + 1];
-        s2 += w * xf[f + 2];
+#pragma unroll
+        for (int l = 0; l < 3; l++) s[l] += w * xf[f + l];
       }
     }
   }
-  const int g = 3 * (t + Xc * Yc * k);
-  yc[g] = s0;
-  yc[g + 1] = s1;
-  yc[g + 2] = s2;
+#pragma unroll
+  for (int l = 0; l < 3; l++) {
+    const T v = ((m >> l) & 1u) ? T(0) : s[l];
+    yc[g + l] = v;
+    if (p) p[g + l] = scale * (v * d[l]);
+  }
 }
 
 // Q2 embedding (transfer option 1): the fine nodal values of the coarse Q2
@@ -998,7 +995,6 @@ struct ptmf_mg_s {
   rocblas_handle blas = nullptr;
   ptmf::MFFactor *mf = nullptr; // multifrontal Cholesky of level 0 (sparse coarse factor)
   double *Adense = nullptr;     // explicit inverse, full symmetric (column-major)
-  double *dense_part = nullptr; // partial sums of the inverse's product
   int ndense = 0;
   int *dinfo = nullptr;
   // Krylov workspaces (finest level, FP64): velocity block and saddle point
@@ -1133,16 +1129,22 @@ int prolong_add(ptmf_mg_s *mg, int l, const T *xc, T *yf) {
   return PTMF_OK;
 }
 
+// (bcn, dinv, scale, p: as in k_restrict)
 template <typename T>
-int restrict_(ptmf_mg_s *mg, int l, const T *xf, T *yc) {
+int restrict_(ptmf_mg_s *mg, int l, const T *xf, T *yc, const uint8_t *bcn = nullptr, const T *dinv = nullptr,
+              T scale = T(0), T *p = nullptr) {
   const Box &bf = mg->lev[l].op->box, &bc = mg->lev[l - 1].op->box;
   if (mg->opt.transfer == 1) {
     k_restrict_q2<T><<<nblocks(bc.nnodes), kBS, 0, mg->stream>>>(bc.X, bc.Y, bc.Z, bf.X, bf.Y, bf.Z, xf, yc);
+    PTMF_HIP(hipGetLastError());
+    const ptmf_op_s *op = mg->lev[l - 1].op;
+    if (bcn) PTMF_TRY(launch_bc_set<T>(op->bcidx, op->nbc, T(0), yc, mg->stream));
+    if (p) k_cheb_first<T><<<nblocks(3 * bc.nnodes), kBS, 0, mg->stream>>>(3 * bc.nnodes, yc, nullptr, nullptr, dinv, scale, p);
   } else {
     PTMF_CHECK(3 * bf.nnodes < (1L << 31), PTMF_ERR_UNSUPPORTED, "restrict: level too large for 32-bit indices");
     const int bpp = (int)((bc.X * bc.Y + kBS - 1) / kBS);
     k_restrict<T><<<dim3((unsigned)(bpp * bc.Z)), kBS, 0, mg->stream>>>((int)bc.X, (int)bc.Y, (int)bf.X, (int)bf.Y,
-                                                                       (int)bf.Z, bpp, xf, yc);
+                                                                       (int)bf.Z, bpp, xf, yc, bcn, dinv, scale, p);
   }
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
@@ -1154,9 +1156,10 @@ int restrict_(ptmf_mg_s *mg, int l, const T *xf, T *yc) {
 // x64: the result goes to x64 in FP64 (the last step stores it) and x is not
 // written.  Both fold the precision casts of an FP32 V-cycle's finest level
 // into the smoother's first and last kernels.
+// started: the first step from zero is in the level's first work vector already.
 template <typename T>
 int cheb(ptmf_mg_s *mg, MGLevel &L, const T *b, T *x, int its, bool nonzero, const double *b64 = nullptr,
-         double *x64 = nullptr) {
+         double *x64 = nullptr, bool started = false) {
   hipStream_t s = mg->stream;
   const long n = L.n;
   T *p[3], *r;
@@ -1188,6 +1191,7 @@ int cheb(ptmf_mg_s *mg, MGLevel &L, const T *b, T *x, int its, bool nonzero, con
     PTMF_TRY(matmult<T>(L, x, r));
     k_cheb_first<T><<<nblocks(n), kBS, 0, s>>>(n, b, r, x, dinv, (T)scale, cur);
     prev = x;
+  } else if (started) {
   } else if (b64) {
     k_cheb_first<T, double><<<nblocks(n), kBS, 0, s>>>(n, b64, nullptr, nullptr, dinv, (T)scale, cur, (T *)b);
   } else {
@@ -1236,10 +1240,7 @@ int cheb(ptmf_mg_s *mg, MGLevel &L, const T *b, T *x, int its, bool nonzero, con
 // latency-bound triangular solves per V-cycle
 int dense_solve(ptmf_mg_s *mg, const double *b, double *x) {
   const long n = mg->ndense;
-  const int nchunks = (int)((n + kGvCols - 1) / kGvCols);
-  const dim3 grid((unsigned)((n + kGvRows - 1) / kGvRows), (unsigned)nchunks);
-  k_gemv_part<<<grid, kGvRows, 0, mg->stream>>>(n, n, mg->Adense, n, b, mg->dense_part);
-  k_gemv_sum<<<nblocks(n), kBS, 0, mg->stream>>>(n, nchunks, mg->dense_part, x);
+  k_symv<<<dim3((unsigned)((n + kBS / 64 - 1) / (kBS / 64))), kBS, 0, mg->stream>>>(n, mg->Adense, b, x);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }
@@ -1253,7 +1254,8 @@ int coarse_solve(ptmf_mg_s *mg, int lc, const double *b, double *x);
 // FP64, with b and x the level's buffers in T (the casts are folded into the
 // smoother's first and last kernels).
 template <typename T>
-int vcycle(ptmf_mg_s *mg, int l, int lc, const T *b, T *x, const double *b64 = nullptr, double *x64 = nullptr) {
+int vcycle(ptmf_mg_s *mg, int l, int lc, const T *b, T *x, const double *b64 = nullptr, double *x64 = nullptr,
+           bool started = false) {
   MGLevel &L = mg->lev[l];
   hipStream_t s = mg->stream;
   if (l == lc) {
@@ -1268,7 +1270,7 @@ int vcycle(ptmf_mg_s *mg, int l, int lc, const T *b, T *x, const double *b64 = n
   T *bc = sizeof(T) == 8 ? (T *)C.b64 : (T *)C.b32;
   T *xc = sizeof(T) == 8 ? (T *)C.x64 : (T *)C.x32;
   // pre-smooth from zero
-  PTMF_TRY(cheb<T>(mg, L, b, x, mg->opt.pre_its, false, b64));
+  PTMF_TRY(cheb<T>(mg, L, b, x, mg->opt.pre_its, false, b64, nullptr, started));
   // residual and restriction
   if (!L.galerkin) {
     PTMF_TRY(launch_a11_update<T>(L.op, x, r, RowUpdate<T>{b, nullptr, nullptr, T(1), T(0), T(0), r, false}));
@@ -1277,12 +1279,16 @@ int vcycle(ptmf_mg_s *mg, int l, int lc, const T *b, T *x, const double *b64 = n
     k_residual<T><<<nblocks(L.n), kBS, 0, s>>>(L.n, b, r, r);
     PTMF_HIP(hipGetLastError());
   }
-  PTMF_TRY(restrict_<T>(mg, l, r, bc));
   // coarse correction vanishing on the Dirichlet dofs: the coarse Dirichlet
   // rows are identities, so a nonzero restricted residual there would act as
   // boundary data of the correction
-  if (mg->opt.bc_transfer) PTMF_TRY(launch_bc_set<T>(C.op->bcidx, C.op->nbc, (T)0, bc, s));
-  PTMF_TRY(vcycle<T>(mg, l - 1, lc, bc, xc));
+  // (the coarse level's first smoothing step goes with the restriction)
+  const bool smooth = l - 1 > lc;
+  const T *dinv = sizeof(T) == 8 ? (const T *)C.dinv64 : (const T *)C.dinv32;
+  T *p = sizeof(T) == 8 ? (T *)C.p64[0] : (T *)C.p32[0];
+  PTMF_TRY(restrict_<T>(mg, l, r, bc, mg->opt.bc_transfer ? C.op->bcnode : nullptr, dinv,
+                        (T)(2.0 / (C.emax + C.emin)), smooth ? p : nullptr));
+  PTMF_TRY(vcycle<T>(mg, l - 1, lc, bc, xc, nullptr, nullptr, smooth));
   PTMF_TRY(prolong_add<T>(mg, l, xc, x));
   // post-smooth from the corrected iterate
   PTMF_TRY(cheb<T>(mg, L, b, x, mg->opt.post_its, true, nullptr, x64));
@@ -1499,11 +1505,9 @@ int assemble_dense(ptmf_mg_s *mg) {
   PTMF_HIP(hipStreamSynchronize(s));
   PTMF_CHECK(info == 0, PTMF_ERR_DIVERGED, "coarse inverse failed (info %d)", info);
   // full symmetric inverse for the project's own product kernel (the V-cycle
-  // graph then holds no library nodes); partial sums buffer of that product
+  // graph then holds no library nodes)
   k_symmetrize<<<nblocks(n * n), kBS, 0, s>>>(n, mg->Adense);
   PTMF_HIP(hipGetLastError());
-  if (!mg->dense_part)
-    PTMF_TRY(dalloc((void **)&mg->dense_part, sizeof(double) * n * ((n + kGvCols - 1) / kGvCols)));
   PTMF_HIP(hipStreamSynchronize(s));
   return PTMF_OK;
 }
@@ -1540,8 +1544,7 @@ int setup_coarse(ptmf_mg_s *mg) {
   if (cf == 1 || (cf == 0 && L.n <= kDenseMaxDofs)) return assemble_dense(mg);
   // the dense inverse of an earlier set-up must not be used any more
   (void)hipFree(mg->Adense);
-  (void)hipFree(mg->dense_part);
-  mg->Adense = mg->dense_part = nullptr;
+  mg->Adense = nullptr;
   mg->ndense = 0;
   // all-Dirichlet nodes (identity rows, zero columns) stay out of the factor
   std::vector<uint8_t> bch(L.op->box.nnodes);
@@ -1947,7 +1950,6 @@ int ptmf_mg_destroy(ptmf_mg *pmg) {
   if (mg->coef_host) (void)hipHostFree(mg->coef_host);
   ptmf::mf_destroy(mg->mf);
   (void)hipFree(mg->Adense);
-  (void)hipFree(mg->dense_part);
   (void)hipFree(mg->dinfo);
   if (mg->red_host) (void)hipHostFree(mg->red_host);
   if (mg->blas) rocblas_destroy_handle(mg->blas);
