@@ -725,7 +725,7 @@ __global__ void __launch_bounds__(64) k_q1_to_qp(int mx, int my, long nel, const
 // points of the same element each, one sum per lane; the runs then go to
 // memory with FP64 atomics (so the sums are formed in no fixed order), 18 next
 // to each other.  40 x 40 x 24 elements of 27 points: in element order (long
-// runs, close to the 41 MB it reads) 15 us, in no order (a run a point, bound
+// runs, close to the 41 MB it reads) 13 us, in no order (a run a point, bound
 // by the atomics) 140 us; with 54 atomics a point 3,040 and 2,480 us.
 constexpr int kPointRounds = 4;
 __global__ void __launch_bounds__(64) k_q1_point_sums(long npts, const long *__restrict__ elem,
@@ -736,12 +736,23 @@ __global__ void __launch_bounds__(64) k_q1_point_sums(long npts, const long *__r
   const int lane = threadIdx.x, g = lane / 18, i = lane - 18 * g;
   const double *wa = w[i < 16 ? i & 7 : 9], *wb = w[i < 8 || i == 16 ? 8 : 9];
   w[9][lane] = 1.0;
+  long en = 0;
+  double xn[3] = {0.0, 0.0, 0.0}, vn = 0.0;
+  auto fetch = [&](long p0) {  // the point of this lane, in flight while the points before it are added up
+    const long p = min(p0 + lane, npts - 1);
+    en = elem[p];
+    for (int d = 0; d < 3; d++) xn[d] = xi[3 * p + d];
+    vn = val[p];
+  };
+  const long first = 64L * blockIdx.x * kPointRounds;
+  fetch(first);
   for (int r = 0; r < kPointRounds; r++) {
-    const long p0 = 64 * ((long)blockIdx.x * kPointRounds + r);
+    const long p0 = first + 64 * r;
     if (p0 >= npts) break;
     const int np = (int)min(64L, npts - p0);
-    const long p = p0 + min(lane, np - 1), e = elem[p];
-    const double x0 = xi[3 * p], x1 = xi[3 * p + 1], x2 = xi[3 * p + 2], v = val[p];
+    const long e = en;
+    const double x0 = xn[0], x1 = xn[1], x2 = xn[2], v = vn;
+    if (r + 1 < kPointRounds) fetch(p0 + 64);
     const double f0[2] = {0.5 * (1.0 - x0), 0.5 * (1.0 + x0)}, f1[2] = {0.5 * (1.0 - x1), 0.5 * (1.0 + x1)},
                  f2[2] = {0.5 * (1.0 - x2), 0.5 * (1.0 + x2)};
     __syncthreads();
@@ -762,6 +773,7 @@ __global__ void __launch_bounds__(64) k_q1_point_sums(long npts, const long *__r
         end = g == h ? n : end;
       }
       double sum = 0.0;
+#pragma unroll 4
       for (int t = start; t < end; t++) sum += wa[t] * wb[t];
       if (start < end) atomicAdd(&sums[18 * se[start] + i], sum);
     }
@@ -770,27 +782,34 @@ __global__ void __launch_bounds__(64) k_q1_point_sums(long npts, const long *__r
 
 // nodal field of the element sums: a corner node's A / B from the corner sums
 // of its elements, another node's from their plain sums
-__global__ void k_q1_point_nodes(int mx, int my, int mz, const double *__restrict__ sums,
-                                 double *__restrict__ nodal) {
-  const long X = 2L * mx + 1, Y = 2L * my + 1, N = X * Y * (2L * mz + 1);
-  for (long n = blockIdx.x * (long)blockDim.x + threadIdx.x; n < N; n += (long)gridDim.x * blockDim.x) {
-    const long r = n / X, I = n - X * r, K = r / Y, J = r - Y * K;
-    long ex[2], ey[2], ez[2];
-    int lx[2], ly[2], lz[2];
-    const int nx = lattice_owners(I, mx, ex, lx), ny = lattice_owners(J, my, ey, ly),
-              nz = lattice_owners(K, mz, ez, lz);
-    const bool corner = !((I | J | K) & 1);
-    double A = 0.0, B = 0.0;
-    for (int c = 0; c < nz; c++)
-      for (int b = 0; b < ny; b++)
-        for (int a = 0; a < nx; a++) {
-          const int l = corner ? (lx[a] >> 1) + (ly[b] & 2) + 2 * (lz[c] & 2) : 16;
-          const double *s = sums + 18 * (ex[a] + mx * (ey[b] + (long)my * ez[c])) + l;
-          A += s[0];
-          B += s[corner ? 8 : 1];
-        }
-    nodal[n] = A / B;
+// (its loads are all in flight together)
+__global__ void __launch_bounds__(kBS) k_q1_point_nodes(int mx, int my, int mz, const double *__restrict__ sums,
+                                                        double *__restrict__ nodal) {
+  const unsigned n = blockIdx.x * (unsigned)kBS + threadIdx.x, X = 2u * mx + 1, Y = 2u * my + 1;
+  const unsigned r = n / X, I = n - X * r, K = r / Y, J = r - Y * K;
+  if (K > 2u * mz) return;
+  const bool corner = !((I | J | K) & 1);
+  double a[8], b[8], A = 0.0, B = 0.0;
+#pragma unroll
+  for (int s = 0; s < 8; s++) {  // elements before and after the node's plane in each direction, lowest first
+    const bool dx = s & 1, dy = s & 2, dz = s & 4;
+    const int x = (int)(I >> 1) - (dx ? 0 : 1), y = (int)(J >> 1) - (dy ? 0 : 1), z = (int)(K >> 1) - (dz ? 0 : 1);
+    const bool has = (dx ? x < mx : !(I & 1) && x >= 0) && (dy ? y < my : !(J & 1) && y >= 0) &&
+                     (dz ? z < mz : !(K & 1) && z >= 0);
+    a[s] = b[s] = 0.0;
+    if (!has) continue;
+    const int l = corner ? (dx ? 0 : 1) + (dy ? 0 : 2) + (dz ? 0 : 4) : 16;
+    const double *p = sums + 18 * (x + (long)mx * (y + (long)my * z)) + l;
+    a[s] = p[0];
+    b[s] = p[corner ? 8 : 1];
   }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    A += a[s];
+    B += b[s];
+  }
+  nodal[n] = A / B;
 }
 
 // ---------------------------------------------------------------------------
@@ -2617,8 +2636,8 @@ int ptmf_op_project_points(ptmf_op op, long npts, const long *elem, const double
   PTMF_CHECK(npts >= 0, PTMF_ERR_ARG, "project_points: %ld points", npts);
   const ptmf::Box &b = op->box;
   const long blocks = (npts + 64 * ptmf::kPointRounds - 1) / (64 * ptmf::kPointRounds);
-  PTMF_CHECK(blocks < (1L << 31) && b.nel < (64L << 31) - 64, PTMF_ERR_ARG, "project_points: too many points (%ld)",
-             npts);
+  PTMF_CHECK(blocks < (1L << 31) && b.nnodes < (1L << 32) - ptmf::kBS, PTMF_ERR_ARG,
+             "project_points: too many points (%ld) or nodes (%ld)", npts, b.nnodes);
   // the element sums and the nodal field stay with the operator; the call
   // waits for its kernels, so holding the lock makes it safe from any thread
   std::lock_guard<std::mutex> lock(op->points_mu);
@@ -2633,7 +2652,7 @@ int ptmf_op_project_points(ptmf_op op, long npts, const long *elem, const double
     if (hipGetLastError() != hipSuccess) st = ptmf_set_error(PTMF_ERR_DEVICE, "project_points: launch");
   }
   if (st == PTMF_OK) {
-    ptmf::k_q1_point_nodes<<<ptmf::nblocks(b.nnodes), ptmf::kBS, 0, s>>>(b.mx, b.my, b.mz, sums, nodal);
+    ptmf::k_q1_point_nodes<<<dim3((unsigned)((b.nnodes + ptmf::kBS - 1) / ptmf::kBS)), ptmf::kBS, 0, s>>>(b.mx, b.my, b.mz, sums, nodal);
     ptmf::k_q1_to_qp<<<dim3((unsigned)((b.nel + 63) / 64)), 64, 0, s>>>(b.mx, b.my, b.nel, nodal, eta);
     if (hipGetLastError() != hipSuccess) st = ptmf_set_error(PTMF_ERR_DEVICE, "project_points: launch");
   }
