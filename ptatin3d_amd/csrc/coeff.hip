@@ -196,11 +196,13 @@ __global__ void __launch_bounds__(64)
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
   double *const s1 = sm + 2 * 6 * kLPlane;
+  const double org = lane_origin(a, q, xc);
+  const double *const first = xc + 3 * lane_node(a, tb, 2 * tb.z0);
   PlaneRows r1, r2;
   {
     const long n = lane_node(a, tb, 2 * tb.z0);
     r2.load(q, a.X, xc + 3 * n, u + 3 * n);
-    r2.store<kLPlane>(q, sm);
+    r2.store<kLPlane>(q, sm, org);
   }
   for (int kz = 0; kz < tb.nzt; kz++) {
     const int ek = tb.z0 + kz;
@@ -212,11 +214,11 @@ __global__ void __launch_bounds__(64)
     r2.load(q, a.X, xc + 3 * n2, u + 3 * n2);
 #pragma unroll
     for (int f = 0; f < 3; f++) {
-      ctr[f] = xc[3 * nc + f];
+      ctr[f] = xc[3 * nc + f] - first[f];
       ctr[3 + f] = u[3 * nc + f];
     }
-    r1.store<kOdd>(q, s1);
-    r2.store<kLPlane>(q, s2);
+    r1.store<kOdd>(q, s1, org);
+    r2.store<kLPlane>(q, s2, org);
     __syncthreads();
     double X[3][9], XZ[3][9], U[3][9], UZ[3][9], e2[3][9];
     int lq = q.li;

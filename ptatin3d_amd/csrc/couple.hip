@@ -151,12 +151,14 @@ __global__ void __launch_bounds__(64)
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
   double *const s1 = sm + 2 * 6 * kLPlane;
+  const double org = lane_origin(a, q, xc);
+  const double *const first = xc + 3 * lane_node(a, tb, 2 * tb.z0);
   PlaneRows r1, r2;
   {
     const long n = lane_node(a, tb, 2 * tb.z0);
     r2.load(q, a.X, xc + 3 * n, u + 3 * n);
     r2.mask(lane_bc_word(a, q, bcw, 2 * tb.z0));
-    r2.store<kLPlane>(q, sm);
+    r2.store<kLPlane>(q, sm, org);
   }
   for (int kz = 0; kz < tb.nzt; kz++) {
     const int ek = tb.z0 + kz;
@@ -169,7 +171,7 @@ __global__ void __launch_bounds__(64)
     r2.load(q, a.X, xc + 3 * n2, u + 3 * n2);
 #pragma unroll
     for (int f = 0; f < 3; f++) {
-      ctr[f] = xc[3 * nc + f];
+      ctr[f] = xc[3 * nc + f] - first[f];
       ctr[3 + f] = u[3 * nc + f];
     }
     r1.mask(m1);
@@ -179,8 +181,8 @@ __global__ void __launch_bounds__(64)
         ctr[3 + f] = ((__shfl(m1, 3 * (2 * q.cx + 1) + f) >> (2 * q.cy + 1)) & 1u) ? 0.0 : ctr[3 + f];
     }
     r2.mask(m2);
-    r1.store<kOdd>(q, s1);
-    r2.store<kLPlane>(q, s2);
+    r1.store<kOdd>(q, s1, org);
+    r2.store<kLPlane>(q, s2, org);
     __syncthreads();
     double xb[3], L[3], X[3][9], XZ[3][9], U[3][9], UZ[3][9], acc[4] = {0.0, 0.0, 0.0, 0.0};
     int lq = q.li;

@@ -41,12 +41,19 @@ __device__ __forceinline__ void plane_fields(const double *s0, const double *s1,
                                            kD[c][2], V[f], Z[f], kP1 < kLPlane ? centre[f] : 0.0);
 }
 
+// the first node of the tile's chunk, the coordinate of the lane's rows
+__device__ __forceinline__ double lane_origin(const TileArgs &a, const LaneTile &q, const double *__restrict__ xc) {
+  return xc[3 * lane_node(a, q.tb, 2 * q.tb.z0) + q.d];
+}
+
 // Middle node planes may lack the element centres, which a lane then holds
 // itself: a smaller slot.
 constexpr int kOdd = 234;  // nodes of a plane slot without the element centres
 
 // One node plane of the tile on its way to its slot: the rows of its
 // coordinates and velocity; all of a layer's are in flight together.
+// Positions are kept from the tile's first node: an element's differences then
+// lose no digits to its distance from the origin.  org: lane_origin.
 struct PlaneRows {
   double x[kLRows], u[kLRows];
   __device__ __forceinline__ void load(const LaneTile &q, long X, const double *xc, const double *u_) {
@@ -60,14 +67,14 @@ struct PlaneRows {
   }
   // S: component stride of the slot
   template <int S>
-  __device__ __forceinline__ void store(const LaneTile &q, double *p) const {
+  __device__ __forceinline__ void store(const LaneTile &q, double *p, double org) const {
     const int ev = S * q.d + kLCls[q.il & 1] + (q.il >> 1);
     // (without centres their entries of the odd rows go to the rows' padding)
     const int od = S * q.d + (S == kLPlane ? kLCls[2 + (q.il & 1)] + (q.il >> 1)
                                            : ((q.il & 1) ? kLCls[1] + 8 : kLCls[2] + (q.il >> 1)));
 #pragma unroll
     for (int j = 0; j < kLRows; j++) {
-      p[(j & 1 ? od : ev) + kLRow * (j >> 1)] = x[j];
+      p[(j & 1 ? od : ev) + kLRow * (j >> 1)] = x[j] - org;
       p[(j & 1 ? od : ev) + kLRow * (j >> 1) + 3 * S] = u[j];
     }
   }
@@ -97,18 +104,28 @@ __global__ void __launch_bounds__(64)
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
   auto plane = [&](int P) { return LaneBuf<double>(xc + 3 * lane_node(a, tb, P)); };
+  const double org = lane_origin(a, q, xc);
+  auto shift = [&](double r[kLBatch]) {
+#pragma unroll
+    for (int k = 0; k < kLBatch; k++) r[k] -= org;
+  };
   {
     const LaneBuf<double> v0 = plane(2 * tb.z0), v1 = plane(2 * tb.z0 + 1), v2 = plane(2 * tb.z0 + 2);
     double r0[kLBatch], r1[kLBatch], r2[kLBatch];
     lane_rows_load<double, 0>(r0, q, a.X, v0, v1);
     lane_rows_load<double, 1>(r1, q, a.X, v0, v1);
+    shift(r0);
     lane_rows_store<double, 0>(r0, q, sm, sm + kLSlot);
     lane_rows_load<double, 2>(r2, q, a.X, v0, v1);
+    shift(r1);
     lane_rows_store<double, 1>(r1, q, sm, sm + kLSlot);
     lane_rows_load<double, 0, kLRows>(r0, q, a.X, v2, v2);
     lane_rows_load<double, 1, kLRows>(r1, q, a.X, v2, v2);
+    shift(r2);
     lane_rows_store<double, 2>(r2, q, sm, sm + kLSlot);
+    shift(r0);
     lane_rows_store<double, 0, kLRows>(r0, q, sm + 2 * kLSlot, nullptr);
+    shift(r1);
     lane_rows_store<double, 1, kLRows>(r1, q, sm + 2 * kLSlot, nullptr);
   }
   double out[3][3][9];
@@ -143,6 +160,7 @@ __global__ void __launch_bounds__(64)
     op.template load<0>();
     lane_rows_load<double, 0>(r, q, a.X, v1, v2);
     plane_fields<0>(s0 + lq, s1 + lq, s2 + lq, X, Z);
+    shift(r);
     lane_rows_store<double, 0>(r, q, s3, s4);
     op.template plane<0>(X, Z, out);
     lane_pin<double>(out);
@@ -150,6 +168,7 @@ __global__ void __launch_bounds__(64)
     op.template load<1>();
     lane_rows_load<double, 1>(r, q, a.X, v1, v2);
     plane_fields<1>(s0 + lq, s1 + lq, s2 + lq, X, Z);
+    shift(r);
     lane_rows_store<double, 1>(r, q, s3, s4);
     op.template plane<1>(X, Z, out);
     lane_pin<double>(out);
@@ -160,6 +179,7 @@ __global__ void __launch_bounds__(64)
     m2 = lane_bc_word(a, q, bcw, 2 * ek + 2);
     lane_rows_load<double, 2>(r, q, a.X, v1, v2);
     plane_fields<2>(s0 + lq, s1 + lq, s2 + lq, X, Z);
+    shift(r);
     lane_rows_store<double, 2>(r, q, s3, s4);
     asm volatile("" : "+v"(m0), "+v"(m1), "+v"(m2));
     op.template plane<2>(X, Z, out);
