@@ -92,6 +92,9 @@ __device__ __forceinline__ void col_wave(const ColArgs &a, unsigned wave, const 
 
   T v[18], et[3];  // [x, y, z, u_x, u_y, u_z][z index]
   unsigned m[3];
+  T org[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) org[d] = xc[3 * (node - i - X * j) + d];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const unsigned n = node + XY * k;
@@ -107,17 +110,12 @@ __device__ __forceinline__ void col_wave(const ColArgs &a, unsigned wave, const 
   for (int k = 0; k < 3; k++)
 #pragma unroll
     for (int d = 0; d < 3; d++) v[9 + 3 * d + k] = ((m[k] >> d) & 1u) ? T(0) : v[9 + 3 * d + k];
-  if constexpr (sizeof(T) == 4) {
-    // positions from the element's first node: no digits are lost to the
-    // element's distance from the origin
-    T o[3];
+  // positions from the element's first node: no digits are lost to the
+  // element's distance from the origin
 #pragma unroll
-    for (int d = 0; d < 3; d++) o[d] = __shfl(v[3 * d], 4 * s);
+  for (int d = 0; d < 3; d++)
 #pragma unroll
-    for (int d = 0; d < 3; d++)
-#pragma unroll
-      for (int k = 0; k < 3; k++) v[3 * d + k] -= o[d];
-  }
+    for (int k = 0; k < 3; k++) v[3 * d + k] -= org[d];
 #pragma unroll
   for (int f = 0; f < 6; f++) interp3<T>(v[3 * f], v[3 * f + 1], v[3 * f + 2], v[3 * f], v[3 * f + 1], v[3 * f + 2]);
 #pragma unroll
