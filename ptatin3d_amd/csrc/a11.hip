@@ -19,7 +19,7 @@
 //   * Viscosity is stored quadrature-point-major (eta[q*nel + e]) so the
 //     lanes of a wave read consecutive elements.
 //
-// Scatter (MatMult path, a11_tile_kernel + a11_face_kernel):
+// Scatter (MatMult path, a11_tile_kernel + a11_face_copy_kernel):
 //   * A wave owns a TX x TY tile of elements in x-y (TX*TY <= 21) and marches
 //     through a chunk of ZC element layers in z.  Element outputs are summed
 //     into an LDS window of three node planes (ordered plain read-add-write,
@@ -28,10 +28,13 @@
 //   * A tile owns its node range [2x0,2x1) x [2y0,2y1) x [2z0,2z1) (plus the
 //     closing planes at the domain's upper boundary).  Contributions to the
 //     tile's upper faces go to per-tile face buffers (x face first, then y,
-//     then z), and a11_face_kernel adds them into the owning tile's lower
+//     then z), and a11_face_copy_kernel adds them into the owning tile's lower
 //     faces.  No global atomics, no clearing of y, deterministic sums.
-//   * Dirichlet rows (y = x) are written last, over the compact list of
-//     Dirichlet dofs.
+//   * Dirichlet rows (y = x) are written by work-groups of the same launch,
+//     over the compact list of Dirichlet dofs.
+// This tile kernel has the large deformed meshes and the tilings and variants of
+// the caller's choice; rectilinear meshes take a11_lane.h and small boxes
+// a11_col.h (lane_plan and col_box below).
 // The spmv path (y += A u, no boundary handling) keeps a one-pass kernel with
 // global atomic adds; it serves the host-array PETSc adapter contract.
 #include <string.h>
@@ -1052,8 +1055,8 @@ __global__ void __launch_bounds__(64)
 // wave would walk one dependent load/store round after another.
 constexpr int kFaceThreads = 256;
 
-// It adds the face sums and copies the Dirichlet rows y = x, which the face sums
-// leave alone, in work-groups of their own: beside the sums and not after them
+// It adds the face sums and copies the Dirichlet rows y = x
+// (BCListInsertDirichlet_MatMult with scale 1), which the face sums leave alone, in work-groups of their own: beside the sums and not after them
 // (64^3: 13 us for both, apart 5 us more; copied by the lane kernel as it writes
 // the other rows 16 us more).
 constexpr int kCopyGroup = 4 * kFaceThreads;  // rows per work-group

@@ -197,8 +197,6 @@ int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>
 int launch_fill(T *x, T v, long n, hipStream_t s);
 template <typename T>
-int launch_bc_copy(const long *idx, long n, const T *x, T *y, hipStream_t s);
-template <typename T>
 int launch_bc_set(const long *idx, long n, T v, T *y, hipStream_t s);
 int launch_copy16(const void *x, void *y, long n16, hipStream_t s);
 int launch_eta_qpmajor(long nel, const double *em, double *q64, float *q32, hipStream_t s);

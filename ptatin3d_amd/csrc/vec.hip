@@ -11,17 +11,7 @@ __global__ void fill_kernel(T *__restrict__ x, T v, long n) {
     x[i] = v;
 }
 
-// y[idx[k]] = x[idx[k]]  (BCListInsertDirichlet_MatMult with scale 1)
-template <typename T>
-__global__ void bc_copy_kernel(const long *__restrict__ idx, long n, const T *__restrict__ x,
-                               T *__restrict__ y) {
-  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
-    const long g = idx[k];
-    y[g] = x[g];
-  }
-}
-
-// y[idx[k]] = v  (BCListInsertZero / BCListInsertValueIntoDirichletSlot)
+// y[idx[k]] = v
 template <typename T>
 __global__ void bc_set_kernel(const long *__restrict__ idx, long n, T v, T *__restrict__ y) {
   for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x)
@@ -80,14 +70,6 @@ int launch_fill(T *x, T v, long n, hipStream_t s) {
 }
 
 template <typename T>
-int launch_bc_copy(const long *idx, long n, const T *x, T *y, hipStream_t s) {
-  if (n <= 0) return PTMF_OK;
-  bc_copy_kernel<T><<<grid_for(n, 256), 256, 0, s>>>(idx, n, x, y);
-  PTMF_HIP(hipGetLastError());
-  return PTMF_OK;
-}
-
-template <typename T>
 int launch_bc_set(const long *idx, long n, T v, T *y, hipStream_t s) {
   if (n <= 0) return PTMF_OK;
   bc_set_kernel<T><<<grid_for(n, 256), 256, 0, s>>>(idx, n, v, y);
@@ -113,8 +95,6 @@ int launch_eta_qpmajor(long nel, const double *em, double *q64, float *q32, hipS
 template int launch_fill<double>(double *, double, long, hipStream_t);
 template int launch_fill<float>(float *, float, long, hipStream_t);
 template int launch_fill<int>(int *, int, long, hipStream_t);
-template int launch_bc_copy<double>(const long *, long, const double *, double *, hipStream_t);
-template int launch_bc_copy<float>(const long *, long, const float *, float *, hipStream_t);
 template int launch_bc_set<double>(const long *, long, double, double *, hipStream_t);
 template int launch_bc_set<float>(const long *, long, float, float *, hipStream_t);
 
