@@ -1056,9 +1056,10 @@ __global__ void __launch_bounds__(64)
 constexpr int kFaceThreads = 256;
 
 // It adds the face sums and copies the Dirichlet rows y = x
-// (BCListInsertDirichlet_MatMult with scale 1), which the face sums leave alone, in work-groups of their own: beside the sums and not after them
-// (64^3: 13 us for both, apart 5 us more; copied by the lane kernel as it writes
-// the other rows 16 us more).
+// (BCListInsertDirichlet_MatMult with scale 1), which the face sums leave alone,
+// in work-groups of their own: beside the sums and not after them (64^3: 13 us for
+// both, apart 5 us more; copied by the lane kernel as it writes the other rows
+// 16 us more).
 constexpr int kCopyGroup = 4 * kFaceThreads;  // rows per work-group
 template <typename T>
 __global__ void __launch_bounds__(kFaceThreads)
@@ -1329,7 +1330,7 @@ bool lane_plan(const Box &b, const Tiling &t, LaneOther other, TileArgs &a) {
   a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
   a.fbz_n = kLRows * kLRows;
   // byte offsets of the 27 quadrature points' viscosities and of 17 node rows
-  return 8 * 27 * b.nel < (1L << 32) && 8 * 3 * 17 * b.X < (1L << 32) && a.ntiles < (1L << 31);
+  return 8 * 27 * b.nel < (1L << 32) && lane_fits(b) && a.ntiles < (1L << 31);
 }
 
 // the same for an operator with face buffers of fb_doubles
@@ -1422,7 +1423,8 @@ int alloc_lane_data(ptmf_op_s *op) {
   const Box &b = op->box;
   const long na = b.mx + b.my + b.mz;
   const long planes = (long)((b.mx + kLT - 1) / kLT) * ((b.my + kLT - 1) / kLT) * b.Z;
-  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) + 64 * sizeof(unsigned) * planes));
+  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) +
+                                               64 * sizeof(unsigned) * planes));
   op->ax32 = (float *)(op->ax64 + na + 3);
   op->rect_bad = (int *)(op->ax32 + na);
   op->bcword = (unsigned *)(op->rect_bad + 1);

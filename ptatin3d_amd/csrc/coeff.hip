@@ -283,7 +283,8 @@ int launch_a11_diag(const ptmf_op_s *op, double *d) {
 int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, double nexp, double eta_min,
                     double eta_max, double *eta) {
   const TileArgs a = lane_args(op->box, 1024, 0.2);
-  PTMF_CHECK(a.ntiles < (1L << 31), PTMF_ERR_ARG, "powerlaw: mesh too large (%ld tiles)", a.ntiles);
+  PTMF_CHECK(a.ntiles < (1L << 31) && lane_fits(op->box), PTMF_ERR_ARG, "powerlaw: mesh too large (%ld tiles of a box %d wide)",
+             a.ntiles, a.mx);
   powerlaw_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(
       a, op->d64.coords, u, B, 0.5 * (1.0 / nexp - 1.0), eta_min, eta_max, eta);
   PTMF_HIP(hipGetLastError());

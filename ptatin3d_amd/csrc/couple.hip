@@ -224,7 +224,8 @@ int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
 
 int launch_a21(const ptmf_op_s *op, const double *u, double *yp) {
   const TileArgs a = lane_args(op->box, 1024, 0.2);
-  PTMF_CHECK(a.ntiles < (1L << 31), PTMF_ERR_ARG, "a21: mesh too large (%ld tiles)", a.ntiles);
+  PTMF_CHECK(a.ntiles < (1L << 31) && lane_fits(op->box), PTMF_ERR_ARG, "a21: mesh too large (%ld tiles of a box %d wide)",
+             a.ntiles, a.mx);
   a21_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, op->d64.coords, op->bcword, u, yp);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;

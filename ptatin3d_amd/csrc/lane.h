@@ -57,6 +57,9 @@ struct LaneBuf {
   }
 };
 
+// a tile's node rows lie within the 32-bit row offset
+inline bool lane_fits(const Box &b) { return 8 * 3 * (b.Y < kLRows ? b.Y : kLRows) * b.X < (1L << 32); }
+
 // Work decomposition of a lane kernel that runs `waves` waves at a time, each
 // spending `ends` of a layer's time on its first and last planes.
 inline TileArgs lane_args(const Box &b, long waves, double ends) {

@@ -1158,7 +1158,8 @@ int restrict_(ptmf_mg_s *mg, int l, const T *xf, T *yc, const uint8_t *bcn = nul
     PTMF_HIP(hipGetLastError());
     const ptmf_op_s *op = mg->lev[l - 1].op;
     if (bcn) PTMF_TRY(launch_bc_set<T>(op->bcidx, op->nbc, T(0), yc, mg->stream));
-    if (p) k_cheb_first<T><<<nblocks(3 * bc.nnodes), kBS, 0, mg->stream>>>(3 * bc.nnodes, yc, nullptr, nullptr, dinv, scale, p);
+    if (p)
+      k_cheb_first<T><<<nblocks(3 * bc.nnodes), kBS, 0, mg->stream>>>(3 * bc.nnodes, yc, nullptr, nullptr, dinv, scale, p);
   } else {
     PTMF_CHECK(3 * bf.nnodes < (1L << 31), PTMF_ERR_UNSUPPORTED, "restrict: level too large for 32-bit indices");
     const int bpp = (int)((bc.X * bc.Y + kBS - 1) / kBS);
@@ -2652,7 +2653,8 @@ int ptmf_op_project_points(ptmf_op op, long npts, const long *elem, const double
     if (hipGetLastError() != hipSuccess) st = ptmf_set_error(PTMF_ERR_DEVICE, "project_points: launch");
   }
   if (st == PTMF_OK) {
-    ptmf::k_q1_point_nodes<<<dim3((unsigned)((b.nnodes + ptmf::kBS - 1) / ptmf::kBS)), ptmf::kBS, 0, s>>>(b.mx, b.my, b.mz, sums, nodal);
+    ptmf::k_q1_point_nodes<<<dim3((unsigned)((b.nnodes + ptmf::kBS - 1) / ptmf::kBS)), ptmf::kBS, 0, s>>>(
+        b.mx, b.my, b.mz, sums, nodal);
     ptmf::k_q1_to_qp<<<dim3((unsigned)((b.nel + 63) / 64)), 64, 0, s>>>(b.mx, b.my, b.nel, nodal, eta);
     if (hipGetLastError() != hipSuccess) st = ptmf_set_error(PTMF_ERR_DEVICE, "project_points: launch");
   }
