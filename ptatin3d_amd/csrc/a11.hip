@@ -1678,6 +1678,7 @@ int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const 
   PTMF_CHECK(tl.TX * tl.TY <= kEPW && (2 * tl.TX + 1) * (2 * tl.TY + 1) <= kWinNodes && tl.ZC > 0,
              PTMF_ERR_ARG, "a11: invalid tiling %d x %d x %d", tl.TX, tl.TY, tl.ZC);
   PTMF_CHECK(fb != nullptr, PTMF_ERR_NOT_SETUP, "a11: face buffers not allocated");
+  std::lock_guard<std::mutex> lock(op->faces_mu);
   const int variant = noalloc && op->variant >= 2 ? 0 : op->variant;
   if (variant == 3) {
     // coloured scatter: no tiles, no face buffers
@@ -1749,6 +1750,7 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   PTMF_CHECK(tl.TX * tl.TY <= kEPW && (2 * tl.TX + 1) * (2 * tl.TY + 1) <= kWinNodes && tl.ZC > 0,
              PTMF_ERR_ARG, "stokes: invalid tiling %d x %d x %d", tl.TX, tl.TY, tl.ZC);
   PTMF_CHECK(op->faces != nullptr, PTMF_ERR_NOT_SETUP, "stokes: face buffers not allocated");
+  std::lock_guard<std::mutex> lock(op->faces_mu);
   const long nu = 3 * op->box.nnodes;
   // (by lane_plan's rule for the MatMult: at 24^3 both take 42 us, at 28^3 the
   // lane kernel 41 us and the tile kernel 62 us, and further apart above)

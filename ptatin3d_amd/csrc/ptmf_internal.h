@@ -130,6 +130,9 @@ struct ptmf_op_s {
   int et_tiling[2][3] = {{0, 0, 0}, {0, 0, 0}};
   void *faces = nullptr;          // tile face buffers (sized for FP64)
   long faces_doubles = 0;
+  // held while kernels that pass sums through `faces` are put on the stream, so
+  // that two threads' products do not come between one another
+  mutable std::mutex faces_mu;
   double *host_stage = nullptr;   // device staging for the host-array entry points
   double *host_stage2 = nullptr;
   double *points = nullptr;       // point projection: 18 sums per element, then the nodal field

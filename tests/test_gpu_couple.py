@@ -4,11 +4,14 @@ chunk and a shorter last one, one element, Dirichlet dofs inside the box, and
 a mesh far from the origin (the pressure basis' frame cancels).
 
 Tolerance: 1e-12 relative to the oracle, the bar of every FP64 operator here."""
+import threading
+
 import numpy as np
 import pytest
 
 from oracle import oracle as O
 from ptatin3d_amd import fields as F
+from ptatin3d_amd._lib import DeviceArray
 from ptatin3d_amd.operators import MatStokesMF
 
 from conftest import rel_inf
@@ -30,4 +33,28 @@ def test_couplings_parity(gpu, m):
     assert not y[bc.astype(bool)].any()
     assert rel_inf(A.a21_host(u), O.a21_matmult(*m, coords, bc, u)) <= 1e-12
     assert np.array_equal(y, A.a12_host(p))  # no atomics: repeats are bit-identical
+    A.destroy()
+
+
+def test_products_from_two_threads(gpu):
+    """One operator's MatMult and A12 share the face buffers: from two threads
+    each gives what it gives alone, to the bit."""
+    m = (40, 32, 32)
+    rng = np.random.default_rng(5)
+    E = m[0] * m[1] * m[2]
+    A = MatStokesMF(*m).setup(F.box_coords(*m), F.eta_loguniform(E, 0.5, 2.0, rng), F.dirichlet_all_faces(*m))
+    x = [DeviceArray.from_host(rng.uniform(-1, 1, n)) for n in (3 * F.nnodes(*m), 4 * E)]
+    mult = (A.mult, A.mult_a12)
+    alone = [DeviceArray(3 * F.nnodes(*m)) for _ in mult]
+    for f, v, y in zip(mult, x, alone):
+        f(v, y)
+    ys = [[DeviceArray(3 * F.nnodes(*m)) for _ in range(30)] for _ in mult]
+    threads = [threading.Thread(target=lambda f, v, out: [f(v, y) for y in out], args=a) for a in zip(mult, x, ys)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for want, out in zip(alone, ys):
+        w = want.download()
+        assert all(np.array_equal(w, y.download()) for y in out)
     A.destroy()
