@@ -1599,6 +1599,7 @@ int launch_face_copy(const ptmf_op_s *op, const TileArgs &a, const T *fbx, const
   // (whole rounds of the XCDs, so that each keeps its own tiles; a row copied twice is the same)
   const long copies = 8 * ((op->nbc + 8 * kCopyGroup - 1) / (8 * kCopyGroup)), groups = a.ntiles + copies;
   PTMF_CHECK(groups < (1L << 31), PTMF_ERR_ARG, "a11: mesh too large (%ld work-groups)", groups);
+  if (groups == 0) return PTMF_OK;  // (no faces, no Dirichlet dofs: the coloured variant on a free box)
   a11_face_copy_kernel<T><<<dim3((unsigned)groups), dim3(kFaceThreads), 0, op->stream>>>(
       a, fbx, fby, fbz, y, op->bcnode, op->bcidx, op->nbc, x);
   PTMF_HIP(hipGetLastError());
