@@ -171,8 +171,10 @@ int ptmf_op_create(int mx, int my, int mz, ptmf_op *out) {
     op->tiling = ptmf::choose_tiling(mx, my, mz);
     op->faces_doubles = std::max(ptmf::face_buffer_doubles(op->tiling.TX, op->tiling.TY, op->tiling.ZC,
                                                            op->tiling.ntiles),
-                                 std::max(ptmf::lane_face_doubles(b, op->tiling), ptmf::couple_face_doubles(b)));
+                                 ptmf::lane_face_doubles(b, op->tiling));
     st = ptmf_malloc(&op->faces, sizeof(double) * op->faces_doubles);
+    op->node_faces_doubles = ptmf::node_face_doubles(b);
+    alloc((void **)&op->node_faces, sizeof(double) * op->node_faces_doubles);
   }
   if (st != PTMF_OK) {
     ptmf_op tmp = op;
@@ -194,6 +196,7 @@ int ptmf_op_destroy(ptmf_op *pop) {
   (void)hipFree(op->bcnode);
   (void)hipFree(op->bcidx);
   (void)hipFree(op->faces);
+  (void)hipFree(op->node_faces);
   (void)hipFree(op->host_stage);
   (void)hipFree(op->host_stage2);
   (void)hipFree(op->pa64);

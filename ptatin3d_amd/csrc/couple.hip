@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(64)
 
 }  // namespace
 
-long couple_face_doubles(const Box &b) {
+long node_face_doubles(const Box &b) {
   const TileArgs a = lane_args(b, 1024, 0.45);
   return face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles);
 }

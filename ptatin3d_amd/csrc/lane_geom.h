@@ -212,14 +212,14 @@ __global__ void __launch_bounds__(kFaceThreads)
   face_sum<double, true>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
 }
 
-// the kernel and its faces, with face buffers fb
+// the kernel and its faces
 template <typename Op>
 int launch_node_lane(const ptmf_op_s *op, const TileArgs &a, const Op &nodal, double *y) {
-  PTMF_CHECK(face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= op->faces_doubles && a.ntiles < (1L << 31) &&
+  PTMF_CHECK(face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= op->node_faces_doubles && a.ntiles < (1L << 31) &&
                  lane_fits(op->box),
              PTMF_ERR_ARG, "mesh too large (%ld tiles of a box %d wide)", a.ntiles, a.mx);
-  std::lock_guard<std::mutex> lock(op->faces_mu);
-  double *fbx = (double *)op->faces, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
+  std::lock_guard<std::mutex> lock(op->node_faces_mu);
+  double *fbx = op->node_faces, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
   node_lane_kernel<Op><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, nodal, op->d64.coords, op->bcword, y,
                                                                               fbx, fby, fbz);
   PTMF_HIP(hipGetLastError());

@@ -133,6 +133,11 @@ struct ptmf_op_s {
   // held while kernels that pass sums through `faces` are put on the stream, so
   // that two threads' products do not come between one another
   mutable std::mutex faces_mu;
+  // face buffers of launch_node_lane, apart from `faces`: batches and captured
+  // V-cycles use those on their own, and A12 or the diagonal may be called beside them
+  double *node_faces = nullptr;
+  long node_faces_doubles = 0;
+  mutable std::mutex node_faces_mu;  // as faces_mu
   double *host_stage = nullptr;   // device staging for the host-array entry points
   double *host_stage2 = nullptr;
   double *points = nullptr;       // point projection: 18 sums per element, then the nodal field
@@ -194,7 +199,7 @@ int classify_mesh(ptmf_op_s *op);
 // does not run there); part of every operator's allocation, whatever its mesh,
 // so that new coordinates never move the buffers
 long lane_face_doubles(const Box &b, const Tiling &t);
-long couple_face_doubles(const Box &b);  // of launch_a12
+long node_face_doubles(const Box &b);  // of launch_a12 and launch_a11_diag
 // set-up: op->bcword from the operator's Dirichlet bits
 int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>

@@ -1,0 +1,82 @@
+"""Calls on one operator from two threads, one of them a batched MatMult or a
+V-cycle replayed as a graph, each with kernels that hand sums on through a
+buffer of the operator: every result is what the call gives alone, to the bit."""
+import threading
+
+import numpy as np
+import pytest
+
+from ptatin3d_amd import fields as F
+from ptatin3d_amd._lib import DeviceArray
+from ptatin3d_amd.multigrid import GMG, default_options
+from ptatin3d_amd.operators import BatchA11, MatStokesMF
+
+pytestmark = pytest.mark.gpu
+
+N = 40  # calls per thread
+
+
+def _together(calls):
+    """calls: name -> (function of an output array, its length; 0: checks itself)"""
+    alone, outs = {}, {}
+    for k, (f, n) in calls.items():
+        y, outs[k] = (DeviceArray(n), [DeviceArray(n) for _ in range(N)]) if n else (None, [None] * N)
+        f(y)
+        alone[k] = y.download() if n else None
+    threads = [threading.Thread(target=lambda f=f, ys=outs[k]: [f(y) for y in ys]) for k, (f, _) in calls.items()]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, ys in outs.items():
+        assert all(y is None or np.array_equal(alone[k], y.download()) for y in ys), k
+
+
+def _operator(m, rng):
+    return MatStokesMF(*m).setup(F.box_coords(*m), F.eta_loguniform(m[0] * m[1] * m[2], 0.5, 2.0, rng),
+                                 F.dirichlet_all_faces(*m))
+
+
+@pytest.mark.parametrize("m", [(24, 20, 18), (48, 48, 48)])  # column and tile kernel in the batch
+@pytest.mark.parametrize("other", ["a12", "diagonal"])
+def test_batch_beside_products_of_a_member(gpu, m, other):
+    rng = np.random.default_rng(5)
+    ops = [_operator(m, rng), _operator((9, 7, 5), rng)]
+    n = [3 * F.nnodes(*m), 3 * F.nnodes(9, 7, 5)]
+    x = [DeviceArray.from_host(rng.uniform(-1, 1, k)) for k in n]
+    p, rest = DeviceArray.from_host(rng.uniform(-1, 1, 4 * ops[0].nel)), DeviceArray(n[1])
+    B = BatchA11(ops)
+    _together({"batch": (lambda y: B.mult(x, [y, rest], 64), n[0]),
+               other: (lambda y: ops[0].mult_a12(p, y) if other == "a12" else ops[0].get_diagonal(y), n[0])})
+    B.destroy()
+    for A in ops:
+        A.destroy()
+
+
+@pytest.mark.parametrize("other", ["a12", "diagonal"])
+def test_replayed_vcycle_beside_products_of_its_operator(gpu, other):
+    m = (32, 32, 16)
+    rng = np.random.default_rng(6)
+    mg = GMG(*m, 3)
+    mg.set_coordinates(F.box_coords(*m))
+    mg.set_viscosity(2, F.eta_loguniform(m[0] * m[1] * m[2], 0.5, 2.0, rng))
+    mg.coarsen_viscosity("qp-arithmetic")
+    mg.set_dirichlet_all_faces()
+    mg.setup(default_options(smoother_precision=64))
+    A = MatStokesMF.borrow(mg.level_op_handle(2), *m)
+    n = 3 * F.nnodes(*m)
+    b, x = DeviceArray.from_host(rng.uniform(-1, 1, n)), DeviceArray(n)
+    p = DeviceArray.from_host(rng.uniform(-1, 1, 4 * A.nel))
+    for _ in range(3):
+        mg.vcycle(b, x)  # (captured before the threads start)
+    want = x.download()
+    same = []
+
+    def vcycle(_):
+        mg.vcycle(b, x)
+        same.append(np.array_equal(x.download(), want))
+
+    _together({"vcycle": (vcycle, 0),
+               other: (lambda y: A.mult_a12(p, y) if other == "a12" else A.get_diagonal(y), n)})
+    assert len(same) == N + 1 and all(same)
+    mg.destroy()
