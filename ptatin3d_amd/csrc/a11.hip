@@ -1666,20 +1666,23 @@ int launch_col(const ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T 
   return PTMF_OK;
 }
 
-// The MatMult's kernels with the face buffers at fb (the operator's own, or
-// the static scratch of the allocation-free entry point).  noalloc: nothing
-// is allocated on the way (the stored-geometry and coloured variants, which
-// build tables of their own or need no face buffers, give way to the z-march).
+// The MatMult's kernels with the operator's own face buffers or those at
+// `scratch`, of the allocation-free entry point.  With these nothing is
+// allocated on the way (the stored-geometry and coloured variants, which build
+// tables of their own or need no face buffers, give way to the z-march).
 template <typename T>
-int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T *x, T *y, T *fb, long fb_doubles,
-                       bool noalloc = false) {
+int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T *x, T *y, double *scratch = nullptr,
+                       long scratch_doubles = 0) {
   const OpData<T> &d = *(const OpData<T> *)(sizeof(T) == 8 ? (const void *)&op->d64
                                                            : (const void *)&op->d32);
   const Tiling &tl = op->tiling;
   PTMF_CHECK(tl.TX * tl.TY <= kEPW && (2 * tl.TX + 1) * (2 * tl.TY + 1) <= kWinNodes && tl.ZC > 0,
              PTMF_ERR_ARG, "a11: invalid tiling %d x %d x %d", tl.TX, tl.TY, tl.ZC);
-  PTMF_CHECK(fb != nullptr, PTMF_ERR_NOT_SETUP, "a11: face buffers not allocated");
   std::lock_guard<std::mutex> lock(op->faces_mu);
+  const bool noalloc = scratch != nullptr;
+  T *const fb = (T *)(noalloc ? scratch : op->faces);
+  const long fb_doubles = noalloc ? scratch_doubles : op->faces_doubles;
+  PTMF_CHECK(fb != nullptr, PTMF_ERR_NOT_SETUP, "a11: face buffers not allocated");
   const int variant = noalloc && op->variant >= 2 ? 0 : op->variant;
   if (variant == 3) {
     // coloured scatter: no tiles, no face buffers
@@ -1735,12 +1738,12 @@ int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const 
 
 template <typename T>
 int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, bool whole) {
-  return launch_a11_mult_fb<T>(op, whole ? kFinMult : kFinNone, nullptr, x, y, (T *)op->faces, op->faces_doubles);
+  return launch_a11_mult_fb<T>(op, whole ? kFinMult : kFinNone, nullptr, x, y);
 }
 
 template <typename T>
 int launch_a11_update(ptmf_op_s *op, const T *x, T *r, const RowUpdate<T> &up) {
-  return launch_a11_mult_fb<T>(op, kFinUpdate, &up, x, r, (T *)op->faces, op->faces_doubles);
+  return launch_a11_mult_fb<T>(op, kFinUpdate, &up, x, r);
 }
 
 template <typename T>
@@ -1750,8 +1753,8 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   const Tiling &tl = op->tiling;
   PTMF_CHECK(tl.TX * tl.TY <= kEPW && (2 * tl.TX + 1) * (2 * tl.TY + 1) <= kWinNodes && tl.ZC > 0,
              PTMF_ERR_ARG, "stokes: invalid tiling %d x %d x %d", tl.TX, tl.TY, tl.ZC);
-  PTMF_CHECK(op->faces != nullptr, PTMF_ERR_NOT_SETUP, "stokes: face buffers not allocated");
   std::lock_guard<std::mutex> lock(op->faces_mu);
+  PTMF_CHECK(op->faces != nullptr, PTMF_ERR_NOT_SETUP, "stokes: face buffers not allocated");
   const long nu = 3 * op->box.nnodes;
   // (by lane_plan's rule for the MatMult: at 24^3 both take 42 us, at 28^3 the
   // lane kernel 41 us and the tile kernel 62 us, and further apart above)
@@ -1791,6 +1794,7 @@ template int launch_a11_update<float>(ptmf_op_s *, const float *, float *, const
 // ---------------------------------------------------------------------------
 struct ptmf_batch_s {
   std::vector<ptmf_op> ops;
+  std::vector<ptmf_op> distinct;  // the same, for FacesLock
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // device data, rebuilt when the operators' tilings or buffers change
@@ -1965,6 +1969,9 @@ int ptmf_batch_create(const ptmf_op *ops, int nops, ptmf_batch *out) {
   for (int i = 0; i < nops; i++) PTMF_CHECK(ops[i], PTMF_ERR_ARG, "batch_create: null operator %d", i);
   ptmf_batch_s *b = new ptmf_batch_s;
   b->ops.assign(ops, ops + nops);
+  b->distinct = b->ops;
+  std::sort(b->distinct.begin(), b->distinct.end());
+  b->distinct.erase(std::unique(b->distinct.begin(), b->distinct.end()), b->distinct.end());
   hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&b->ev0);
   if (e == hipSuccess) e = hipEventCreate(&b->ev1);
@@ -1994,9 +2001,9 @@ int ptmf_batch_destroy(ptmf_batch *pb) {
   return PTMF_OK;
 }
 
-int ptmf_batch_mult(ptmf_batch b, int precision, const void *const *x, void *const *y) {
-  PTMF_CHECK(b && x && y, PTMF_ERR_ARG, "batch_mult: null argument");
-  PTMF_CHECK(precision == 64 || precision == 32, PTMF_ERR_UNSUPPORTED, "batch_mult: precision %d", precision);
+namespace {
+// the batched MatMult, with the FacesLock held
+int batch_mult_locked(ptmf_batch b, int precision, const void *const *x, void *const *y) {
   for (ptmf_op op : b->ops) PTMF_HIP(hipStreamSynchronize(op->stream));
   if (precision == 64) {
     PTMF_TRY(batch_prepare<double>(b, x, y));
@@ -2008,10 +2015,20 @@ int ptmf_batch_mult(ptmf_batch b, int precision, const void *const *x, void *con
   PTMF_HIP(hipStreamSynchronize(b->stream));
   return PTMF_OK;
 }
+}  // namespace
+
+int ptmf_batch_mult(ptmf_batch b, int precision, const void *const *x, void *const *y) {
+  PTMF_CHECK(b && x && y, PTMF_ERR_ARG, "batch_mult: null argument");
+  PTMF_CHECK(precision == 64 || precision == 32, PTMF_ERR_UNSUPPORTED, "batch_mult: precision %d", precision);
+  ptmf::FacesLock lock(b->distinct);
+  return batch_mult_locked(b, precision, x, y);
+}
 
 int ptmf_batch_time(ptmf_batch b, int precision, const void *const *x, void *const *y, int reps, double *ms) {
   PTMF_CHECK(b && x && y && reps > 0 && ms, PTMF_ERR_ARG, "batch_time: bad arguments");
-  PTMF_TRY(ptmf_batch_mult(b, precision, x, y));  // prepares and warms up
+  PTMF_CHECK(precision == 64 || precision == 32, PTMF_ERR_UNSUPPORTED, "batch_mult: precision %d", precision);
+  ptmf::FacesLock lock(b->distinct);
+  PTMF_TRY(batch_mult_locked(b, precision, x, y));  // prepares and warms up
   PTMF_HIP(hipEventRecord(b->ev0, b->stream));
   for (int r = 0; r < reps; r++) {
     if (precision == 64) PTMF_TRY(batch_launch<double>(b));
@@ -2086,5 +2103,5 @@ extern "C" int ptmf_a11_mult_noalloc(ptmf_op op, const double *x, double *y) {
              need, kScratchDoubles);
   double *fb = nullptr;
   PTMF_TRY(scratch_address(dev, &fb));
-  return ptmf::launch_a11_mult_fb<double>(op, ptmf::kFinMult, nullptr, x, y, fb, kScratchDoubles, true);
+  return ptmf::launch_a11_mult_fb<double>(op, ptmf::kFinMult, nullptr, x, y, fb, kScratchDoubles);
 }

@@ -228,6 +228,7 @@ int ptmf_op_set_tiling(ptmf_op op, int TX, int TY, int ZC) {
   const Box &b = op->box;
   ptmf::Tiling t = ptmf::make_tiling(b.mx, b.my, b.mz, TX, TY < b.my ? TY : TY, ZC);
   const long need = ptmf::face_buffer_doubles(TX, TY, ZC, t.ntiles);
+  std::lock_guard<std::mutex> lock(op->faces_mu);
   PTMF_HIP(hipStreamSynchronize(op->stream));
   if (need > op->faces_doubles) {
     void *p = nullptr;

@@ -1004,6 +1004,7 @@ struct KrylovSpace {
 struct ptmf_mg_s {
   int L = 0;
   ptmf::MGLevel lev[16];
+  std::vector<ptmf_op> ops;  // of the levels, for FacesLock
   ptmf_mg_options opt;
   bool is_setup = false;
   hipStream_t stream = nullptr;
@@ -1903,6 +1904,8 @@ int ptmf_mg_create(int mx, int my, int mz, int nlevels, ptmf_mg *out) {
     st = ptmf_op_create(L.mx, L.my, L.mz, &L.op);
     if (st != PTMF_OK) break;
     ptmf::set_op_stream(L.op, mg->stream);
+    mg->ops.push_back(L.op);
+    std::sort(mg->ops.begin(), mg->ops.end());
     L.n = 3 * L.op->box.nnodes;
     const size_t b8 = sizeof(double) * L.n, b4 = sizeof(float) * L.n;
     void **a8[] = {(void **)&L.diag, (void **)&L.dinv64, (void **)&L.b64, (void **)&L.x64,
@@ -2278,6 +2281,8 @@ int ptmf_mg_vcycle(ptmf_mg mg, const double *b, double *x) {
     if (c.ex && c.b == b && c.x == x) v = &c;
   if (!v) PTMF_TRY(ptmf::capture_vcycle(mg, b, x, &v));
   v->used = ++mg->vtick;
+  // (the replay is a launch of every level operator's kernels)
+  ptmf::FacesLock lock(mg->ops);
   PTMF_HIP(hipGraphLaunch(v->ex, mg->stream));
   return PTMF_OK;
 }

@@ -11,6 +11,7 @@
 #include <stddef.h>
 
 #include <mutex>
+#include <vector>
 
 #include "ptmf.h"
 
@@ -130,8 +131,8 @@ struct ptmf_op_s {
   int et_tiling[2][3] = {{0, 0, 0}, {0, 0, 0}};
   void *faces = nullptr;          // tile face buffers (sized for FP64)
   long faces_doubles = 0;
-  // held while kernels that pass sums through `faces` are put on the stream, so
-  // that two threads' products do not come between one another
+  // held while `faces` is used: by a launch until its kernels are on the
+  // operator's stream, by a batch, which has its own, until they are done
   mutable std::mutex faces_mu;
   // face buffers of launch_node_lane, apart from `faces`: batches and captured
   // V-cycles use those on their own, and A12 or the diagonal may be called beside them
@@ -143,6 +144,25 @@ struct ptmf_op_s {
   double *points = nullptr;       // point projection: 18 sums per element, then the nodal field
   std::mutex points_mu;
 };
+
+namespace ptmf {
+// the operators' faces_mu, all held; ops sorted and without repetition, so that
+// no two holders wait for each other
+class FacesLock {
+ public:
+  explicit FacesLock(const std::vector<ptmf_op> &ops) : ops_(ops) {
+    for (ptmf_op op : ops_) op->faces_mu.lock();
+  }
+  ~FacesLock() {
+    for (ptmf_op op : ops_) op->faces_mu.unlock();
+  }
+  FacesLock(const FacesLock &) = delete;
+  FacesLock &operator=(const FacesLock &) = delete;
+
+ private:
+  const std::vector<ptmf_op> &ops_;
+};
+}  // namespace ptmf
 
 // Error plumbing: every entry point returns a ptmf status code.
 int ptmf_set_error(int code, const char *fmt, ...);

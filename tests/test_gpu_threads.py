@@ -37,8 +37,12 @@ def _operator(m, rng):
                                  F.dirichlet_all_faces(*m))
 
 
+def _product(A, other, x, p):
+    return {"a12": lambda y: A.mult_a12(p, y), "diagonal": A.get_diagonal, "matmult": lambda y: A.mult(x, y)}[other]
+
+
 @pytest.mark.parametrize("m", [(24, 20, 18), (48, 48, 48)])  # column and tile kernel in the batch
-@pytest.mark.parametrize("other", ["a12", "diagonal"])
+@pytest.mark.parametrize("other", ["a12", "diagonal", "matmult"])
 def test_batch_beside_products_of_a_member(gpu, m, other):
     rng = np.random.default_rng(5)
     ops = [_operator(m, rng), _operator((9, 7, 5), rng)]
@@ -47,13 +51,13 @@ def test_batch_beside_products_of_a_member(gpu, m, other):
     p, rest = DeviceArray.from_host(rng.uniform(-1, 1, 4 * ops[0].nel)), DeviceArray(n[1])
     B = BatchA11(ops)
     _together({"batch": (lambda y: B.mult(x, [y, rest], 64), n[0]),
-               other: (lambda y: ops[0].mult_a12(p, y) if other == "a12" else ops[0].get_diagonal(y), n[0])})
+               other: (_product(ops[0], other, x[0], p), n[0])})
     B.destroy()
     for A in ops:
         A.destroy()
 
 
-@pytest.mark.parametrize("other", ["a12", "diagonal"])
+@pytest.mark.parametrize("other", ["a12", "diagonal", "matmult"])
 def test_replayed_vcycle_beside_products_of_its_operator(gpu, other):
     m = (32, 32, 16)
     rng = np.random.default_rng(6)
@@ -77,6 +81,27 @@ def test_replayed_vcycle_beside_products_of_its_operator(gpu, other):
         same.append(np.array_equal(x.download(), want))
 
     _together({"vcycle": (vcycle, 0),
-               other: (lambda y: A.mult_a12(p, y) if other == "a12" else A.get_diagonal(y), n)})
+               other: (_product(A, other, b, p), n)})
     assert len(same) == N + 1 and all(same)
     mg.destroy()
+
+
+def test_tiling_changed_beside_products(gpu):
+    """A tiling with larger face buffers moves them: never under a product that
+    uses them.  (Sums in another order: 1e-12, the bar of every tiling here.)"""
+    m = (48, 48, 48)
+    rng = np.random.default_rng(7)
+    A = _operator(m, rng)
+    x = DeviceArray.from_host(rng.uniform(-1, 1, 3 * F.nnodes(*m)))
+    want, ys = DeviceArray(x.n), [DeviceArray(x.n) for _ in range(N)]
+    A.mult(x, want)
+    threads = [threading.Thread(target=lambda: [A.mult(x, y) for y in ys]),
+               threading.Thread(target=lambda: [A.set_tiling(*t) for t in ((4, 5, 2), (7, 3, 1), (1, 1, 1)) * 3])]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    w = want.download()
+    for y in ys:
+        assert np.abs(y.download() - w).max() <= 1e-12 * np.abs(w).max()
+    A.destroy()
