@@ -1353,7 +1353,7 @@ bool col_box(const ptmf_op_s *op, long fb_doubles) {
 }
 
 // Is the mesh rectilinear?  Axis lines of the three directions first (mid
-// nodes halfway between their neighbours, ax = 2 / h per element), then every
+// nodes halfway between their neighbours, 2 m / h per element), then every
 // node against the lines.  "Equal" is to 4 units of rounding of the largest
 // coordinate of the direction: what a mesh generator's own rounding leaves,
 // and what the general kernel's interpolation of the coordinates rounds off
@@ -1364,7 +1364,12 @@ __global__ void __launch_bounds__(256)
   __shared__ double red[256];
   const int m[3] = {mx, my, mz};
   const long stride[3] = {3, 3 * X, 3 * XY};
-  if (threadIdx.x == 0) *bad = 0;
+  const double unit = ldexp(1.0, ilogb(xc[6] - xc[0]));  // m of a11_lane.h
+  if (threadIdx.x == 0) {
+    *bad = 0;
+    a64[mx + my + mz] = unit;
+    a32[mx + my + mz] = (float)unit;
+  }
   for (int d = 0, first = 0; d < 3; first += m[d], d++) {
     double big = 0.0;
     for (int i = threadIdx.x; i <= 2 * m[d]; i += 256) big = fmax(big, fabs(xc[stride[d] * i + d]));
@@ -1381,8 +1386,8 @@ __global__ void __launch_bounds__(256)
       const double *x = xc + stride[d] * (2 * e) + d;
       const double x0 = x[0], x1 = x[stride[d]], x2 = x[2 * stride[d]], h = x2 - x0;
       if (!(fabs(x1 - 0.5 * (x0 + x2)) <= t) || !(fabs(h) > 64.0 * t) || !isfinite(h)) *bad = 1;
-      a64[first + e] = 2.0 / h;
-      a32[first + e] = (float)(2.0 / h);
+      a64[first + e] = 2.0 * unit / h;
+      a32[first + e] = (float)(2.0 * unit / h);
     }
   }
 }
@@ -1418,15 +1423,15 @@ __global__ void __launch_bounds__(64)
 }  // namespace
 
 int alloc_lane_data(ptmf_op_s *op) {
-  // one allocation: 2 / h in FP64 (and three tolerances) and FP32, the
+  // one allocation: 2 m / h and m in FP64 (and three tolerances) and in FP32, the
   // classification's flag, the Dirichlet words
   const Box &b = op->box;
   const long na = b.mx + b.my + b.mz;
   const long planes = (long)((b.mx + kLT - 1) / kLT) * ((b.my + kLT - 1) / kLT) * b.Z;
-  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 3) + sizeof(float) * na + sizeof(int) +
+  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 4) + sizeof(float) * (na + 1) + sizeof(int) +
                                                64 * sizeof(unsigned) * planes));
-  op->ax32 = (float *)(op->ax64 + na + 3);
-  op->rect_bad = (int *)(op->ax32 + na);
+  op->ax32 = (float *)(op->ax64 + na + 4);
+  op->rect_bad = (int *)(op->ax32 + na + 1);
   op->bcword = (unsigned *)(op->rect_bad + 1);
   return PTMF_OK;
 }
@@ -1446,11 +1451,11 @@ int classify_mesh(ptmf_op_s *op) {
   const long na = b.mx + b.my + b.mz;
   op->rect = 0;
   rect_axes_kernel<<<1, 256, 0, op->stream>>>(b.mx, b.my, b.mz, b.X, b.X * b.Y, op->d64.coords, op->ax64, op->ax32,
-                                              op->ax64 + na, op->rect_bad);
+                                              op->ax64 + na + 1, op->rect_bad);
   long nb = (b.nnodes + 255) / 256;
   if (nb > 8192) nb = 8192;
   rect_check_kernel<<<dim3((unsigned)nb), 256, 0, op->stream>>>(b.nnodes, (int)b.X, (int)b.Y, op->d64.coords,
-                                                               op->ax64 + na, op->rect_bad);
+                                                               op->ax64 + na + 1, op->rect_bad);
   PTMF_HIP(hipGetLastError());
   int bad = 1;
   PTMF_HIP(hipMemcpyAsync(&bad, op->rect_bad, sizeof(int), hipMemcpyDeviceToHost, op->stream));

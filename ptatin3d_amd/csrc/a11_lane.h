@@ -27,12 +27,18 @@
 // AGPRs (96 x 96 x 48 MatMult 171 us, the tile kernel's 485 us; 28^3 41 and 62
 // us).
 
-// per-lane constants of a rectilinear element: the collocation coefficients
-// of the two in-plane directions scaled by 2 / h, and the Jacobian determinant
+// Per-lane constants of a rectilinear element: the collocation coefficients of
+// the in-plane directions scaled by 2 m / h, and the weights.  m is a power of two
+// of about an element's length, one for the mesh: derivatives in space times m
+// are about those in the element, and the weights hold the lengths they lack, so
+// that no product on the way is larger than the terms of the result but for the
+// ratios of the lengths (with weights of det J, eta h^3 overflows FP32 at 3e39: SI
+// units, 100 km elements).  A power of two changes no rounding.
 template <typename T>
 struct LaneGeom {
-  T cx[3], cy[3];  // (5/2, 10/3, 5/6) s times 2 / hx, 2 / hy
-  T az, vol;       // 2 / hz, hx hy hz / 8
+  T cx[3], cy[3];  // (5/2, 10/3, 5/6) s times 2 m / hx, 2 m / hy
+  T az;            // 2 m / hz
+  T vol;           // det J / m^2
 };
 
 // collocated derivative at point a of a line with the scaled coefficients
@@ -63,8 +69,8 @@ __device__ __forceinline__ void ldot_t(int a, const T c[3], T v, T &y0, T &y1, T
 // Stress at the plane's points and its transposed derivatives:
 // out[k][l][3j+i] += the plane's part of (A11_e u)(node (i, j, k), component l)
 // kP: of the saddle-point product.  The pressure basis of a rectilinear element
-// is {1, xi / 2, eta / 2, zeta / 2}; pc: its coefficients, the last three times
-// s / 2; acc += the plane's part of (A21_e u), the last three over s / 2.
+// is {1, xi / 2, eta / 2, zeta / 2}; pc: its coefficients times m, the last three
+// times s / 2 too; acc += the plane's part of (A21_e u), over the same factors.
 template <typename T, int c, bool kP>
 __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const LaneGeom<T> &g, const T et[9],
                                             T out[3][3][9], const T pc[4], T acc[4]) {
@@ -79,7 +85,7 @@ __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const La
 #pragma unroll
     for (int a = 0; a < 3; a++) {
       const int p = 3 * b + a;
-      T G[3][3];  // G[k][l] = d u_l / d x_k
+      T G[3][3];  // G[k][l] = m d u_l / d x_k
 #pragma unroll
       for (int l = 0; l < 3; l++) {
         G[0][l] = ldot<T>(a, g.cx, U[l][3 * b], U[l][3 * b + 1], U[l][3 * b + 2]);
@@ -124,8 +130,8 @@ __device__ __forceinline__ void lane_stress(const T U[3][9], T Z[3][9], const La
     lane_field_t<T, c>(W[l], Z[l], d0, d1, d2, out[0][l], out[1][l], out[2][l]);
 }
 
-// Dirichlet rows are left as the element sums.  bcw: lane_bc_word's.  ax: 2 / h
-// of the mx element columns, the my rows and the mz layers.
+// Dirichlet rows are left as the element sums.  bcw: lane_bc_word's.  ax: 2 m / h
+// of the mx element columns, the my rows and the mz layers, then m.
 // kP: the saddle-point product with p, yp the pressures (4 per element).
 template <typename T, bool kP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
@@ -137,12 +143,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
   __shared__ T sm[5 * kLSlot];
   const LaneTile q = lane_tile(a, (unsigned)xcd_tile(blockIdx.x, a.ntiles));
   const TileBox &tb = q.tb;
-  // 2 / hz of the chunk's layers, one per lane
+  // 2 m / hz of the chunk's layers, one per lane
   const T szs = ax[a.mx + a.my + tb.z0 + min(q.lane, tb.nzt - 1)];
   auto plane = [&](int P) { return LaneBuf<T>(u + 3 * lane_node(a, tb, P)); };
 
   LaneGeom<T> g;
-  const T sx = ax[tb.x0 + q.cx], sy = ax[a.mx + tb.y0 + q.cy];
+  const T sx = ax[tb.x0 + q.cx], sy = ax[a.mx + tb.y0 + q.cy], m = ax[a.mx + a.my + a.mz];
   g.cx[0] = (T)(2.5 * kS) * sx;
   g.cx[1] = (T)(10.0 / 3.0 * kS) * sx;
   g.cx[2] = (T)(5.0 / 6.0 * kS) * sx;
@@ -190,7 +196,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     const LaneBuf<T> eta_k(eta + tb.x0 + (long)a.mx * (tb.y0 + (long)a.my * ek));
     const T sz = __shfl(szs, kz);
     g.az = sz;
-    g.vol = q.live ? T(1) / (sx * sy * sz) : T(0);
+    g.vol = q.live ? m * (T(1) / (sx * sy * sz)) : T(0);
 #pragma unroll
     for (int l = 0; l < 3; l++)
 #pragma unroll
@@ -225,7 +231,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     lane_rows_store<T, 0>(r, q, s3, s4);
     if constexpr (kP) {
 #pragma unroll
-      for (int i = 1; i < 4; i++) pc[i] *= (T)(0.5 * kS);
+      for (int i = 0; i < 4; i++) pc[i] *= i ? (T)(0.5 * kS) * m : m;
     }
     lane_stress<T, 0, kP>(U, Z, g, et, out, pc, acc);
     lane_pin<T>(out);
@@ -251,9 +257,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(
     lane_pin<T>(out);
     if constexpr (kP) {
       if (q.live) {
-        yp[e4] = acc[0];
 #pragma unroll
-        for (int i = 1; i < 4; i++) yp[e4 + i] = (T)(0.5 * kS) * acc[i];
+        for (int i = 0; i < 4; i++) yp[e4 + i] = (i ? (T)(0.5 * kS) * m : m) * acc[i];
       }
     }
     __syncthreads();

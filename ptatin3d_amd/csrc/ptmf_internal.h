@@ -107,8 +107,8 @@ struct ptmf_op_s {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   ptmf::Tiling tiling;
   int tiling_default = 1;         // the tiling is choose_tiling's own
-  // rectilinear mesh (element faces normal to the axes): 2 / h per element of
-  // the mx columns, my rows and mz layers
+  // rectilinear mesh (element faces normal to the axes): 2 m / h per element of
+  // the mx columns, my rows and mz layers, then m (a11_lane.h)
   int rect = 0;
   double *ax64 = nullptr;         // holds ax32, rect_bad and bcword too
   float *ax32 = nullptr;

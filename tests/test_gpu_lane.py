@@ -181,3 +181,18 @@ def test_lane_saddle_point_in_fp32_preconditioner(gpu):
         its.append(out[2])
         mg.destroy()
     assert abs(its[0] - its[1]) <= 1, its
+
+
+@pytest.mark.parametrize("m", [(64, 47, 20), (31, 33, 64)])
+def test_lane_fp32_in_si_units(gpu, m):
+    """Elements of 100 km x 90 km x 10 km, viscosities about 1e25 Pa s and
+    velocities about 1e-9 m/s: eta h^3 is past the largest FP32 number, every
+    term of the result far from it."""
+    coords, eta, bc, u = _case(m, 17)
+    coords = (coords.reshape(-1, 3) * np.array([1e5, 9e4, 1e4]) * m).reshape(-1)
+    eta, u = 1e25 * eta, 1e-9 * u
+    A = MatA11MF(*m).setup(coords, eta, bc)
+    y = A.mult_host(u, precision=32)
+    assert np.isfinite(y).all()
+    assert rel_inf(y, O.a11_matmult(*m, coords, eta, bc, u)) <= 1e-5
+    A.destroy()
