@@ -152,6 +152,15 @@ int ptmf_op_project_points(ptmf_op op, long npts, const long *elem, const double
  * coloring, stokes_operators_cuda.cu:337-397, plays this role there). */
 int ptmf_op_set_tiling(ptmf_op op, int TX, int TY, int ZC);
 int ptmf_op_get_tiling(ptmf_op op, int *TX, int *TY, int *ZC);
+/* The tiling of a new operator.  Set, with kernel variant 0 and one tile per
+ * work-group, it also leaves the choice of the element kernel to the operator
+ * (on rectilinear meshes and on small boxes others are faster than the tiled
+ * z-march); any other tiling asks for the z-march. */
+int ptmf_op_default_tiling(ptmf_op op, int *TX, int *TY, int *ZC);
+/* 1 if the element faces of the operator's mesh are normal to the axes (to
+ * rounding), 0 if not or before its coordinates are set.  The fastest kernel
+ * and tiling of a box depend on it. */
+int ptmf_op_rectilinear(ptmf_op op, int *rectilinear);
 /* MatMult kernel variant: 0 = z-march; 1 = z-march with the next layer's
  * loads issued one stage ahead (software pipelined; equal to 0 to rounding);
  * 2 = stored quadrature-point geometry (partial assembly: 9 values per

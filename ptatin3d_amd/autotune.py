@@ -13,8 +13,9 @@ TX*TY, 2 TX*TY or 4 TX*TY elements per work-group).  `tune(op, ...)` times
 the candidate (shape, variant, tiles per work-group) triples with HIP events on the operator's own stream, in the precision the
 operator will be applied in, and installs the fastest; `tune_hierarchy`
 does that for every level of a multigrid hierarchy in the V-cycle's
-precision.  Choices are cached per (box, precision, candidate set) in memory
-and in a JSON file (PTMF_AUTOTUNE_CACHE, default
+precision.  The operator's default tiling, which leaves the choice of kernel to
+the operator, is always among the candidates.  Choices are cached per (box,
+precision, candidate set, rectilinear mesh or not) in memory and in a JSON file (PTMF_AUTOTUNE_CACHE, default
 ~/.cache/ptmf/autotune.json), so later processes reuse them.
 """
 from __future__ import annotations
@@ -27,6 +28,9 @@ import numpy as np
 
 from ._lib import DeviceArray
 
+# of a cached choice's key, to be changed with the kernels it was made among: a
+# choice made before they could run a default tiling would keep them out
+_KERNELS = "tile-lane-column"
 _CACHE: dict[str, tuple[tuple[int, int, int], int, int]] = {}
 _LOADED = False
 VARIANTS = (0, 1)
@@ -40,7 +44,7 @@ def cache_path() -> str:
 
 
 def _key(mx, my, mz, precision, variants, max_shapes) -> str:
-    return f"{mx}x{my}x{mz}:fp{precision}:v{'-'.join(map(str, variants))}:s{max_shapes}"
+    return f"{_KERNELS}:{mx}x{my}x{mz}:fp{precision}:v{'-'.join(map(str, variants))}:s{max_shapes}"
 
 
 def _load() -> None:
@@ -98,7 +102,8 @@ def tune(op, precision: int = 64, reps: int = 10, max_shapes: int = 8, verbose: 
     Returns ((TX, TY, ZC), variant, tiles) and the sorted timings (empty when
     the choice came from the cache)."""
     _load()
-    key = _key(op.mx, op.my, op.mz, precision, variants, max_shapes) + f":w{'-'.join(map(str, wg_tiles))}"
+    key = (_key(op.mx, op.my, op.mz, precision, variants, max_shapes) + f":w{'-'.join(map(str, wg_tiles))}"
+           + (":rectilinear" if op.rectilinear else ":general"))
     if key in _CACHE:
         t, v, w = _CACHE[key]
         op.set_tiling(*t)
@@ -111,9 +116,7 @@ def tune(op, precision: int = 64, reps: int = 10, max_shapes: int = 8, verbose: 
     y = DeviceArray(n, dt)
     results = []
     base_tiling = op.get_tiling()
-    # the operator's own tiling first: the default one leaves the choice of
-    # kernel to the operator (one lane per element on large rectilinear meshes)
-    cands = [(tuple(base_tiling), 0, 1)] if 0 in variants and 1 in wg_tiles else []
+    cands = [(tuple(op.default_tiling()), 0, 1)] if 0 in variants and 1 in wg_tiles else []
     for v in variants:
         if v == COLOUR:
             cands.append((tuple(base_tiling), v, 1))

@@ -280,6 +280,21 @@ int ptmf_op_get_tiling(ptmf_op op, int *TX, int *TY, int *ZC) {
   return PTMF_OK;
 }
 
+int ptmf_op_default_tiling(ptmf_op op, int *TX, int *TY, int *ZC) {
+  PTMF_CHECK(op, PTMF_ERR_ARG, "default_tiling: null op");
+  const ptmf::Tiling t = ptmf::choose_tiling(op->box.mx, op->box.my, op->box.mz);
+  if (TX) *TX = t.TX;
+  if (TY) *TY = t.TY;
+  if (ZC) *ZC = t.ZC;
+  return PTMF_OK;
+}
+
+int ptmf_op_rectilinear(ptmf_op op, int *rectilinear) {
+  PTMF_CHECK(op && rectilinear, PTMF_ERR_ARG, "rectilinear: null argument");
+  *rectilinear = op->rect;
+  return PTMF_OK;
+}
+
 int ptmf_op_state(ptmf_op op, unsigned long *state) {
   PTMF_CHECK(op && state, PTMF_ERR_ARG, "op_state: null");
   *state = op->state;

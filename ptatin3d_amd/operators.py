@@ -79,6 +79,20 @@ class MatA11MF:
         call("ptmf_op_get_tiling", self.handle, C.byref(a), C.byref(b), C.byref(c))
         return a.value, b.value, c.value
 
+    def default_tiling(self) -> tuple[int, int, int]:
+        """The tiling of a new operator: with variant 0 and one tile per group it
+        leaves the choice of the element kernel to the operator."""
+        a, b, c = C.c_int(), C.c_int(), C.c_int()
+        call("ptmf_op_default_tiling", self.handle, C.byref(a), C.byref(b), C.byref(c))
+        return a.value, b.value, c.value
+
+    @property
+    def rectilinear(self) -> bool:
+        """Whether the mesh's element faces are normal to the axes (to rounding)."""
+        v = C.c_int()
+        call("ptmf_op_rectilinear", self.handle, C.byref(v))
+        return bool(v.value)
+
     def set_kernel_variant(self, variant: int) -> None:
         """0: z-march; 1: z-march with next-layer loads issued one stage ahead;
         2: stored quadrature-point geometry; 3: coloured scatter (no tiles)."""

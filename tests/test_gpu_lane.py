@@ -196,3 +196,18 @@ def test_lane_fp32_in_si_units(gpu, m):
     assert np.isfinite(y).all()
     assert rel_inf(y, O.a11_matmult(*m, coords, eta, bc, u)) <= 1e-5
     A.destroy()
+
+
+def test_kind_of_mesh_and_default_tiling(gpu):
+    m = (12, 10, 9)
+    coords, eta, bc, _ = _case(m, 19)
+    A = MatA11MF(*m)
+    default = A.get_tiling()
+    assert not A.rectilinear
+    A.setup(coords, eta, bc)
+    assert A.rectilinear
+    A.set_tiling(2, 2, 2)
+    assert A.default_tiling() == default != A.get_tiling()
+    A.set_coordinates(F.perturb_interior(coords, *m, 0.1, np.random.default_rng(1)))
+    assert not A.rectilinear
+    A.destroy()

@@ -136,3 +136,68 @@ def test_autotune_cache_persists(tmp_path, monkeypatch):
     autotune._load()
     assert autotune._CACHE[k] == ((4, 5, 2), 3, 2)
     assert autotune._key(64, 64, 64, 64, (0, 1, 3), 4) not in autotune._CACHE
+
+
+class _TimedOperator:
+    """What the autotuner sees of an operator, with made-up times: a default
+    tiling is fast where the operator may choose its kernel, on rectilinear meshes."""
+
+    mx, my, mz, nnodes = 20, 18, 16, 1
+    default = (7, 3, 3)  # (its chunk is not among the autotuner's own)
+
+    def __init__(self, rectilinear):
+        self.rectilinear, self.tiling, self.variant, self.tiles, self.timed = rectilinear, self.default, 0, 1, []
+
+    def get_tiling(self):
+        return self.tiling
+
+    def default_tiling(self):
+        return self.default
+
+    def set_tiling(self, *t):
+        self.tiling = tuple(t)
+
+    def set_kernel_variant(self, v):
+        self.variant = v
+
+    def set_tiles_per_group(self, w):
+        self.tiles = w
+
+    def time_mult(self, x, y, reps):
+        self.timed.append((self.tiling, self.variant, self.tiles))
+        if self.tiling == self.default and self.variant == 0 and self.tiles == 1:
+            return 1.0 if self.rectilinear else 9.0
+        return 2.0 + 0.01 * sum(self.tiling) + 0.1 * self.variant + 0.1 * self.tiles
+
+
+def test_autotune_knows_the_kind_of_mesh(tmp_path, monkeypatch):
+    """A box tuned on one kind of mesh is tuned anew on the other; a choice filed
+    before the operator chose its own kernel is not taken; and the default
+    tiling is tried whatever tiling the operator has."""
+    class Array:
+        def __init__(self, n, dt=None):
+            pass
+
+        from_host = classmethod(lambda cls, a: cls(a.size))
+
+        def free(self):
+            pass
+
+    path = tmp_path / "tune.json"
+    path.write_text(json.dumps({f"20x18x16:fp{p}:v0-1:s2:w1-2-4": [[4, 5, 2], 1, 1] for p in (32, 64)}))
+    monkeypatch.setenv("PTMF_AUTOTUNE_CACHE", str(path))
+    monkeypatch.setattr(autotune, "DeviceArray", Array)
+    monkeypatch.setattr(autotune, "_CACHE", {})
+    monkeypatch.setattr(autotune, "_LOADED", False)
+    general = _TimedOperator(False)
+    first, times = autotune.tune(general, max_shapes=2)
+    assert times and first[0] != general.default
+    box = _TimedOperator(True)
+    assert autotune.tune(box, max_shapes=2)[0] == (box.default, 0, 1)
+    assert (box.tiling, box.variant, box.tiles) == (box.default, 0, 1)
+    # both from the cache now, each its own
+    for op, want in ((_TimedOperator(False), first), (_TimedOperator(True), (box.default, 0, 1))):
+        assert autotune.tune(op, max_shapes=2) == (want, []) and not op.timed
+    other = _TimedOperator(True)
+    other.set_tiling(4, 5, 2)
+    assert autotune.tune(other, precision=32, max_shapes=2)[0] == (box.default, 0, 1)
