@@ -282,11 +282,19 @@ int launch_a11_diag(const ptmf_op_s *op, double *d) {
 
 int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, double nexp, double eta_min,
                     double eta_max, double *eta) {
-  const TileArgs a = lane_args(op->box, 1024, 0.2);
-  PTMF_CHECK(a.ntiles < (1L << 31) && lane_fits(op->box), PTMF_ERR_ARG, "powerlaw: mesh too large (%ld tiles of a box %d wide)",
-             a.ntiles, a.mx);
-  powerlaw_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(
-      a, op->d64.coords, u, B, 0.5 * (1.0 / nexp - 1.0), eta_min, eta_max, eta);
+  const double half_exp = 0.5 * (1.0 / nexp - 1.0);
+  double layers;
+  const TileArgs a = lane_args(op->box, 1024, 0.2, &layers);
+  // In microseconds, 27 lanes per element take 14.5 and 1.33 per thousand elements,
+  // the lane kernel 8 and 27.3 per layer that a wave marches through, however
+  // much of its 8 x 8 tile the box fills.  Measured, 27 lanes and one lane:
+  // 8^3 17 and 40, 24^3 33 and 41, 32^3 57 and 43, 48^3 160 and 77; 256 x 1 x 256
+  // 100 and 234, 512 x 2 x 64 101 and 127, 17 x 17 x 300 129 and 101.
+  const bool lane = 8.0 + 27.3 * layers < 14.5 + 1.33e-3 * (double)op->box.nel;
+  if (!lane || a.ntiles >= (1L << 31) || !lane_fits(op->box))
+    return launch_powerlaw_elems(op, u, B, half_exp, eta_min, eta_max, eta);
+  powerlaw_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, op->d64.coords, u, B, half_exp,
+                                                                             eta_min, eta_max, eta);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

@@ -1,5 +1,5 @@
-// elem.hip -- per-element Q2 kernels: the A11 diagonal and its l1 row sums, the
-// Schur blocks and the power-law viscosity.
+// elem.hip -- per-element Q2 kernels: the l1 row sums of A11, the Schur blocks,
+// and the power-law viscosity of boxes too small or too thin for the lane kernel.
 //
 // Layout of a work-group: 64 lanes, 2 elements, lanes 32h + q (q < 27) own
 // quadrature point q of element h, lanes 32h + n (n < 27) own node n in the
@@ -47,6 +47,25 @@ __device__ __forceinline__ void lane_tab_node(int n, LaneTab &T) {
       T.B[d][a] = pick3(nd[d], kB[a][0], kB[a][1], kB[a][2]);
       T.D[d][a] = pick3(nd[d], kD[a][0], kD[a][1], kD[a][2]);
     }
+}
+
+// the rows of a lane that owns quadrature point (a, b, c): B[d][n] = kB[q_d][n]
+__device__ __forceinline__ void lane_tab_qp(int q, LaneTab &T) {
+  const int qd[3] = {q % 3, (q / 3) % 3, q / 9};
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+      T.B[d][r] = pick3(qd[d], kB[0][r], kB[1][r], kB[2][r]);
+      T.D[d][r] = pick3(qd[d], kD[0][r], kD[1][r], kD[2][r]);
+    }
+}
+
+// reference gradient of the (node, point) pair whose other index is (x, y, z)
+__device__ __forceinline__ void tab_grad(const LaneTab &T, int x, int y, int z, double gr[3]) {
+  gr[0] = T.D[0][x] * T.B[1][y] * T.B[2][z];
+  gr[1] = T.B[0][x] * T.D[1][y] * T.B[2][z];
+  gr[2] = T.B[0][x] * T.B[1][y] * T.D[2][z];
 }
 
 __device__ void qp_geometry(const double (*xe)[3], int q, QpGeom &g) {
@@ -378,6 +397,53 @@ __global__ void __launch_bounds__(64)
   }
 }
 
+// ---- power-law viscosity at the quadrature points (see coeff.hip): 27 lanes per
+// element, one point each.  A wave is done after one element's work, where a lane
+// kernel marches through a layer of 64 however few of them there are.  Positions
+// from the element's first node: no digits are lost to its distance from the origin.
+__global__ void __launch_bounds__(64)
+    powerlaw_elem_kernel(int mx, int my, long nel, long X, long XY, const double *__restrict__ xc,
+                         const double *__restrict__ u, const double *__restrict__ B, double half_exp, double eta_min,
+                         double eta_max, double *__restrict__ eta) {
+  __shared__ double sx[kEPB][27][3];
+  __shared__ double su[kEPB][27][3];
+  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
+  long e = (long)blockIdx.x * kEPB + h;
+  const bool live = e < nel;
+  if (!live) e = nel - 1;
+  if (t < 27) {
+    const long first = elem_node(mx, my, X, XY, e, 0), node = first + t % 3 + X * (t / 3 % 3) + XY * (t / 9);
+    for (int d = 0; d < 3; d++) {
+      sx[h][t][d] = xc[3 * node + d] - xc[3 * first + d];
+      su[h][t][d] = u[3 * node + d];
+    }
+  }
+  __syncthreads();
+  if (t < 27 && live) {
+    QpGeom g;
+    qp_geometry(sx[h], t, g);
+    double L[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // L[l][k] = d u_l / d x_k
+    LaneTab T;
+    lane_tab_qp(t, T);
+#pragma unroll
+    for (int n = 0; n < 27; n++) {
+      double gr[3], gp[3];
+      tab_grad(T, n % 3, (n / 3) % 3, n / 9, gr);
+      for (int k = 0; k < 3; k++) gp[k] = g.G[k][0] * gr[0] + g.G[k][1] * gr[1] + g.G[k][2] * gr[2];
+      for (int l = 0; l < 3; l++)
+        for (int k = 0; k < 3; k++) L[l][k] += su[h][n][l] * gp[k];
+    }
+    double e2 = 0.0;
+    for (int l = 0; l < 3; l++)
+      for (int k = 0; k < 3; k++) {
+        const double dlk = 0.5 * (L[l][k] + L[k][l]);
+        e2 += 0.5 * dlk * dlk;
+      }
+    if (e2 < 1.0e-34) e2 = 1.0e-34;  // e_II >= 1e-17
+    eta[27 * e + t] = fmin(fmax(B[27 * e + t] * pow(e2, half_exp), eta_min), eta_max);
+  }
+}
+
 // yp[4e+i] = sum_j Minv_e[i][j] rp[4e+j] (+ beta yp when beta != 0)
 __global__ void schur_apply_kernel(long nel, const double *__restrict__ Minv, const double *__restrict__ rp,
                                    double *__restrict__ yp) {
@@ -429,6 +495,16 @@ int launch_schur_bdb(const ptmf_op_s *op, const double *dg, double *Minv, int *s
   schur_bdb_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.nel, b.X, b.X * b.Y,
                                                                       op->d64.coords, op->bcnode, dg, Minv,
                                                                       singular);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
+int launch_powerlaw_elems(const ptmf_op_s *op, const double *u, const double *B, double half_exp, double eta_min,
+                          double eta_max, double *eta) {
+  const Box &b = op->box;
+  const long nblk = (b.nel + kEPB - 1) / kEPB;
+  powerlaw_elem_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(
+      b.mx, b.my, b.nel, b.X, b.X * b.Y, op->d64.coords, u, B, half_exp, eta_min, eta_max, eta);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

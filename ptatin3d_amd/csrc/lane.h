@@ -61,8 +61,9 @@ struct LaneBuf {
 inline bool lane_fits(const Box &b) { return 8 * 3 * (b.Y < kLRows ? b.Y : kLRows) * b.X < (1L << 32); }
 
 // Work decomposition of a lane kernel that runs `waves` waves at a time, each
-// spending `ends` of a layer's time on its first and last planes.
-inline TileArgs lane_args(const Box &b, long waves, double ends) {
+// spending `ends` of a layer's time on its first and last planes.  layers: the
+// time it takes, in those of a layer.
+inline TileArgs lane_args(const Box &b, long waves, double ends, double *layers = nullptr) {
   TileArgs a;
   a.mx = b.mx; a.my = b.my; a.mz = b.mz;
   a.X = b.X; a.XY = b.X * b.Y; a.nel = b.nel;
@@ -81,6 +82,7 @@ inline TileArgs lane_args(const Box &b, long waves, double ends) {
   }
   a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
   a.fbz_n = kLRows * kLRows;
+  if (layers) *layers = best;
   return a;
 }
 

@@ -242,6 +242,9 @@ int batch_apply(ptmf_batch_s *b, int precision, const void *const *xs, void *con
                 const int *active = nullptr);
 int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, double nexp, double eta_min,
                     double eta_max, double *eta);
+// the same with 27 lanes per element; half_exp = (1/n - 1) / 2
+int launch_powerlaw_elems(const ptmf_op_s *op, const double *u, const double *B, double half_exp, double eta_min,
+                          double eta_max, double *eta);
 int launch_a11_diag(const ptmf_op_s *op, double *d);
 int launch_a11_l1(const ptmf_op_s *op, double *d);
 int launch_schur_blocks(const ptmf_op_s *op, double *Me, double *Minv);

@@ -64,3 +64,19 @@ def test_viscosity_copies(gpu, m, tiling):
         assert np.array_equal(ops[0].mult_host(u, precision=prec), ops[1].mult_host(u, precision=prec))
     for A in ops:
         A.destroy()
+
+
+@pytest.mark.parametrize("m", [(1, 1, 7), (2, 3, 300), (70, 1, 60), (1, 64, 65), (26, 25, 31), (30, 25, 31)])
+def test_powerlaw_of_thin_and_small_boxes(gpu, m):
+    """27 lanes per element where a lane per element would leave most of a wave
+    idle, and the first boxes past that: against the oracle, in place too."""
+    rng = np.random.default_rng(14)
+    coords = F.perturb_interior(F.box_coords(*m), *m, 0.1, rng) + 5.0
+    E = m[0] * m[1] * m[2]
+    u, B = rng.uniform(-1.0, 1.0, 3 * F.nnodes(*m)), 10.0 ** rng.uniform(-2.0, 2.0, 27 * E)
+    A = MatA11MF(*m).setup(coords, np.ones(27 * E), F.dirichlet_all_faces(*m))
+    ref = O.powerlaw_eta(*m, coords, u, B, 2.5, 1e-3, 1e3)
+    du, dB = DeviceArray.from_host(u), DeviceArray.from_host(B)
+    A.powerlaw_viscosity(du, dB, 2.5, 1e-3, 1e3, dB)
+    assert rel_inf(dB.download(), ref) <= 1e-12
+    A.destroy()
