@@ -4,6 +4,8 @@
 // Both need no division: with A = det(J) J^-1 the adjugate, w det(J) d_k N_n is
 // w sum_j A[k][j] (dN_n / d xi_j) and w det(J) div u is w sum_jk A[k][j] (du_k /
 // d xi_j).
+#include <algorithm>
+
 #include "lane_geom.h"
 
 namespace ptmf {
@@ -223,9 +225,15 @@ int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
 }
 
 int launch_a21(const ptmf_op_s *op, const double *u, double *yp) {
-  const TileArgs a = lane_args(op->box, 1024, 0.2);
-  PTMF_CHECK(a.ntiles < (1L << 31) && lane_fits(op->box), PTMF_ERR_ARG, "a21: mesh too large (%ld tiles of a box %d wide)",
-             a.ntiles, a.mx);
+  double layers;
+  const TileArgs a = lane_args(op->box, 1024, 0.2, &layers);
+  // In microseconds, 27 lanes per element take 17.5, or 11 and 2.85 per thousand
+  // elements, the lane kernel 9 and 14.2 per layer that a wave marches through,
+  // however much of its 8 x 8 tile the box fills.  Measured, 27 lanes and one lane:
+  // 8^3 18 and 26, 16^3 23 and 26, 20^3 34 and 26, 48^3 324 and 47; 2 x 2 x 20000
+  // 238 and 287, 256 x 1 x 256 196 and 127.
+  const bool lane = 9.0 + 14.2 * layers < std::max(17.5, 11.0 + 2.85e-3 * (double)op->box.nel);
+  if (!lane || a.ntiles >= (1L << 31) || !lane_fits(op->box)) return launch_a21_elems(op, u, yp);
   a21_lane_kernel<<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, op->d64.coords, op->bcword, u, yp);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;

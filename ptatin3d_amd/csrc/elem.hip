@@ -1,5 +1,6 @@
 // elem.hip -- per-element Q2 kernels: the l1 row sums of A11, the Schur blocks,
-// and the power-law viscosity of boxes too small or too thin for the lane kernel.
+// and, for boxes too small or too thin for the lane kernels, A21 and the power-law
+// viscosity.
 //
 // Layout of a work-group: 64 lanes, 2 elements, lanes 32h + q (q < 27) own
 // quadrature point q of element h, lanes 32h + n (n < 27) own node n in the
@@ -218,6 +219,55 @@ __global__ void __launch_bounds__(128)
     }
     const long node = elem_node(mx, my, X, XY, e, a);
     atomicAdd(&l1[3 * node + c], sum);
+  }
+}
+
+// ---- B^T u (see couple.hip), 27 lanes per element, one point each, and a sum
+// over them.  Positions from the element's first node, as in powerlaw_elem_kernel.
+__global__ void __launch_bounds__(64)
+    a21_elem_kernel(int mx, int my, long nel, long X, long XY, const double *__restrict__ xc,
+                    const uint8_t *__restrict__ bcn, const double *__restrict__ u, double *__restrict__ yp) {
+  __shared__ double sx[kEPB][27][3];
+  __shared__ double su[kEPB][27][3];
+  __shared__ double sr[kEPB][32][4];
+  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
+  long e = (long)blockIdx.x * kEPB + h;
+  const bool live = e < nel;
+  if (!live) e = nel - 1;
+  if (t < 27) {
+    const long first = elem_node(mx, my, X, XY, e, 0), node = first + t % 3 + X * (t / 3 % 3) + XY * (t / 9);
+    const unsigned m = bcn[node];
+    for (int d = 0; d < 3; d++) {
+      sx[h][t][d] = xc[3 * node + d] - xc[3 * first + d];
+      su[h][t][d] = ((m >> d) & 1u) ? 0.0 : u[3 * node + d];
+    }
+  }
+  __syncthreads();
+  double val[4] = {0, 0, 0, 0};
+  if (t < 27) {
+    QpGeom g;
+    qp_geometry(sx[h], t, g);
+    double Np[4];
+    p1_basis(sx[h], g.xq, Np);
+    double div = 0.0;
+    LaneTab T;
+    lane_tab_qp(t, T);
+#pragma unroll
+    for (int n = 0; n < 27; n++) {
+      double gr[3];
+      tab_grad(T, n % 3, (n / 3) % 3, n / 9, gr);
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+        div += su[h][n][k] * (g.G[k][0] * gr[0] + g.G[k][1] * gr[1] + g.G[k][2] * gr[2]);
+    }
+    for (int i = 0; i < 4; i++) val[i] = -g.wdet * Np[i] * div;
+  }
+  for (int i = 0; i < 4; i++) sr[h][t][i] = val[i];
+  __syncthreads();
+  if (t < 4 && live) {
+    double s = 0.0;
+    for (int q = 0; q < 27; q++) s += sr[h][q][t];
+    yp[4 * e + t] = s;
   }
 }
 
@@ -495,6 +545,15 @@ int launch_schur_bdb(const ptmf_op_s *op, const double *dg, double *Minv, int *s
   schur_bdb_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.nel, b.X, b.X * b.Y,
                                                                       op->d64.coords, op->bcnode, dg, Minv,
                                                                       singular);
+  PTMF_HIP(hipGetLastError());
+  return PTMF_OK;
+}
+
+int launch_a21_elems(const ptmf_op_s *op, const double *u, double *yp) {
+  const Box &b = op->box;
+  const long nblk = (b.nel + kEPB - 1) / kEPB;
+  a21_elem_kernel<<<dim3((unsigned)nblk), dim3(64), 0, op->stream>>>(b.mx, b.my, b.nel, b.X, b.X * b.Y, op->d64.coords,
+                                                                     op->bcnode, u, yp);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
 }

@@ -265,4 +265,5 @@ long mf_factor_doubles(const MFFactor *m);
 double mf_setup_ms(const MFFactor *m);
 int mf_depths(const MFFactor *m);
 int launch_a21(const ptmf_op_s *op, const double *u, double *yp);
+int launch_a21_elems(const ptmf_op_s *op, const double *u, double *yp);  // with 27 lanes per element
 }  // namespace ptmf
