@@ -219,9 +219,14 @@ long node_face_doubles(const Box &b) {
 }
 
 int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
+  // Measured, 27 lanes and one lane: one element 21 and 30 us, 2^3 63 and 31, 48^3
+  // 252 and 58; 1 x 1 x 5000 36 and 91, 2 x 2 x 20000 197 and 302, 256 x 1 x 256
+  // 154 and 136.
+  TileArgs a;
+  if (!node_lane_plan(op->box, 14.3, 6.4, 1.7, 9.0, 14.6, a)) return launch_a12_elems(op, p, yu);
   A12Op b{};
   b.p = p;
-  return launch_node_lane(op, lane_args(op->box, 1024, 0.45), b, yu);
+  return launch_node_lane(op, a, b, yu);
 }
 
 int launch_a21(const ptmf_op_s *op, const double *u, double *yp) {

@@ -1,6 +1,6 @@
 // elem.hip -- per-element Q2 kernels: the l1 row sums of A11, the Schur blocks,
-// and, for boxes too small or too thin for the lane kernels, A21 and the power-law
-// viscosity.
+// and, for boxes too small or too thin for the lane kernels, A12, A21, the A11
+// diagonal and the power-law viscosity.
 //
 // Layout of a work-group: 64 lanes, 2 elements, lanes 32h + q (q < 27) own
 // quadrature point q of element h, lanes 32h + n (n < 27) own node n in the
@@ -219,6 +219,84 @@ __global__ void __launch_bounds__(128)
     }
     const long node = elem_node(mx, my, X, XY, e, a);
     atomicAdd(&l1[3 * node + c], sum);
+  }
+}
+
+// ---- Nodal sums with 27 lanes per element, one parity class of elements per
+// launch: no two of a class share a node, so their sums go into the zeroed vector
+// with plain read-add-write.  op.point: the scalar s of the lane's quadrature
+// point; op.add: the point's part of a node from s and the node's gradient there.
+// Positions from the element's first node, as in powerlaw_elem_kernel.
+struct DiagElems {  // diag(A11), see coeff.hip
+  const double *eta;
+  long nel;
+  __device__ __forceinline__ double point(const double (*)[3], const QpGeom &g, long e, int q) const {
+    return g.wdet * eta[(long)q * nel + e];
+  }
+  __device__ __forceinline__ void add(double s, const double gp[3], double acc[3]) const {
+    const double g2 = gp[0] * gp[0] + gp[1] * gp[1] + gp[2] * gp[2];
+#pragma unroll
+    for (int c = 0; c < 3; c++) acc[c] += s * (g2 + gp[c] * gp[c]);
+  }
+};
+
+struct A12Elems {  // B p, see couple.hip
+  const double *p;
+  __device__ __forceinline__ double point(const double (*xe)[3], const QpGeom &g, long e, int) const {
+    double Np[4];
+    p1_basis(xe, g.xq, Np);
+    return -g.wdet * (Np[0] * p[4 * e] + Np[1] * p[4 * e + 1] + Np[2] * p[4 * e + 2] + Np[3] * p[4 * e + 3]);
+  }
+  __device__ __forceinline__ void add(double s, const double gp[3], double acc[3]) const {
+#pragma unroll
+    for (int c = 0; c < 3; c++) acc[c] += s * gp[c];
+  }
+};
+
+template <typename Op>
+__global__ void __launch_bounds__(64)
+    node_elem_kernel(int mx, int my, int mz, long X, long XY, int color, const double *__restrict__ xc, Op op,
+                     double *__restrict__ y) {
+  __shared__ double sx[kEPB][27][3];
+  __shared__ double sG[kEPB][27][10];
+  const int h = threadIdx.x >> 5, t = threadIdx.x & 31;
+  bool live;
+  const long e = class_element(mx, my, mz, color, (long)blockIdx.x * kEPB + h, live);
+  const long first = elem_node(mx, my, X, XY, e, 0), node = first + t % 3 + X * (t / 3 % 3) + XY * (t / 9);
+  if (t < 27)
+    for (int d = 0; d < 3; d++) sx[h][t][d] = xc[3 * node + d] - xc[3 * first + d];
+  __syncthreads();
+  if (t < 27) {
+    QpGeom g;
+    qp_geometry(sx[h], t, g);
+    for (int r = 0; r < 3; r++)
+      for (int s = 0; s < 3; s++) sG[h][t][3 * r + s] = g.G[r][s];
+    sG[h][t][9] = op.point(sx[h], g, e, t);
+  }
+  __syncthreads();
+  if (t < 27 && live) {
+    LaneTab T;
+    lane_tab_node(t, T);
+    double acc[3] = {0, 0, 0};
+    // one quadrature plane per trip (the unrolled 9 points keep their
+    // geometry loads in registers; all 27 at once would spill)
+#pragma unroll 1
+    for (int qc = 0; qc < 3; qc++) {
+      const double bk = pick3(qc, T.B[2][0], T.B[2][1], T.B[2][2]), dk = pick3(qc, T.D[2][0], T.D[2][1], T.D[2][2]);
+#pragma unroll
+      for (int qb = 0; qb < 3; qb++)
+#pragma unroll
+        for (int qa = 0; qa < 3; qa++) {
+          const double *G = sG[h][qa + 3 * qb + 9 * qc];
+          const double gr[3] = {T.D[0][qa] * T.B[1][qb] * bk, T.B[0][qa] * T.D[1][qb] * bk,
+                                T.B[0][qa] * T.B[1][qb] * dk};
+          double gp[3];
+#pragma unroll
+          for (int k = 0; k < 3; k++) gp[k] = G[3 * k] * gr[0] + G[3 * k + 1] * gr[1] + G[3 * k + 2] * gr[2];
+          op.add(G[9], gp, acc);
+        }
+    }
+    for (int c = 0; c < 3; c++) y[3 * node + c] += acc[c];
   }
 }
 
@@ -547,6 +625,29 @@ int launch_schur_bdb(const ptmf_op_s *op, const double *dg, double *Minv, int *s
                                                                       singular);
   PTMF_HIP(hipGetLastError());
   return PTMF_OK;
+}
+
+// y = sums of `nodal`, its Dirichlet rows bc
+template <typename Op>
+int launch_node_elems(const ptmf_op_s *op, const Op &nodal, double bc, double *y) {
+  const Box &b = op->box;
+  PTMF_TRY(launch_fill<double>(y, 0.0, 3 * b.nnodes, op->stream));
+  for (int color = 0; color < 8; color++) {
+    const long n = class_count(b, color);
+    if (n == 0) continue;
+    node_elem_kernel<Op><<<dim3((unsigned)((n + kEPB - 1) / kEPB)), dim3(64), 0, op->stream>>>(
+        b.mx, b.my, b.mz, b.X, b.X * b.Y, color, op->d64.coords, nodal, y);
+    PTMF_HIP(hipGetLastError());
+  }
+  return launch_bc_set<double>(op->bcidx, op->nbc, bc, y, op->stream);
+}
+
+int launch_a11_diag_elems(const ptmf_op_s *op, double *d) {
+  return launch_node_elems(op, DiagElems{op->d64.eta, op->box.nel}, 1.0, d);
+}
+
+int launch_a12_elems(const ptmf_op_s *op, const double *p, double *yu) {
+  return launch_node_elems(op, A12Elems{p}, 0.0, yu);
 }
 
 int launch_a21_elems(const ptmf_op_s *op, const double *u, double *yp) {

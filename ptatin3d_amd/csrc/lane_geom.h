@@ -212,12 +212,26 @@ __global__ void __launch_bounds__(kFaceThreads)
   face_sum<double, true>(a, xcd_tile(blockIdx.x, a.ntiles), fbx, fby, fbz, y, bcn);
 }
 
+// The decomposition of box b; false where 27 lanes per element are faster: in
+// microseconds these take `few` and `launch` for each parity class that has
+// elements and `elem` per thousand elements, the lane kernel `first` and `layer`
+// per layer that a wave marches through, however much of its 8 x 8 tile the box
+// fills.  (They also have the boxes past the lane kernel's 32-bit offsets.)
+inline bool node_lane_plan(const Box &b, double few, double launch, double elem, double first, double layer,
+                           TileArgs &a) {
+  double layers;
+  a = lane_args(b, 1024, 0.45, &layers);
+  int classes = 0;
+  for (int color = 0; color < 8; color++) classes += class_count(b, color) > 0;
+  return first + layer * layers < few + launch * classes + 1e-3 * elem * (double)b.nel && a.ntiles < (1L << 31) &&
+         lane_fits(b);
+}
+
 // the kernel and its faces
 template <typename Op>
 int launch_node_lane(const ptmf_op_s *op, const TileArgs &a, const Op &nodal, double *y) {
-  PTMF_CHECK(face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= op->node_faces_doubles && a.ntiles < (1L << 31) &&
-                 lane_fits(op->box),
-             PTMF_ERR_ARG, "mesh too large (%ld tiles of a box %d wide)", a.ntiles, a.mx);
+  PTMF_CHECK(face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) <= op->node_faces_doubles, PTMF_ERR_NOT_SETUP,
+             "face buffers not allocated");
   std::lock_guard<std::mutex> lock(op->node_faces_mu);
   double *fbx = op->node_faces, *fby = fbx + 3 * a.fbx_n * a.ntiles, *fbz = fby + 3 * a.fby_n * a.ntiles;
   node_lane_kernel<Op><<<dim3((unsigned)a.ntiles), dim3(64), 0, op->stream>>>(a, nodal, op->d64.coords, op->bcword, y,

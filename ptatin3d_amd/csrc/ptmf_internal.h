@@ -246,11 +246,13 @@ int launch_powerlaw(const ptmf_op_s *op, const double *u, const double *B, doubl
 int launch_powerlaw_elems(const ptmf_op_s *op, const double *u, const double *B, double half_exp, double eta_min,
                           double eta_max, double *eta);
 int launch_a11_diag(const ptmf_op_s *op, double *d);
+int launch_a11_diag_elems(const ptmf_op_s *op, double *d);  // with 27 lanes per element
 int launch_a11_l1(const ptmf_op_s *op, double *d);
 int launch_schur_blocks(const ptmf_op_s *op, double *Me, double *Minv);
 int launch_schur_apply(const ptmf_op_s *op, const double *Minv, const double *rp, double *yp);
 // yu = B p, Dirichlet rows 0
 int launch_a12(const ptmf_op_s *op, const double *p, double *yu);
+int launch_a12_elems(const ptmf_op_s *op, const double *p, double *yu);  // with 27 lanes per element
 // Multifrontal Cholesky of a level operator given as its 125-point 3x3-block
 // stencil S (device, S[((o*9)+3r+c)*N + m] = A(3m+r, 3(m+off_o)+c), SPD with
 // unit Dirichlet rows), nested-dissection ordered (coarse.hip).  mf_solve is
