@@ -1,8 +1,9 @@
 """The diagonal of A11 and the power-law viscosity with one lane per element, at
 the sizes where they can go wrong: partial 8 x 8 tiles in either direction, one
-to many layers a chunk and a shorter last one, one element, Dirichlet dofs
-inside the box, sheared elements (the diagonal's mixed products are large) and
-velocities at rest.
+to many chunks of a layer (test_gpu_lane_layers.py has chunks of several), one
+element, Dirichlet dofs inside the box, sheared elements (the diagonal's mixed
+products are large) and velocities at rest; the power law of the smaller ones
+takes 27 lanes per element.
 
 Tolerance: 1e-12 relative to the oracle, the FP64 bar of both operators."""
 import numpy as np

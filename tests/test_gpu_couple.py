@@ -1,7 +1,8 @@
 """The couplings A12 and A21 with one lane per element, at the sizes where they
-can go wrong: partial 8 x 8 tiles in either direction, one to many layers a
-chunk and a shorter last one, one element, Dirichlet dofs inside the box, and
-a mesh far from the origin (the pressure basis' frame cancels).
+can go wrong: partial 8 x 8 tiles in either direction, one to many chunks of a
+layer (test_gpu_lane_layers.py has chunks of several), one element, Dirichlet
+dofs inside the box, and a mesh far from the origin (the pressure basis' frame
+cancels); A21 of the smaller ones takes 27 lanes per element.
 
 Tolerance: 1e-12 relative to the oracle, the bar of every FP64 operator here."""
 import threading
@@ -37,8 +38,8 @@ def test_couplings_parity(gpu, m):
 
 
 def test_products_from_two_threads(gpu):
-    """One operator's MatMult and A12 share the face buffers: from two threads
-    each gives what it gives alone, to the bit."""
+    """One operator's MatMult and A12 hand sums on through buffers of the operator:
+    from two threads each gives what it gives alone, to the bit."""
     m = (40, 32, 32)
     rng = np.random.default_rng(5)
     E = m[0] * m[1] * m[2]
