@@ -161,6 +161,11 @@ int ptmf_op_default_tiling(ptmf_op op, int *TX, int *TY, int *ZC);
  * rounding), 0 if not or before its coordinates are set.  The fastest kernel
  * and tiling of a box depend on it. */
 int ptmf_op_rectilinear(ptmf_op op, int *rectilinear);
+/* The element kernel of ptmf_a11_mult (precision 64) or ptmf_a11_mult_f32 (32)
+ * with the operator's present mesh, tiling, variant and tiles per work-group:
+ * 0..3 the variants of ptmf_op_set_kernel_variant; 4 one lane per element, 5 one
+ * lane per node column of an element (both the operator's own choice). */
+int ptmf_op_mult_kernel(ptmf_op op, int precision, int *kernel);
 /* MatMult kernel variant: 0 = z-march; 1 = z-march with the next layer's
  * loads issued one stage ahead (software pipelined; equal to 0 to rounding);
  * 2 = stored quadrature-point geometry (partial assembly: 9 values per

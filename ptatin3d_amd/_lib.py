@@ -59,6 +59,7 @@ SIGNATURES: dict[str, tuple] = {
     "ptmf_op_get_tiles_per_group": (_I, [_P, C.POINTER(_I)]),
     "ptmf_op_get_tiling": (_I, [_P, C.POINTER(_I), C.POINTER(_I), C.POINTER(_I)]),
     "ptmf_op_default_tiling": (_I, [_P, C.POINTER(_I), C.POINTER(_I), C.POINTER(_I)]),
+    "ptmf_op_mult_kernel": (_I, [_P, _I, C.POINTER(_I)]),
     "ptmf_op_rectilinear": (_I, [_P, C.POINTER(_I)]),
     "ptmf_a11_spmv": (_I, [_P, _P, _P]),
     "ptmf_a11_spmv_host": (_I, [_P, _P, _P]),

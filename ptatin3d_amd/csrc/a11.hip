@@ -1671,6 +1671,18 @@ int launch_col(const ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const T 
   return PTMF_OK;
 }
 
+// The element kernel of a MatMult with face buffers of fb_doubles; la: the
+// decomposition of the lane kernel.  noalloc: as in launch_a11_mult_fb.
+enum MultKernel { kMultTile, kMultPipelined, kMultStored, kMultColoured, kMultLane, kMultColumn };  // (variants first)
+
+template <typename T>
+MultKernel mult_kernel(const ptmf_op_s *op, long fb_doubles, bool noalloc, TileArgs &la) {
+  if (op->variant != 0 && !(noalloc && op->variant >= 2)) return (MultKernel)op->variant;
+  const bool col = col_box(op, fb_doubles);
+  if (lane_tiles<T>(op, fb_doubles, col ? kOtherCol : kOtherTile, la)) return kMultLane;
+  return col ? kMultColumn : kMultTile;
+}
+
 // The MatMult's kernels with the operator's own face buffers or those at
 // `scratch`, of the allocation-free entry point.  With these nothing is
 // allocated on the way (the stored-geometry and coloured variants, which build
@@ -1688,8 +1700,9 @@ int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const 
   T *const fb = (T *)(noalloc ? scratch : op->faces);
   const long fb_doubles = noalloc ? scratch_doubles : op->faces_doubles;
   PTMF_CHECK(fb != nullptr, PTMF_ERR_NOT_SETUP, "a11: face buffers not allocated");
-  const int variant = noalloc && op->variant >= 2 ? 0 : op->variant;
-  if (variant == 3) {
+  TileArgs la;
+  const MultKernel kernel = mult_kernel<T>(op, fb_doubles, noalloc, la);
+  if (kernel == kMultColoured) {
     // coloured scatter: no tiles, no face buffers
     const Box &b = op->box;
     PTMF_TRY(launch_fill<T>(y, T(0), 3 * b.nnodes, op->stream));
@@ -1706,15 +1719,12 @@ int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const 
     one.ntiles = 0;
     return finish_rows<T>(op, one, fin, up, nullptr, nullptr, nullptr, x, y);
   }
-  TileArgs la;
-  const LaneOther other = col_box(op, fb_doubles) ? kOtherCol : kOtherTile;
-  if (variant == 0 && lane_tiles<T>(op, fb_doubles, other, la))
-    return launch_lane<T, false>(op, la, fin, up, x, nullptr, y, nullptr, fb);
-  if (variant == 0 && col_box(op, fb_doubles)) return launch_col<T>(op, fin, up, x, y, fb);
+  if (kernel == kMultLane) return launch_lane<T, false>(op, la, fin, up, x, nullptr, y, nullptr, fb);
+  if (kernel == kMultColumn) return launch_col<T>(op, fin, up, x, y, fb);
   const TileArgs a = tile_args(op);
   const long ntiles = tl.ntiles;
   T *fbx = fb, *fby = fbx + 3 * a.fbx_n * ntiles, *fbz = fby + 3 * a.fby_n * ntiles;
-  if (variant == 2) {
+  if (kernel == kMultStored) {
     PTMF_TRY(ensure_pa<T>(op));
     const T *pa = sizeof(T) == 8 ? (const T *)op->pa64 : (const T *)op->pa32;
     a11_tile_pa_kernel<T, true><<<dim3((unsigned)ntiles), dim3(64), 0, op->stream>>>(
@@ -1724,7 +1734,7 @@ int launch_a11_mult_fb(ptmf_op_s *op, Finish fin, const RowUpdate<T> *up, const 
     const T *et = sizeof(T) == 8 ? (const T *)op->et64 : (const T *)op->et32;
     const int kw = op->wg_tiles;
     const long nwg = (ntiles + kw - 1) / kw;
-    if (variant == 1)
+    if (kernel == kMultPipelined)
       a11_tile_pf_kernel<T, true><<<dim3((unsigned)ntiles), dim3(64), 0, op->stream>>>(
           a, d.coords, et, op->bcnode, x, y, fbx, fby, fbz);
     else if (kw == 2)
@@ -1782,6 +1792,12 @@ int launch_stokes_mult(ptmf_op_s *op, const double *x, double *y) { return launc
 // FP32 saddle-point MatMult (FP32 coordinates, viscosity and accumulation):
 // the preconditioner's A12 product of an FP32 velocity V-cycle.
 int launch_stokes_mult_f32(ptmf_op_s *op, const float *x, float *y) { return launch_stokes_mult_t<float>(op, x, y); }
+
+int a11_mult_kernel(const ptmf_op_s *op, int precision) {
+  TileArgs la;
+  return precision == 64 ? mult_kernel<double>(op, op->faces_doubles, false, la)
+                         : mult_kernel<float>(op, op->faces_doubles, false, la);
+}
 
 int prepare_eta_tiled(ptmf_op_s *op) { return ensure_eta_tiled<double>(op); }
 

@@ -295,6 +295,13 @@ int ptmf_op_rectilinear(ptmf_op op, int *rectilinear) {
   return PTMF_OK;
 }
 
+int ptmf_op_mult_kernel(ptmf_op op, int precision, int *kernel) {
+  PTMF_CHECK(op && kernel, PTMF_ERR_ARG, "mult_kernel: null argument");
+  PTMF_CHECK(precision == 64 || precision == 32, PTMF_ERR_UNSUPPORTED, "mult_kernel: precision %d (64 or 32)", precision);
+  *kernel = ptmf::a11_mult_kernel(op, precision);
+  return PTMF_OK;
+}
+
 int ptmf_op_state(ptmf_op op, unsigned long *state) {
   PTMF_CHECK(op && state, PTMF_ERR_ARG, "op_state: null");
   *state = op->state;

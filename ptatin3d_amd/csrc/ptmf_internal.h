@@ -195,6 +195,8 @@ int launch_a11(const ptmf_op_s *op, const T *u, T *y, bool mask_columns);
 // whole: false for the element kernel alone, for timing
 template <typename T>
 int launch_a11_mult(ptmf_op_s *op, const T *x, T *y, bool whole);
+// its kernel, numbered as by ptmf_op_mult_kernel
+int a11_mult_kernel(const ptmf_op_s *op, int precision);
 // A row update in place of the product itself: out = os dinv (b - A x) + om1 prev
 // + om x, the second term left out with prev nullptr; with dinv nullptr the
 // residual b - A x alone.  out (FP64 where out64) may be prev or r but not x.

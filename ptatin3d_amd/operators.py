@@ -93,6 +93,12 @@ class MatA11MF:
         call("ptmf_op_rectilinear", self.handle, C.byref(v))
         return bool(v.value)
 
+    def mult_kernel(self, precision: int = 64) -> str:
+        """The element kernel that the MatMult runs as the operator stands."""
+        v = C.c_int()
+        call("ptmf_op_mult_kernel", self.handle, int(precision), C.byref(v))
+        return ("tile", "pipelined", "stored", "coloured", "lane", "column")[v.value]
+
     def set_kernel_variant(self, variant: int) -> None:
         """0: z-march; 1: z-march with next-layer loads issued one stage ahead;
         2: stored quadrature-point geometry; 3: coloured scatter (no tiles)."""

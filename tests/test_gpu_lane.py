@@ -211,3 +211,22 @@ def test_kind_of_mesh_and_default_tiling(gpu):
     A.set_coordinates(F.perturb_interior(coords, *m, 0.1, np.random.default_rng(1)))
     assert not A.rectilinear
     A.destroy()
+
+
+def test_the_kernel_is_told(gpu):
+    """Boxes on either side of the choices between tile, lane and column kernel,
+    and each setting of the caller's."""
+    for m, mesh, prec, want in (((27, 27, 27), "box", 64, "lane"), ((16, 16, 16), "box", 64, "column"),
+                                ((30, 30, 30), "general", 64, "column"), ((48, 48, 48), "general", 64, "tile"),
+                                ((48, 48, 48), "box", 32, "lane"), ((65, 40, 48), "box", 32, "tile")):
+        A = MatA11MF(*m)
+        x = F.box_coords(*m)
+        A.set_coordinates(x if mesh == "box" else F.perturb_interior(x, *m, 0.1, np.random.default_rng(2)))
+        assert A.mult_kernel(prec) == want, (m, mesh, prec)
+        for v, name in ((1, "pipelined"), (2, "stored"), (3, "coloured")):
+            A.set_kernel_variant(v)
+            assert A.mult_kernel(prec) == name
+        A.set_kernel_variant(0)
+        A.set_tiles_per_group(2)
+        assert A.mult_kernel(prec) == "tile"
+        A.destroy()
