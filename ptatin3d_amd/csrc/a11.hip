@@ -1267,33 +1267,37 @@ TileArgs tile_args(const ptmf_op_s *op) {
 // The lane kernel's decomposition of box b in precision T; false where the tile
 // kernel runs instead (as it does on a mesh that is not rectilinear, or with a
 // tiling, variant or tiles per work-group of the caller's choice): with arrays
-// past the 32-bit offsets of the lane kernel, in FP32 with more than 64 elements in a
-// direction (there the tile kernel's FP32 interpolation of the coordinates
-// rounds the Jacobian off by more than 1e-5, and the two kernels would differ
-// by that), and where the tile kernel is faster.
+// past the 32-bit offsets of the lane kernel, in FP32 with more than 64 elements in
+// a direction, and where the tile kernel is faster.  The FP32 line is no choice by
+// speed or accuracy: larger boxes keep the tile kernel's results, which err by its
+// FP32 interpolation of the coordinates (1.9e-5 of the largest at 64^3, 2.4e-5 at
+// 65^3, 5.1e-5 at 128^3; this kernel 2.3e-7 at each) and take 105 us at 65^3 and
+// 746 us at 128^3 where this kernel takes 56 and 323 us.
 // The costs are microseconds per round of one wave on each of the 1024 SIMDs,
 // times the layers a wave marches through.  Measured on boxes from 8^3 to
 // 96 x 96 x 48, FP64: 14 us per layer of 64 elements (lane) and 14.6 us per
 // layer of 20 (tile); FP32, two waves per SIMD: 14.2 and 15.7 us for both, 10 and
 // 10.5 us with one; the lane kernel's first and last planes add 0.57 (0.45) of a
-// layer.  So the tile kernel keeps the boxes that it takes in one round (16^3:
-// 13.5 us against 15.6 us; 20^3: 15.6 and 16.0 us), and the lane kernel has the
-// rest (28^3: 17.8 us against 33.6 us, FP32 13.7 and 17.2 us; 48 x 48 x 32: 32
-// and 71 us, FP32 18 and 31 us; 64^3: 63 and 178 us, FP32 35 and 82 us).
+// layer.  So the tile kernel keeps the boxes that it takes in one round (16^3: 13.1
+// us against 14.9 us; 20^3: 14.7 and 15.0 us; this concerns the saddle point, the
+// MatMult having the column kernel there), and the lane kernel has the rest (28^3:
+// 16.5 us against 28.6 us, FP32 13.2 and 13.7 us; 48 x 48 x 32: 29 and 61 us, FP32
+// 17 and 27 us; 64^3: 56 and 175 us, FP32 31 and 77 us).
 //
 // The column kernel (a11_col.h) has the boxes of up to 100,000 elements, whose
 // element sums fit 64 MiB, on meshes that are not rectilinear (MatMult against
-// the tile kernel's: 8^3 9.2 and 18.4 us, 24^3 20 and 24 us, 45 x 37 x 29 44 and
-// 62 us, 48 x 48 x 32 62 and 82 us, FP32 41 and 43 us; 64 x 64 x 32 in FP32 70
-// and 68 us), and the small rectilinear ones: its MatMult takes 8.5 + E / 1333 us
-// (FP32 7.5 + E / 2222), the lane kernel's that of its kernel above, rounded up
-// for a chip not full, and 1 us (5.5 us): 24^3 20 against 21 us, 32^3 32 against
-// 27 us; FP32 14 against 18 us, 24 against 22 us.
+// the tile kernel's: 8^3 7.8 and 16.5 us, 24^3 15 and 21 us, 45 x 37 x 29 40 and
+// 61 us, 48 x 48 x 32 57 and 71 us, FP32 34 and 36 us), and the small rectilinear
+// ones: its MatMult takes 6.6 + E / 1390 us (FP32 6.9 + E / 2670), the lane kernel's
+// that of its kernel above and in FP32 3.7 us (in FP64 the kernel's time falls
+// short of the model by its face pass): 27^3 19.6 against 21.8 us, 28^3 22.4 and
+// 21.7 us, 30^3 24 and 22 us, 32^3 30 and 23 us; FP32 28^3 15 and 18 us, 31^3 17.7
+// and 18.4 us, 32^3 20 and 18 us.
 constexpr long kColDoubles = 8L << 20;
 
 template <typename T>
 double col_cost(long nel) {
-  return sizeof(T) == 8 ? 8.5 + 0.75e-3 * (double)nel : 7.5 + 0.45e-3 * (double)nel;
+  return sizeof(T) == 8 ? 6.6 + 0.72e-3 * (double)nel : 6.9 + 0.375e-3 * (double)nel;
 }
 
 template <typename T>
@@ -1326,7 +1330,7 @@ bool lane_plan(const Box &b, const Tiling &t, LaneOther other, TileArgs &a) {
     }
   }
   if (other == kOtherTile && best >= t.ZC * lane_rounds<T>(t.ntiles, f64 ? 14.6 : 10.5, 15.7)) return false;
-  if (other == kOtherCol && best + (f64 ? 1.0 : 5.5) >= col_cost<T>(b.nel)) return false;
+  if (other == kOtherCol && best + (f64 ? 0.0 : 3.7) >= col_cost<T>(b.nel)) return false;
   a.fbx_n = a.fby_n = (long)kLRows * (2 * a.ZC + 1);
   a.fbz_n = kLRows * kLRows;
   // byte offsets of the 27 quadrature points' viscosities and of 17 node rows

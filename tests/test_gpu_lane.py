@@ -216,7 +216,7 @@ def test_kind_of_mesh_and_default_tiling(gpu):
 def test_the_kernel_is_told(gpu):
     """Boxes on either side of the choices between tile, lane and column kernel,
     and each setting of the caller's."""
-    for m, mesh, prec, want in (((27, 27, 27), "box", 64, "lane"), ((16, 16, 16), "box", 64, "column"),
+    for m, mesh, prec, want in (((28, 28, 28), "box", 64, "lane"), ((27, 27, 27), "box", 64, "column"),
                                 ((30, 30, 30), "general", 64, "column"), ((48, 48, 48), "general", 64, "tile"),
                                 ((48, 48, 48), "box", 32, "lane"), ((65, 40, 48), "box", 32, "tile")):
         A = MatA11MF(*m)
