@@ -205,9 +205,9 @@ int ptmf_a11_mult_f32(ptmf_op op, const float *x, float *y);
 /* ptmf_a11_mult that allocates nothing (no hipMalloc / hipFree / allocating
  * library call).  No counterpart in the reference: it is for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops,
- * harnesses that forbid allocation).  The z-march's face buffers live in a
- * static device array of 64 MiB per GPU (8,388,608 doubles, held until the
- * process ends): a box and tiling whose face buffers need more return
+ * harnesses that forbid allocation).  The kernels' face buffers or element sums
+ * live in a static device array of 64 MiB per GPU (8,388,608 doubles, held until
+ * the process ends): a box and tiling whose face buffers need more return
  * PTMF_ERR_UNSUPPORTED.  Same kernels and results as ptmf_a11_mult (the
  * stored-geometry and coloured kernel variants run as the default z-march).
  * The operator must be set up (ptmf_op_set_viscosity / ptmf_op_set_tiling
@@ -339,8 +339,11 @@ int ptmf_mg_fcg(ptmf_mg mg, const double *b, double *x, double rtol, int maxit, 
  * tiling and Dirichlet data); ptmf_batch_mult applies MatMult_MFStokes_A11 to
  * every box, x and y being host arrays of nops device pointers (double** for
  * precision 64, float** for 32).  The work of all boxes is one list of
- * (box, tile) items, so small boxes no longer cost a launch each.  No
- * counterpart in the reference (one PETSc Mat per problem). */
+ * (box, tile) or, for the kernel with one lane per node column, (box, wave)
+ * items, so small boxes no longer cost a launch each.  The call holds the
+ * operators' face buffers until its kernels are done: a MatMult of a member from
+ * another thread waits for it.  No counterpart in the reference (one PETSc Mat
+ * per problem). */
 int ptmf_batch_create(const ptmf_op *ops, int nops, ptmf_batch *batch);
 int ptmf_batch_destroy(ptmf_batch *batch);
 int ptmf_batch_mult(ptmf_batch batch, int precision, const void *const *x, void *const *y);

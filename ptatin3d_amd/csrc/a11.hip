@@ -1775,8 +1775,8 @@ int launch_stokes_mult_t(ptmf_op_s *op, const T *x, T *y) {
   std::lock_guard<std::mutex> lock(op->faces_mu);
   PTMF_CHECK(op->faces != nullptr, PTMF_ERR_NOT_SETUP, "stokes: face buffers not allocated");
   const long nu = 3 * op->box.nnodes;
-  // (by lane_plan's rule for the MatMult: at 24^3 both take 42 us, at 28^3 the
-  // lane kernel 41 us and the tile kernel 62 us, and further apart above)
+  // (by lane_plan's rule: at 24^3, with the tile kernel, 37 us; at 28^3 the lane
+  // kernel takes 33 us and the tile kernel 56 us, and further apart above)
   TileArgs la;
   if (lane_tiles<T>(op, op->faces_doubles, kOtherTile, la))
     return launch_lane<T, true>(op, la, kFinMult, nullptr, x, x + nu, y, y + nu, (T *)op->faces);

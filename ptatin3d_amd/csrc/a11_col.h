@@ -7,13 +7,14 @@
 // lanes of a quad, y through LDS.  The element's 81 sums go to memory; a second
 // pass adds up each node's up to eight elements in a fixed order.
 //
-// What bounds it: on small boxes one wave's latency, a third of the tile
-// kernel's, whose lanes do the work of three of these (16^3: 6.0 us and 5.4 us
-// for the sums, the tile kernel 13.6 and 5.3 us).  On larger ones instruction
-// issue, at three waves per SIMD (1,220 vector instructions for five elements,
-// 753 of them FP64; VALU busy 87 %), and the 650 bytes of sums per element:
-// 45 x 37 x 29 in 30 and 13 us (tile kernel 51 and 10 us).  With x in LDS too,
-// seven elements to a wave, bank conflicts bound it (16^3 6.9 us).
+// What bounds it: on small boxes one wave's latency, less than half of the tile
+// kernel's, whose lanes do the work of three of these (16^3, kernel and what
+// follows it in one launch after the other: 6.0 us and 3.3 us for the sums, the
+// tile kernel 13.1 and 3.8 us).  On larger ones instruction issue, at three waves
+// per SIMD (1,210 vector instructions for five elements, 730 of them FP64; VALU
+// busy 87 %), and the 650 bytes of sums per element: 45 x 37 x 29 in 31 and 9 us
+// (tile kernel 55 and 6 us).  With x in LDS too, seven elements to a wave, bank
+// conflicts bound it (16^3 6.9 us).
 
 constexpr int kColElems = 5;  // elements of a wave
 

@@ -14,8 +14,8 @@
 // What bounds it: instruction issue of the one (FP64) or two (FP32) waves per
 // SIMD that the registers allow.  FP64: 256 VGPRs + 168 AGPRs, about 4,200
 // vector instructions per layer of which 3,050 are FP64 arithmetic, VALU busy
-// 57 % of the wave's cycles, waiting 20 %.  64^3, MI355X: 62 us in FP64 (tile
-// kernel 178 us), 35 us in FP32 (82 us).  The loads are the delicate part: a value that
+// 57 % of the wave's cycles, waiting 20 %.  64^3, MI355X: 54 us in FP64 (tile
+// kernel 175 us), 32 us in FP32 (77 us).  The loads are the delicate part: a value that
 // is still in flight when the registers run short is waited for at once, to
 // be moved to an accumulation register or to scratch, one round trip each (the
 // same kernel with its loads in flight across the stress stage took 130 us,
@@ -23,9 +23,9 @@
 // stage and used up at its end, where few registers are live.
 //
 // The saddle-point product runs the same way: the couplings add some 10
-// instructions a point, the pressure basis being that of the unit cube, and 66
-// AGPRs (96 x 96 x 48 MatMult 171 us, the tile kernel's 485 us; 28^3 41 and 62
-// us).
+// instructions a point, the pressure basis being that of the unit cube, and 38
+// AGPRs (96 x 96 x 48 MatMult 143 us, the tile kernel's 485 us before its face
+// pass became faster; 28^3 33 and 56 us, 48^3 53 and 145 us).
 
 // Per-lane constants of a rectilinear element: the collocation coefficients of
 // the in-plane directions scaled by 2 m / h, and the weights.  m is a power of two

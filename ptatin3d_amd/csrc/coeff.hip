@@ -17,7 +17,7 @@ namespace {
 // contracted with h A[c][i] A[c][j], h = w eta / detJ, A the adjugate: 2,700
 // operations an element by sum factorisation where 27 x 27 gradients take
 // 20,000.  Bound by instruction issue at one wave per SIMD (6,500 FP64
-// instructions a layer, 3,500 of them the geometry): 48^3 in 56 us and 10 us of
+// instructions a layer, 3,500 of them the geometry): 48^3 in 56 us and 9 us of
 // faces, and no fill or Dirichlet pass; eight passes over element classes, 27
 // lanes per element, took 230 us.
 // ---------------------------------------------------------------------------

@@ -48,8 +48,8 @@ __device__ __forceinline__ void pressure_frame(const double *s0, const double *s
 //
 // Bound by instruction issue at one wave
 // per SIMD (4,100 FP64 instructions a layer of 64 elements, two thirds of the
-// kernel's): 64 x 48 x 40 in 44 us and 11 us of faces; one 27-lane group per
-// element with atomic adds to y took 290 us.
+// kernel's): 64 x 48 x 40 in 44 us and 9 us of faces; eight passes over element
+// classes, 27 lanes per element, took 290 us.
 // ---------------------------------------------------------------------------
 struct A12Op {
   static constexpr LaneBC kBC = kLaneZero;
