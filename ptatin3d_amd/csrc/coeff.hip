@@ -273,12 +273,19 @@ __global__ void __launch_bounds__(64)
 
 }  // namespace
 
-int launch_a11_diag(const ptmf_op_s *op, double *d) {
-  // Measured, 27 lanes and one lane: one element 22 and 35 us, 2^3 76 and 37, 48^3
-  // 233 and 70; 1 x 1 x 5000 37 and 117, 256 x 1 x 256 143 and 178, 128 x 1 x 128 67
-  // and 61, 512 x 2 x 64 163 and 104.
+// Measured, 27 lanes and one lane: one element 22 and 35 us, 2^3 76 and 37, 48^3 233
+// and 70; 1 x 1 x 5000 37 and 117, 256 x 1 x 256 143 and 178, 128 x 1 x 128 67 and
+// 61, 512 x 2 x 64 163 and 104.
+static bool diag_lane(const Box &b, TileArgs &a) { return node_lane_plan(b, 14.0, 8.0, 1.5, 8.5, 19.6, a); }
+
+bool a11_diag_lane(const Box &b) {
   TileArgs a;
-  if (!node_lane_plan(op->box, 14.0, 8.0, 1.5, 8.5, 19.6, a)) return launch_a11_diag_elems(op, d);
+  return diag_lane(b, a);
+}
+
+int launch_a11_diag(const ptmf_op_s *op, double *d) {
+  TileArgs a;
+  if (!diag_lane(op->box, a)) return launch_a11_diag_elems(op, d);
   DiagOp g{};
   g.eta = op->d64.eta;
   g.nel = op->box.nel;

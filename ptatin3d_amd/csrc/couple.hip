@@ -213,17 +213,20 @@ __global__ void __launch_bounds__(64)
 
 }  // namespace
 
+// Measured, 27 lanes and one lane: one element 21 and 30 us, 2^3 63 and 31, 48^3 252
+// and 58; 1 x 1 x 5000 36 and 91, 2 x 2 x 20000 197 and 302, 256 x 1 x 256 154 and
+// 136.
+static bool a12_lane(const Box &b, TileArgs &a) { return node_lane_plan(b, 14.3, 6.4, 1.7, 9.0, 14.6, a); }
+
 long node_face_doubles(const Box &b) {
-  const TileArgs a = lane_args(b, 1024, 0.45);
-  return face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles);
+  TileArgs a;
+  // (the diagonal's decomposition is the same)
+  return a12_lane(b, a) || a11_diag_lane(b) ? face_buffer_doubles(kLT, kLT, a.ZC, a.ntiles) : 0;
 }
 
 int launch_a12(const ptmf_op_s *op, const double *p, double *yu) {
-  // Measured, 27 lanes and one lane: one element 21 and 30 us, 2^3 63 and 31, 48^3
-  // 252 and 58; 1 x 1 x 5000 36 and 91, 2 x 2 x 20000 197 and 302, 256 x 1 x 256
-  // 154 and 136.
   TileArgs a;
-  if (!node_lane_plan(op->box, 14.3, 6.4, 1.7, 9.0, 14.6, a)) return launch_a12_elems(op, p, yu);
+  if (!a12_lane(op->box, a)) return launch_a12_elems(op, p, yu);
   A12Op b{};
   b.p = p;
   return launch_node_lane(op, a, b, yu);

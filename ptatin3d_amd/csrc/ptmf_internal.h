@@ -221,7 +221,9 @@ int classify_mesh(ptmf_op_s *op);
 // does not run there); part of every operator's allocation, whatever its mesh,
 // so that new coordinates never move the buffers
 long lane_face_doubles(const Box &b, const Tiling &t);
-long node_face_doubles(const Box &b);  // of launch_a12 and launch_a11_diag
+// face buffers of launch_a12's and launch_a11_diag's lane kernels (0: neither runs on box b)
+long node_face_doubles(const Box &b);
+bool a11_diag_lane(const Box &b);
 // set-up: op->bcword from the operator's Dirichlet bits
 int mark_dirichlet_planes(ptmf_op_s *op);
 template <typename T>
