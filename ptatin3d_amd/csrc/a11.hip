@@ -1427,13 +1427,17 @@ __global__ void __launch_bounds__(64)
 }  // namespace
 
 int alloc_lane_data(ptmf_op_s *op) {
-  // one allocation: 2 m / h and m in FP64 (and three tolerances) and in FP32, the
-  // classification's flag, the Dirichlet words
+  // one allocation: the face buffers of A12 and the diagonal, 2 m / h and m in FP64
+  // (and three tolerances) and in FP32, the classification's flag, the Dirichlet words
   const Box &b = op->box;
   const long na = b.mx + b.my + b.mz;
   const long planes = (long)((b.mx + kLT - 1) / kLT) * ((b.my + kLT - 1) / kLT) * b.Z;
-  PTMF_TRY(ptmf_malloc((void **)&op->ax64, sizeof(double) * (na + 4) + sizeof(float) * (na + 1) + sizeof(int) +
-                                               64 * sizeof(unsigned) * planes));
+  const long nf = node_face_doubles(b);
+  PTMF_TRY(ptmf_malloc((void **)&op->lane_data, sizeof(double) * (nf + na + 4) + sizeof(float) * (na + 1) + sizeof(int) +
+                                                    64 * sizeof(unsigned) * planes));
+  op->node_faces = op->lane_data;
+  op->node_faces_doubles = nf;
+  op->ax64 = op->lane_data + nf;
   op->ax32 = (float *)(op->ax64 + na + 4);
   op->rect_bad = (int *)(op->ax32 + na + 1);
   op->bcword = (unsigned *)(op->rect_bad + 1);

@@ -173,8 +173,6 @@ int ptmf_op_create(int mx, int my, int mz, ptmf_op *out) {
                                                            op->tiling.ntiles),
                                  ptmf::lane_face_doubles(b, op->tiling));
     st = ptmf_malloc(&op->faces, sizeof(double) * op->faces_doubles);
-    op->node_faces_doubles = ptmf::node_face_doubles(b);
-    alloc((void **)&op->node_faces, sizeof(double) * op->node_faces_doubles);
   }
   if (st != PTMF_OK) {
     ptmf_op tmp = op;
@@ -196,7 +194,6 @@ int ptmf_op_destroy(ptmf_op *pop) {
   (void)hipFree(op->bcnode);
   (void)hipFree(op->bcidx);
   (void)hipFree(op->faces);
-  (void)hipFree(op->node_faces);
   (void)hipFree(op->host_stage);
   (void)hipFree(op->host_stage2);
   (void)hipFree(op->pa64);
@@ -204,7 +201,7 @@ int ptmf_op_destroy(ptmf_op *pop) {
   (void)hipFree(op->pa_bad);
   (void)hipFree(op->et64);
   (void)hipFree(op->et32);
-  (void)hipFree(op->ax64);
+  (void)hipFree(op->lane_data);
   (void)hipFree(op->points);
   if (op->ev0) (void)hipEventDestroy(op->ev0);
   if (op->ev1) (void)hipEventDestroy(op->ev1);

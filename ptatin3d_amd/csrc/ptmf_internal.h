@@ -110,7 +110,8 @@ struct ptmf_op_s {
   // rectilinear mesh (element faces normal to the axes): 2 m / h per element of
   // the mx columns, my rows and mz layers, then m (a11_lane.h)
   int rect = 0;
-  double *ax64 = nullptr;         // holds ax32, rect_bad and bcword too
+  double *lane_data = nullptr;    // holds node_faces, ax64, ax32, rect_bad and bcword
+  double *ax64 = nullptr;
   float *ax32 = nullptr;
   int *rect_bad = nullptr;
   int variant = 0;  // MatMult kernel: 0 z-march, 1 software-pipelined, 2 stored geometry, 3 coloured
@@ -213,7 +214,7 @@ int launch_a11_update(ptmf_op_s *op, const T *x, T *r, const RowUpdate<T> &up);
 // build (or rebuild) the FP64 tile-ordered viscosity for the current
 // coefficients and tiling (allocates; set-up time)
 int prepare_eta_tiled(ptmf_op_s *op);
-// the operator's data of the lane kernel (freed through op->ax64)
+// the operator's data of the lane kernels (op->lane_data and the pointers into it)
 int alloc_lane_data(ptmf_op_s *op);
 // set-up: op->rect and op->ax* from the operator's coordinates
 int classify_mesh(ptmf_op_s *op);
